@@ -6,36 +6,40 @@
 // else nd, and s1 = +-1 from qweight1 (TriSMoE_cuda_kernel.cu:665-774); the
 // products are formed with packed fp16 multiplies (round to nearest even, as
 // __hmul) on column factors staged negated (P_j = fp16(-C_j * R_j) = -fp16(C_j * R_j)
-// exactly).  The choice of j and the sign come from the bit planes as two
-// selector pairs sd, sn in {0, +1, -1}: w = fma(sd, P_d, sn * P_nd), exact
-// because one of the two terms is zero.  Salient columns (a few per cent,
-// w = fp16(+-fp16(C0*R0) +- fp16(C1*R1))) are zero in that operand and get
-// their own MFMA pass over an LDS table of their exact weights.  Products with the activations are
+// exactly); the split bits pick P_d or P_nd and the sign bits flip it (mf_row_b).
+// Salient columns (a few per cent, w = fp16(+-fp16(C0*R0) +- fp16(C1*R1))) are zero in
+// that operand and get MFMA steps of their own.  Products with the activations are
 // exact in fp32 and accumulate in fp32, as in the reference's tensor-core
 // kernel (TriSMoE_cuda_kernel.cu:4889-5093).
 //
-// Operand layout (v_mfma_f32_16x16x32_f16): A rows are up to 16 rows of one
-// segment; lane group kg (lanes 16kg..16kg+15) supplies the 8 columns
-// k = kg + 4i (i = 0..7) of each 32-column packed row, so after one shift the
-// sign / split / salient bits of those columns sit at nibble positions 4i of a
-// word.  OR-ing in the fp4 (e2m1) exponent pattern gives eight fp4 selectors
-// (+-1.0 = 0b0010 / 0b1010, 0 = 0b0000) that v_cvt_scalef32_pk_f16_fp4
-// expands two at a time to fp16 pairs.  Activations and the column factors are
+// Operand layout of the decode kernel (v_mfma_f32_16x16x32_f16): A rows are up to 16 rows
+// of one segment; lane group kg (lanes 16kg..16kg+15) supplies the 8 columns kg + 4i and
+// kg + 4i + 16 (i < 4) of each 32-column packed row.  Activations and the column factors are
 // staged in LDS in the same permuted column order, so each lane reads its 8
 // values with one 16-byte LDS load.
 //
-// Work decomposition: workgroup = 4 wavefronts = one 64-output tile x one
-// tile of <= 16 rows of one segment x one projection (blockIdx.z).  The
+// Work decomposition of the decode kernel: workgroup = 4 wavefronts = a run of 64-output
+// tiles x one tile of <= 16 rows of one segment x one projection (blockIdx.z).  The
 // workgroup stages the rows' activations and the column factors of a 512-column
-// chunk in LDS once; wavefront w then owns outputs [16w, 16w+16) over the whole
-// chunk, issuing its weight loads (one column per lane, 16 packed rows) before
-// computing, so no partial sums cross wavefronts.  Salient columns are zero in
-// that pass; afterwards each lane writes the exact salient weights of its
-// column (lane group kg takes the salient columns k = kg (mod 4)) into an LDS
-// table, and one or two more MFMA steps multiply the activations gathered at
-// the salient columns by it, into the same fp32 accumulator.  Requires each
-// 64-column K tile to lie in a single group (the reference's UniformK64Groups
+// chunk in LDS once; wavefront w then owns outputs [16w, 16w+16) of each tile over the whole
+// chunk, two tiles at a time, while its weight words of the next two are in flight, so no
+// partial sums cross wavefronts.  Salient columns are zero in that pass; afterwards each lane
+// builds the exact salient weights of its column, and one or two more MFMA steps multiply the
+// activations gathered at the salient columns by them, into the same fp32 accumulator.
+// Requires each 64-column K tile to lie in a single group (the reference's UniformK64Groups
 // case) and rank % 64 == 0.
+//
+// What bounds the decode kernel.  At decode sizes a launch is short (10 to 30 us), and three
+// things share it: the operand build (VALU issue, see mf_row_b); the way to the first tile, a
+// chain of dependent scalar and vector loads and some 700 instructions which every wavefront
+// runs; and fetching the instructions, since a launch starts with a cold instruction cache.  So
+// the kernel asks for its scalars and row indices at once, keeps the K loop rolled, and hides
+// the sizes and the lane index from the compiler per row tile, which otherwise computes
+// every address of the rare paths ahead of the loop.  T = 16 gate/up launch at the Mixtral shape
+// 31.5 -> 27.7 us, T = 64 42.3 -> 36.3 us; OLMoE T = 16 gate/up 17.6 -> 12.7, down 16.3 -> 11.9 us;
+// A3B T = 1024 gate/up 67 -> 49, down 113 -> 79 us.
+#include <type_traits>
+
 #include "tris_common.h"
 
 namespace tris {
@@ -70,6 +74,7 @@ struct MfmaArgs {
   const int32_t* expert_ids;
   const int32_t* segment_offsets;
   int num_segments;
+  int batch;              // routed rows
   int decoded_by_expert;  // 0: decoded holds one slot per segment; 1: one per expert id (every expert decoded)
   // One token's combine in the launch (two units, proj[1] == proj[0]; null: none): the token's two routed rows are
   // row tiles 0 and 1, one a unit, and unit 0 writes dt(fp16(out_r0 * w_r0) + fp16(out_r1 * w_r1)) to comb_out.
@@ -79,9 +84,9 @@ struct MfmaArgs {
   int comb_bf16;            // comb_out is bf16 (else fp16)
 };
 
-// Position of column k (0..31) of a packed row in the staged order: lane group
-// k % 4, element k / 4.
-__device__ __forceinline__ int mf_perm32(int k) { return 8 * (k & 3) + (k >> 2); }
+// Position of column k (0..31) of a packed row in the staged order: lane group k % 4, elements 2 i and 2 i + 1 of it
+// columns k % 4 + 4 i and 16 past that, so that a packed pair of weights takes its bits from the two halves of a word.
+__device__ __forceinline__ int mf_perm32(int k) { return 8 * (k & 3) + 2 * ((k >> 2) & 3) + (k >> 4); }
 
 // Nibbles 2i, 2i+1 (byte i) of eight fp4 values -> two fp16 (low nibble -> low half).
 __device__ __forceinline__ f16x2 fp4x2_to_f16x2(uint32_t nib, int byte_sel) {
@@ -114,24 +119,18 @@ __device__ inline bool mf_map_row_tile(const int32_t* __restrict__ seg, const in
       const int len = hi - lo;
       t = len > 0 ? (len + row_tile - 1) / row_tile : 0;
     }
-    int incl = t;
-#pragma unroll
-    for (int d = 1; d < kWave; d <<= 1) {
-      const int v = __shfl_up(incl, d);
-      if (lane >= d) incl += v;
-    }
-    const int total = __shfl(incl, kWave - 1);
-    if (tile < base + total) {
+    const int incl = wave_incl_sum_i32(t);
+    const int total = __builtin_amdgcn_readlane(incl, kWave - 1);
+    if (tile < base + total) {  // wave-uniform
       const uint64_t hit = __ballot(i < nseg && tile < base + incl);
-      const int L = __ffsll(static_cast<unsigned long long>(hit)) - 1;
-      const int excl = __shfl(incl - t, L);
-      const int local = tile - base - excl;
-      const int row0 = __shfl(lo, L) + local * row_tile;
-      const int end = __shfl(hi, L);
+      const int L = __builtin_amdgcn_readfirstlane(__ffsll(static_cast<unsigned long long>(hit)) - 1);
+      const int local = tile - base - __builtin_amdgcn_readlane(incl - t, L);
+      const int row0 = __builtin_amdgcn_readlane(lo, L) + local * row_tile;
+      const int end = __builtin_amdgcn_readlane(hi, L);
       *s_out = c + L;
       *row0_out = row0;
       *rc_out = (end - row0) < row_tile ? (end - row0) : row_tile;
-      *e_out = __shfl(ex, L);
+      *e_out = __builtin_amdgcn_readlane(ex, L);
       return true;
     }
     base += total;
@@ -160,12 +159,7 @@ __device__ inline MfSegScan mf_scan_segments(const int32_t* __restrict__ seg, co
     const int ex = expert_ids[ic];
     int t = 0;
     if (i < nseg) t = hi > lo ? (hi - lo + row_tile - 1) / row_tile : 0;
-    int incl = t;
-#pragma unroll
-    for (int d = 1; d < kWave; d <<= 1) {
-      const int v = __shfl_up(incl, d);
-      if (lane >= d) incl += v;
-    }
+    const int incl = wave_incl_sum_i32(t);
     if (c == 0) {
       r.lo = lo;
       r.hi = hi;
@@ -173,7 +167,7 @@ __device__ inline MfSegScan mf_scan_segments(const int32_t* __restrict__ seg, co
       r.t = t;
       r.incl = incl;
     }
-    r.total += __shfl(incl, kWave - 1);
+    r.total += __builtin_amdgcn_readlane(incl, kWave - 1);
   }
   return r;
 }
@@ -185,14 +179,14 @@ __device__ inline void mf_map_scanned(const MfSegScan& sc, const int32_t* __rest
   if (nseg <= kWave) {
     const int lane = static_cast<int>(__lane_id());
     const uint64_t hit = __ballot(lane < nseg && tile < sc.incl);
-    const int L = __ffsll(static_cast<unsigned long long>(hit)) - 1;
-    const int local = tile - __shfl(sc.incl - sc.t, L);
-    const int row0 = __shfl(sc.lo, L) + local * row_tile;
-    const int end = __shfl(sc.hi, L);
+    const int L = __builtin_amdgcn_readfirstlane(__ffsll(static_cast<unsigned long long>(hit)) - 1);
+    const int local = tile - __builtin_amdgcn_readlane(sc.incl - sc.t, L);
+    const int row0 = __builtin_amdgcn_readlane(sc.lo, L) + local * row_tile;
+    const int end = __builtin_amdgcn_readlane(sc.hi, L);
     *s_out = L;
     *row0_out = row0;
     *rc_out = (end - row0) < row_tile ? (end - row0) : row_tile;
-    *e_out = __shfl(sc.ex, L);
+    *e_out = __builtin_amdgcn_readlane(sc.ex, L);
     return;
   }
   mf_map_row_tile(seg, expert_ids, nseg, tile, row_tile, s_out, row0_out, rc_out, e_out);
@@ -214,13 +208,13 @@ constexpr int kMfCus = 256;  // MI355X compute units
 // groups and 64 salient columns per expert) fits four workgroups per CU.
 constexpr int mf_groups_cap(bool compact) { return compact ? 4 : kMfMaxGroups; }
 constexpr int mf_sal_slots(bool compact) { return compact ? 64 : kMfChunk; }
-// per wavefront and copy buffer: qweight1 and split words of 16 columns, their row-scale block and a zero word
+// per wavefront and tile: a zero word, the qweight1 and split words of 16 columns and their row-scale block
 constexpr int mf_wave_alloc_bytes(bool compact) {
-  return (2 * (kMfChunk / 32) * 16 + 16 * mf_groups_cap(compact) * 2 + 4) * 4;
+  return (4 + 2 * (kMfChunk / 32) * 16 + 16 * mf_groups_cap(compact) * 2) * 4;
 }
 constexpr int kMfRuns = kMfRows * (kMfChunk / 8) / kMfThreads;  // activation runs per thread of a unit
 
-constexpr int kMfExchBytes = kMfThreads * 4 * 4;  // SwiGLU: the up unit's accumulators for the gate unit
+constexpr int kMfExchBytes = kMfThreads * 4 * 4;  // SwiGLU: the up unit's accumulators of a tile for the gate unit
 
 // Bump allocation of 16-byte aligned pieces (byte offsets into dynamic LDS).
 __host__ __device__ inline int mf_take(int* o, int b) {
@@ -231,15 +225,15 @@ __host__ __device__ inline int mf_take(int* o, int b) {
 
 // Static LDS of the decode kernel with `units` units and `rows` staged activation rows (as declared there).
 constexpr int mf_static_lds_bytes(int units, int rows, bool compact) {
-  return units * (rows * kMfXStride * 2 + kMfChunk * (2 + 2) + mf_sal_slots(compact) * (4 + 2 + 4) + 16 * 4 +
+  return units * (rows * kMfXStride * 2 + kMfChunk * (2 + 2) + mf_sal_slots(compact) * (4 + 2 + 4) + 48 + (kMfChunk / kTileK) * 8 +
                   2 * kMfWaves * mf_wave_alloc_bytes(compact)) +
-         (units == 2 ? kMfExchBytes : 16);
+         (units == 2 ? 2 * kMfExchBytes : 16);
 }
 
 struct MfChunk {       // a unit's staged chunk
   uint16_t* xs;        // [rows][kMfXStride] activations, staged column order; column kMfChunk is zero (decode)
-  uint16_t* cds;       // -C_d, staged column order (0 for salient columns)
-  uint16_t* cns;       // -C_nd, staged column order (0 for salient columns)
+  uint16_t* cds;       // -C_d, staged column order (0 for salient columns); decode: -C_nd follows
+  uint16_t* cns;       // weight-stationary: -C_nd (0 for salient columns)
   // Weight-stationary kernel (natural column order):
   uint32_t* col_sal;   // C0 | C1 << 16, natural order
   uint16_t* sal_col;   // chunk column of the chunk's q-th salient column
@@ -247,11 +241,13 @@ struct MfChunk {       // a unit's staged chunk
   // kMfSalWin, read as zero weights and zero activations):
   uint32_t* sal_w;     // bits 0-4: (column - 15) mod 32, the right rotation that puts the column's qweight1 bit
                        // at bit 15; bits 8-15: byte offset of its group's R0 | R1 in a column's row-scale block;
-                       // bits 16-31: byte offset of its packed row in a wavefront's qweight1 words
+                       // bits 16-31: byte offset of its packed row in a wavefront's weight words
   uint16_t* sal_xo;    // byte offset of its activation in a staged row (the zero column for padding slots)
   uint32_t* sal_cp;    // C0 | C1 << 16 with both signs flipped (decode), or as stored (weight-stationary)
   uint16_t* sal_xi;    // weight-stationary: its position in the staged column order
-  int32_t* meta;       // [t < 8] group of K tile t (-1: none); [8] first salient index; [9] end
+  int32_t* meta;       // weight-stationary: [t < 8] group of K tile t (-1: none); [8] first salient index; [9] end
+  uint2* goff;         // decode: per K tile, where a column's R_d | R_nd word lies in a tile's words: byte offset, and a
+                       // mask of the lane's column offset (a K tile without a group reads the zero word: 0, 0)
 };
 struct MfTileBuf {     // one output tile's weight words
   uint32_t* q1;        // [kMfPR][kMfQ1Stride] qweight1 words of the tile's 64 columns
@@ -259,30 +255,26 @@ struct MfTileBuf {     // one output tile's weight words
   uint32_t* rs;        // [64][G][2] row_pack3: R0 | R1 << 16, R_d | R_nd << 16
 };
 
-// Decode kernel: each wavefront copies only the weight words of its own 16 output columns, so no other
-// wavefront waits for them.  Per wavefront and buffer: qweight1 [kMfPR][16], split words [kMfPR][16] and the
-// row-scale block [16 columns][kMfMaxGroups][2]; every piece is a whole number of 64-lane copies, so a tile
-// always takes kMfWDma copies (a fixed count lets each wavefront wait for exactly its own).
+// Decode kernel: each wavefront loads only the weight words of its own 16 output columns of a tile, so no other
+// wavefront waits for them: into registers (MfWaveRegs) while the tiles before are computed, then into its own LDS
+// words.  Per tile: a zero word (read for K tiles without a group); packed rows 2 t and 2 t + 1 of a column together,
+// qweight1 and split word each; the row-scale block [16 columns][G][R0 | R1, R_d | R_nd].
 constexpr int kMfWCols = 16;
-constexpr int kMfWq1 = 0;
-constexpr int kMfWgw = kMfPR * kMfWCols;
-constexpr int kMfWrs = 2 * kMfPR * kMfWCols;
+constexpr int kMfWw = 4;                            // word offset of the weight words (the zero word is word 0)
+constexpr int kMfWrs = kMfWw + 2 * kMfPR * kMfWCols;  // word offset of the row scales
 template <bool kCompact>
 struct MfWaveWords {
-  static constexpr int kRsCopies = kMfWCols * mf_groups_cap(kCompact) * 2 / kWave;
-  static constexpr int kWords = kMfWrs + kRsCopies * kWave;
-  static constexpr int kDma = kWords / kWave;
-  static constexpr int kAlloc = kWords + 4;  // + a zero word that no copy writes (read for K tiles without a group)
-  static_assert(kMfWCols * mf_groups_cap(kCompact) * 2 % kWave == 0 && kMfWgw % kWave == 0 && kMfWrs % kWave == 0,
-                "whole 64-lane copies");
-  static_assert(kAlloc * 4 == mf_wave_alloc_bytes(kCompact), "LDS accounting");
+  static constexpr int kRsLane = kMfWCols * mf_groups_cap(kCompact) * 2 / kWave;  // row-scale words a lane loads
+  static constexpr int kAlloc = kMfWrs + kRsLane * kWave;
+  static_assert(kRsLane * kWave == kMfWCols * mf_groups_cap(kCompact) * 2 && (kRsLane == 2 || kRsLane == 4),
+                "one 8- or 16-byte row-scale load a lane");
+  static_assert(kAlloc * 4 == mf_wave_alloc_bytes(kCompact) && kMfWrs % 4 == 0, "LDS accounting");
 };
-struct MfWaveBuf {     // one wavefront's copy of its 16 columns' words
-  uint32_t* q1;        // [kMfPR][16]
-  uint32_t* gw;        // [kMfPR][16]
-  uint32_t* rs;        // [16][G][2]
-  uint32_t* zero;      // a word that holds 0
+template <bool kCompact>
+struct MfWaveRegs {    // a tile's words in flight: lane l holds columns 4 (l % 4) .. + 3 of packed row l / 4, and
+  uint32_t q[4], g[4], rs[MfWaveWords<kCompact>::kRsLane];  // row-scale words kRsLane l .. of the 16 columns' run
 };
+constexpr uint32_t kMfOob = 0x80000000u;  // a byte offset past every buffer (each is below 2 GiB): reads 0, drops stores
 
 // Byte offset of 8 activation columns [c, c + 8) of segment row row0 + r (r < rc), or `oob` (an offset
 // past the buffer: the load reads zeros) for rows outside the tile, columns past the rank and gathered
@@ -299,15 +291,9 @@ __device__ __forceinline__ uint32_t mf_hidden_voff(const MfmaProj& pa, int row0,
   return static_cast<uint32_t>(src * rank + c) * 2u;
 }
 
-// The activation buffer resource of rows [row0, row0 + rc) and its size (the offset that reads zeros).  With
-// partial sums the activations are staged from them (mf_partials_stage): an empty resource, whose loads read zeros
-// without a memory access.
+// The activation buffer resource of rows [row0, row0 + rc) and its size (the offset that reads zeros).
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t mf_hidden_rsrc(const MfmaProj& pa, int row0, int rc, int rank,
-                                                                 uint32_t* bytes, bool part = false) {
-  if (part) {
-    *bytes = 0u;
-    return make_rsrc(pa.partials, 0u);
-  }
+                                                                 uint32_t* bytes) {
   if (pa.row_index != nullptr) {
     *bytes = static_cast<uint32_t>(pa.hidden_rows) * rank * 2u;
     return make_rsrc(pa.hidden, *bytes);
@@ -327,7 +313,8 @@ __device__ __forceinline__ uint4 bload128(__amdgpu_buffer_rsrc_t r, uint32_t vof
   const auto v = __builtin_amdgcn_raw_buffer_load_b128(r, voff, soff, 0);
   return make_uint4(v[0], v[1], v[2], v[3]);
 }
-// Buffer loads straight into LDS: lane l's 4 (16) bytes land at dst + 4l (16l); dst is wave-uniform.
+// Buffer loads straight into LDS (the weight-stationary kernel): lane l's 4 (16) bytes land at dst + 4l (16l); dst is
+// wave-uniform.
 __device__ __forceinline__ void dma32(__amdgpu_buffer_rsrc_t r, void* dst, uint32_t voff, uint32_t soff) {
   __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (__attribute__((address_space(3))) void*)dst, 4, voff, soff, 0, 0);
 }
@@ -335,51 +322,29 @@ __device__ __forceinline__ void dma128(__amdgpu_buffer_rsrc_t r, void* dst, uint
   __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (__attribute__((address_space(3))) void*)dst, 16, voff, soff, 0, 0);
 }
 
-// s_waitcnt on the vector memory counter alone (gfx9 encoding: vmcnt in bits 3:0 and 15:14; the export and LDS
-// counters left at their maxima): wait until at most N vector memory operations are outstanding.
-template <int N>
-__device__ __forceinline__ void wait_vmcnt() {
-  static_assert(N >= 0 && N < 64, "vmcnt is 6 bits");
-  __builtin_amdgcn_s_waitcnt((N & 15) | ((N >> 4) << 14) | (7 << 4) | (15 << 8));
-}
-
-// Register-staged loads of a unit's chunk, held between issue and write.
+// Weight-stationary kernel: register-staged column loads of a unit's chunk, held between issue and write.
 struct MfRegs {
-  uint4 xv[kMfRuns];  // activation runs: row 4h + wave, 8 columns at lane * 8
   uint64_t cpv[2];    // col_pack3 of columns kc + utid, kc + utid + 256
   uint32_t cmt[2];    // their salient words
   int q2t[2];         // their packed rows' salient prefix
-  int gt[2];          // their groups (g_idx), -1 past the rank
   int sbase0;         // salient prefix at the chunk's first packed row
-  int send;           // salient prefix at the chunk's end
   int32_t mv;         // metadata word (see mf_chunk_issue)
 };
 
-// Issue the register loads of chunk [kc, kc + 512) of one projection for rows [row0, row0 + rc) of
-// expert e.  utid is the thread's index within its unit.  Every load is issued unconditionally (a
-// branch around a load makes the compiler wait for it at the join); invalid lanes get an offset past
-// their buffer, which reads 0.
-__device__ __forceinline__ void mf_chunk_issue(const MfmaProj& pa, int e, int row0, int rc, int kc, int utid,
-                                               MfRegs& R, bool part = false) {
+// Issue the register loads of the columns of chunk [kc, kc + 512) of one projection of expert e.  utid is the thread's
+// index within its unit.  Every load is issued unconditionally (a branch around a load makes the compiler wait for it
+// at the join); invalid lanes get an offset past their buffer, which reads 0, or a clamped index.
+__device__ __forceinline__ void mf_chunk_issue(const MfmaProj& pa, int e, int kc, int utid, MfRegs& R) {
   const tris_compact3_payload& p = pa.p;
   const int rank = p.rank;
-  const int wave = __builtin_amdgcn_readfirstlane(utid / kWave);  // wave-uniform
-  const int lane = utid % kWave;
   const int packed_rows = rank / 32;  // rank % 64 == 0
   const int pr0 = kc / 32;
   const int npr = (packed_rows - pr0) < kMfPR ? (packed_rows - pr0) : kMfPR;
-  uint32_t hid_bytes;
-  const __amdgpu_buffer_rsrc_t r_hid = mf_hidden_rsrc(pa, row0, rc, rank, &hid_bytes, part);
   const uint32_t col_bytes = static_cast<uint32_t>(rank) * 8u;
   const __amdgpu_buffer_rsrc_t r_col = make_rsrc(p.col_pack3 + static_cast<int64_t>(e) * rank, col_bytes);
-  const int32_t* cmap_e = p.c_map + static_cast<int64_t>(e) * packed_rows;
-  const int32_t* q2p_e = p.qweight2_sparse_prefix + static_cast<int64_t>(e) * (packed_rows + 1);
-  const int32_t* gidx_e = p.g_idx + static_cast<int64_t>(e) * rank;
-#pragma unroll
-  for (int h = 0; h < kMfRuns; ++h) {
-    const int r = 4 * h + wave;
-    R.xv[h] = bload128(r_hid, mf_hidden_voff(pa, row0, r, rc, kc + lane * 8, rank, hid_bytes), 0u);
-  }
+  gmem_i32* cmap_e = as_gmem(p.c_map + static_cast<int64_t>(e) * packed_rows);
+  gmem_i32* q2p_e = as_gmem(p.qweight2_sparse_prefix + static_cast<int64_t>(e) * (packed_rows + 1));
+  gmem_i32* gidx_e = as_gmem(p.g_idx + static_cast<int64_t>(e) * rank);
 #pragma unroll
   for (int h = 0; h < 2; ++h) {
     const int k = kc + utid + h * kMfThreads;
@@ -388,13 +353,11 @@ __device__ __forceinline__ void mf_chunk_issue(const MfmaProj& pa, int e, int ro
     R.cpv[h] = bload64(r_col, kv ? static_cast<uint32_t>(k) * 8u : col_bytes, 0u);
     R.cmt[h] = static_cast<uint32_t>(cmap_e[pr]);
     R.q2t[h] = q2p_e[pr];
-    R.gt[h] = kv ? gidx_e[k] : -1;
   }
   R.sbase0 = q2p_e[pr0];
-  R.send = q2p_e[pr0 + npr];
   // metadata: utid 64..71 -> group of K tile utid - 64; 72 / 73 -> salient prefix at the chunk's
   // start / end
-  const int32_t* mp = q2p_e + pr0;
+  gmem_i32* mp = q2p_e + pr0;
   if (utid >= 64 && utid < 72) {
     const int kt = kc + (utid - 64) * kTileK;
     mp = gidx_e + (kt < rank ? kt : rank - 1);
@@ -404,72 +367,153 @@ __device__ __forceinline__ void mf_chunk_issue(const MfmaProj& pa, int e, int ro
   R.mv = *mp;
 }
 
-// Write a unit's register-staged chunk to LDS (waits for those loads).  Salient columns get zero
-// C_d / C_nd, so the main pass gives them zero weights whatever their selector bits.
-__device__ __forceinline__ void mf_chunk_write(const MfmaProj& pa, int rc, int kc, int utid, const MfChunk& ch,
-                                               const MfRegs& R, bool natural = false, int sal_cap = kMfChunk,
-                                               bool part = false) {
+// Decode kernel: the columns of a unit's chunk, two neighbours a thread (2 utid and 2 utid + 1 of the chunk: one packed
+// row and, with uniform groups, one group), held between issue and write.
+struct MfColRegs {
+  uint4 cp;      // their col_pack3 entries
+  uint32_t cm;   // their packed row's salient word
+  int q2t;       // its salient prefix
+  int g;         // their group (g_idx)
+  int sbase0;    // salient prefix at the chunk's first packed row (the same in every lane)
+  int send;      // salient prefix at the chunk's end (the same in every lane)
+};
+__device__ __forceinline__ void mf_cols_issue(const MfmaProj& pa, int e, int kc, int utid, MfColRegs& R) {
   const tris_compact3_payload& p = pa.p;
   const int rank = p.rank;
-  const int G = p.num_groups;
-  const int wave = __builtin_amdgcn_readfirstlane(utid / kWave);  // wave-uniform
-  const int lane = utid % kWave;
-#pragma unroll
-  for (int h = 0; h < kMfRuns; ++h) {
-    const int r = 4 * h + wave;
-    if (r < rc && !part) {  // wave-uniform; partial sums are staged by mf_partials_stage
-      const int c = lane * 8;  // run start within the chunk (a multiple of 8)
-      // columns c + b and c + b + 4 (b < 4) are neighbours in the staged order
-      const uint32_t w[4] = {R.xv[h].x, R.xv[h].y, R.xv[h].z, R.xv[h].w};
-      const int base = (c & ~31) + ((c & 31) >> 2);
-#pragma unroll
-      for (int b = 0; b < 4; ++b) {
-        const uint32_t lo = (w[b >> 1] >> (16 * (b & 1))) & 0xFFFFu;
-        const uint32_t hi = (w[2 + (b >> 1)] >> (16 * (b & 1))) & 0xFFFFu;
-        *reinterpret_cast<uint32_t*>(&ch.xs[r * kMfXStride + base + 8 * b]) = lo | (hi << 16);
-      }
-    }
-  }
+  const int packed_rows = rank / 32;  // rank % 64 == 0
+  const int end = kc + kMfChunk < rank ? kc + kMfChunk : rank;
+  const __amdgpu_buffer_rsrc_t r_col =
+      make_rsrc(p.col_pack3 + static_cast<int64_t>(e) * rank, static_cast<uint32_t>(rank) * 8u);
+  const __amdgpu_buffer_rsrc_t r_cm =
+      make_rsrc(p.c_map + static_cast<int64_t>(e) * packed_rows, static_cast<uint32_t>(packed_rows) * 4u);
+  const __amdgpu_buffer_rsrc_t r_pre = make_rsrc(p.qweight2_sparse_prefix + static_cast<int64_t>(e) * (packed_rows + 1),
+                                                 static_cast<uint32_t>(packed_rows + 1) * 4u);
+  const __amdgpu_buffer_rsrc_t r_g = make_rsrc(p.g_idx + static_cast<int64_t>(e) * rank, static_cast<uint32_t>(rank) * 4u);
+  // columns past the rank read zeros (zero factors, not salient)
+  const uint32_t k = static_cast<uint32_t>(kc + 2 * utid);
+  R.cp = bload128(r_col, k * 8u, 0u);
+  R.cm = bload32(r_cm, (k >> 5) * 4u, 0u);
+  R.q2t = static_cast<int>(bload32(r_pre, (k >> 5) * 4u, 0u));
+  R.g = static_cast<int>(bload32(r_g, k * 4u, 0u));
+  R.sbase0 = static_cast<int>(bload32(r_pre, static_cast<uint32_t>(kc / 32) * 4u, 0u));
+  R.send = static_cast<int>(bload32(r_pre, static_cast<uint32_t>(end / 32) * 4u, 0u));
+}
+
+// Writes the columns to LDS (waits for their loads): the factors of the main pass, staged negated (-C * R rounds to
+// exactly -fp16(C * R), so a set qweight1 bit is the selectors' sign bit) and zero for salient columns, whatever their
+// selector bits; the salient slots; the K tiles' row-scale offsets; the zero columns of the rc staged rows.  sal_cap:
+// the slots staged (a payload whose prefix counts disagree with its salient map writes no slot past them).
+__device__ __forceinline__ void mf_cols_write(const MfmaProj& pa, int rc, int kc, int utid, const MfChunk& ch,
+                                              const MfColRegs& R, int sal_cap) {
+  const int rank = pa.p.rank;
+  const int G = pa.p.num_groups;
+  const int j = 2 * utid;
+  const int pos = (j & ~31) + mf_perm32(j & 31);  // the second column's is pos + 8
+  const bool gv = R.g >= 0 && R.g < G;
+  const int bit = j & 31;
+  const uint32_t sal = kc + j < rank ? (R.cm >> bit) & 3u : 0u;
+  const uint32_t cdn[2] = {R.cp.y ^ 0x80008000u, R.cp.w ^ 0x80008000u};  // C_d | C_nd << 16
 #pragma unroll
   for (int h = 0; h < 2; ++h) {
-    const int j = utid + h * kMfThreads;
-    const int k = kc + j;
-    const int pj = natural ? j : (j & ~31) + mf_perm32(j & 31);
-    const int bit = k & 31;
-    const uint32_t cm = R.cmt[h];
-    const bool sal = k < rank && ((cm >> bit) & 1u);
-    // staged negated (-C * R rounds to exactly -fp16(C * R)), so a set qweight1 bit is the selectors' sign bit
-    ch.cds[pj] = sal ? static_cast<uint16_t>(0) : static_cast<uint16_t>((R.cpv[h] >> 32) ^ 0x8000u);
-    ch.cns[pj] = sal ? static_cast<uint16_t>(0) : static_cast<uint16_t>((R.cpv[h] >> 48) ^ 0x8000u);
-    if (natural) ch.col_sal[j] = static_cast<uint32_t>(R.cpv[h]);
-    if (sal) {
-      const int q = R.q2t[h] - R.sbase0 + __popc(cm & ((1u << bit) - 1u));
-      if (natural) {
-        ch.sal_col[q] = static_cast<uint16_t>(j);
-        ch.sal_xi[q] = static_cast<uint16_t>((j & ~31) + mf_perm32(j & 31));
-        ch.sal_cp[q] = static_cast<uint32_t>(R.cpv[h]);
-      } else if (q >= 0 && q < sal_cap) {
-        // the column's group as the main pass takes it (uniform 64-column groups); an invalid group gives
-        // zero factors, as a K tile without a group does
-        const bool gv = R.gt[h] >= 0 && R.gt[h] < G;
-        ch.sal_w[q] = (static_cast<uint32_t>((j >> 5) * kMfWCols * 4) << 16) |
-                      (static_cast<uint32_t>((gv ? R.gt[h] : 0) * 8) << 8) | (static_cast<uint32_t>(bit - 15) & 31u);
-        ch.sal_xo[q] = static_cast<uint16_t>(pj * 2);
-        ch.sal_cp[q] = (gv ? static_cast<uint32_t>(R.cpv[h]) : 0u) ^ 0x80008000u;
-      }
-    }
+    const uint32_t v = (sal >> h) & 1u ? 0u : cdn[h];
+    ch.cds[pos + 8 * h] = static_cast<uint16_t>(v);
+    ch.cds[kMfChunk + pos + 8 * h] = static_cast<uint16_t>(v >> 16);
   }
-  if (!natural) {
+  // (a column that is not salient writes the spare slot sal_cap, so that no load is put off into a branch and waited
+  // for there, with every load issued after it)
+  int q = R.q2t - R.sbase0 + __popc(R.cm & ((1u << bit) - 1u));
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+    // the column's group as the main pass takes it (uniform 64-column groups); an invalid group gives
+    // zero factors, as a K tile without a group does
+    const bool is = ((sal >> h) & 1u) != 0u;
+    const int at = is && q >= 0 && q < sal_cap ? q : sal_cap;
+    ch.sal_w[at] = (static_cast<uint32_t>((j >> 6) * kMfWCols * 16 + ((j >> 5) & 1) * 8) << 16) |
+                   (static_cast<uint32_t>((gv ? R.g : 0) * 8) << 8) | (static_cast<uint32_t>(bit + h - 15) & 31u);
+    ch.sal_xo[at] = static_cast<uint16_t>((pos + 8 * h) * 2);
+    ch.sal_cp[at] = (gv ? (h ? R.cp.z : R.cp.x) : 0u) ^ 0x80008000u;
+    q += is ? 1 : 0;
+  }
+  if ((utid & 31) == 0) {  // the first column of K tile utid / 32
+    ch.goff[utid >> 5] = kc + j < rank && gv ? make_uint2(static_cast<uint32_t>(kMfWrs * 4 + R.g * 8 + 4), ~0u)
+                                             : make_uint2(0u, 0u);
+  }
+  if (utid < kMfSalWin) {
     // padding slots up to the last window's end read the zero activation column with zero factors
     const int nsal = R.send - R.sbase0;
     const int q = nsal + utid;
-    if (utid < kMfSalWin && q >= 0 && q < sal_cap && q < ((nsal + kMfSalWin - 1) & ~(kMfSalWin - 1))) {
+    if (q >= 0 && q < sal_cap && q < ((nsal + kMfSalWin - 1) & ~(kMfSalWin - 1))) {
       ch.sal_w[q] = 0u;
       ch.sal_xo[q] = static_cast<uint16_t>(kMfChunk * 2);
       ch.sal_cp[q] = 0x80008000u;
     }
     // the zero column (and its neighbour, so that row 0 holds an aligned zero word)
     if (utid < rc) *reinterpret_cast<uint32_t*>(&ch.xs[utid * kMfXStride + kMfChunk]) = 0u;
+  }
+}
+
+// Activation rows of a unit's chunk: wavefront `wave` loads rows 4 h + wave, a row's 512 columns 8 a lane.
+template <int kRuns>
+struct MfRowRegs {
+  uint4 xv[kRuns];
+};
+
+// Issue the loads of the row tile's rows: lane tok0 + r of roff holds the byte offset of row r in r_hid, or kMfOob (rows
+// past the tile, index entries that name no hidden row: they read zeros, as columns past the rank do).
+template <int kRuns>
+__device__ __forceinline__ void mf_rows_issue(__amdgpu_buffer_rsrc_t r_hid, int rank, int kc, int wave, int lane,
+                                              uint32_t roff, int tok0, MfRowRegs<kRuns>& R) {
+  const uint32_t col = kc + lane * 8 < rank ? static_cast<uint32_t>(kc + lane * 8) * 2u : kMfOob;
+#pragma unroll
+  for (int h = 0; h < kRuns; ++h) {
+    const int at = tok0 + 4 * h + wave;  // wave-uniform
+    const uint32_t ro = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(roff), at & (kWave - 1)));
+    R.xv[h] = bload128(r_hid, __builtin_elementwise_add_sat(ro, col), 0u);
+  }
+}
+
+// Writes the loaded rows to LDS in the staged order.
+template <int kRuns>
+__device__ __forceinline__ void mf_rows_write(const MfRowRegs<kRuns>& R, int rc, int wave, int lane, uint16_t* xs) {
+  const int c = lane * 8;  // run start within the chunk
+  uint16_t* const dst = xs + (c & ~31) + 2 * ((c >> 2) & 3) + ((c >> 4) & 1);
+#pragma unroll
+  for (int h = 0; h < kRuns; ++h) {
+    const int r = 4 * h + wave;
+    if (r < rc) {  // wave-uniform
+      const uint32_t w[4] = {R.xv[h].x, R.xv[h].y, R.xv[h].z, R.xv[h].w};
+#pragma unroll
+      for (int x = 0; x < 8; ++x) {  // column c + x
+        dst[r * kMfXStride + 8 * (x & 3) + 2 * (x >> 2)] = static_cast<uint16_t>(w[x >> 1] >> (16 * (x & 1)));
+      }
+    }
+  }
+}
+
+// Weight-stationary kernel: write the register-staged columns to LDS in natural order (waits for those loads).  Salient
+// columns get zero C_d / C_nd, so the main pass gives them zero weights whatever their selector bits.
+__device__ __forceinline__ void mf_chunk_write(const MfmaProj& pa, int kc, int utid, const MfChunk& ch,
+                                               const MfRegs& R) {
+  const tris_compact3_payload& p = pa.p;
+  const int rank = p.rank;
+  const int G = p.num_groups;
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+    const int j = utid + h * kMfThreads;
+    const int k = kc + j;
+    const int bit = k & 31;
+    const uint32_t cm = R.cmt[h];
+    const bool sal = k < rank && ((cm >> bit) & 1u);
+    // staged negated (-C * R rounds to exactly -fp16(C * R)), so a set qweight1 bit is the selectors' sign bit
+    ch.cds[j] = sal ? static_cast<uint16_t>(0) : static_cast<uint16_t>((R.cpv[h] >> 32) ^ 0x8000u);
+    ch.cns[j] = sal ? static_cast<uint16_t>(0) : static_cast<uint16_t>((R.cpv[h] >> 48) ^ 0x8000u);
+    ch.col_sal[j] = static_cast<uint32_t>(R.cpv[h]);
+    if (sal) {
+      const int q = R.q2t[h] - R.sbase0 + __popc(cm & ((1u << bit) - 1u));
+      ch.sal_col[q] = static_cast<uint16_t>(j);
+      ch.sal_xi[q] = static_cast<uint16_t>((j & ~31) + mf_perm32(j & 31));
+      ch.sal_cp[q] = static_cast<uint32_t>(R.cpv[h]);
+    }
   }
   if (utid >= 64 && utid < 72) {
     const bool tv = kc + (utid - 64) * kTileK < rank && R.mv >= 0 && R.mv < G;
@@ -559,90 +603,116 @@ __device__ __forceinline__ void mf_tile_issue(const MfmaProj& pa, int s, int e, 
   }
 }
 
-// Per-lane byte offsets of a wavefront's copies for chunk kc, output tile 0 (mf_wave_tile_issue adds the tile):
-// lane l copies packed row pr0 + 4 i + l / 16 (copy i adds whole rows), column 16 wave + l % 16.
-struct MfWaveOffsets {
-  uint32_t q1;   // into the expert's qweight1 [packed rows][N]
-  uint32_t dec;  // into the segment's predecoded blocks [packed rows / 2][tiles][128]
+// Where a wavefront's words of output tile 0 lie for chunk kc: expert e's tensors (wave-uniform; the tile's own
+// columns are added to the bases) and the lane's byte offsets.
+struct MfWaveSrc {
+  const uint32_t* q1;    // qweight1[e] [packed rows][N]
+  const uint32_t* dec;   // the segment's predecoded blocks [packed rows / 2][tiles][128]
+  const uint32_t* rs;    // row_pack3[e], the wavefront's columns of tile 0
+  uint32_t q1_bytes, dec_bytes;
+  int rs_cols;           // columns from the wavefront's first to the expert's last
+  uint32_t v_q1, v_dec;  // lane l: packed row kc / 32 + l / 4, columns 16 wave + 4 (l % 4) ..
 };
-__device__ __forceinline__ MfWaveOffsets mf_wave_offsets(const MfmaProj& pa, int kc, int wave, int lane) {
+__device__ __forceinline__ MfWaveSrc mf_wave_src(const MfmaProj& pa, int s, int e, int kc, int wave, int lane) {
   const tris_compact3_payload& p = pa.p;
   const int N = p.outfeatures;
-  const int nob = ceil_div(N, kTileOut);
-  const uint32_t pr = static_cast<uint32_t>(kc / 32 + lane / kMfWCols);
-  const uint32_t c = static_cast<uint32_t>(kMfWCols * wave + lane % kMfWCols);
-  MfWaveOffsets o;
-  o.q1 = (pr * N + c) * 4u;
-  o.dec = ((pr >> 1) * nob * kGrWords + (pr & 1u) * kTileOut + c) * 4u;
-  return o;
-}
-
-// The wavefront's LDS copies of its 16 columns of output tile ob for chunk kc: qweight1 and split words of the
-// chunk's packed rows (lane l of copy i: packed row 4 i + l / 16, column l % 16) and the columns' row-scale block.
-// Always MfWaveWords<kCompact>::kDma copies.  Nothing is masked: every offset is checked against its buffer's size (past it reads
-// zeros), and what lies inside it but past the chunk's rows or past column N (the next row's words, the next
-// tile's block) only feeds packed rows the compute skips or output columns that are not stored.  valid = false
-// (a prefetch with no tile to fetch, wave-uniform) empties the buffer ranges, so every copy reads zeros without a
-// memory access: a workgroup does not fetch the tile after its run, which another workgroup reads (likely through
-// another XCD's L2).
-template <bool kCompact>
-__device__ __forceinline__ void mf_wave_tile_issue(const MfmaProj& pa, int s, int e, int ob, const MfWaveOffsets& o,
-                                                   int lane, int wave, const MfWaveBuf& wb, bool valid = true) {
-  const tris_compact3_payload& p = pa.p;
-  const int N = p.outfeatures;
-  const int G = p.num_groups;
   const int packed_rows = p.rank / 32;
   const int nob = ceil_div(N, kTileOut);
   const int nblk = (packed_rows / 2) * nob;
-  const uint32_t q1_bytes = static_cast<uint32_t>(packed_rows) * N * 4u;
-  const uint32_t dec_bytes = static_cast<uint32_t>(nblk) * kGrWords * 4u;
-  const __amdgpu_buffer_rsrc_t r_q1 =
-      make_rsrc(p.qweight1 + static_cast<int64_t>(e) * packed_rows * N, valid ? q1_bytes : 0u);
-  const __amdgpu_buffer_rsrc_t r_dec =
-      make_rsrc(pa.decoded + static_cast<int64_t>(s) * nblk * kGrWords, valid ? dec_bytes : 0u);
+  const uint32_t pr = static_cast<uint32_t>(kc / 32 + lane / 4);
+  const uint32_t c = static_cast<uint32_t>(kMfWCols * wave + 4 * (lane % 4));
+  MfWaveSrc w;
+  w.q1 = reinterpret_cast<const uint32_t*>(p.qweight1) + static_cast<int64_t>(e) * packed_rows * N;
+  w.dec = reinterpret_cast<const uint32_t*>(pa.decoded) + static_cast<int64_t>(s) * nblk * kGrWords;
+  w.rs = reinterpret_cast<const uint32_t*>(p.row_pack3) +
+         (static_cast<int64_t>(e) * N + kMfWCols * wave) * (2 * p.num_groups);
+  w.q1_bytes = static_cast<uint32_t>(packed_rows) * N * 4u;
+  w.dec_bytes = static_cast<uint32_t>(nblk) * kGrWords * 4u;
+  w.rs_cols = N - kMfWCols * wave;
+  w.v_q1 = (pr * N + c) * 4u;
+  w.v_dec = ((pr >> 1) * nob * kGrWords + (pr & 1u) * kTileOut + c) * 4u;
+  return w;
+}
+
+// kWords consecutive words at byte offset voff: one load, or with kSingle one a word (a load that straddles the buffer's
+// end, for column counts that are no multiple of 4, must still return the words inside it).
+template <int kWords, bool kSingle>
+__device__ __forceinline__ void bload_words(__amdgpu_buffer_rsrc_t r, uint32_t voff, uint32_t* dst) {
+  if constexpr (kSingle) {
 #pragma unroll
-  for (int i = 0; i < kMfPR / 4; ++i) {
-    dma32(r_q1, wb.q1 + i * kWave, o.q1 + static_cast<uint32_t>(4 * i * N + ob * kTileOut) * 4u, 0u);
-    dma32(r_dec, wb.gw + i * kWave, o.dec + static_cast<uint32_t>((2 * i * nob + ob) * kGrWords) * 4u, 0u);
-  }
-  // row_pack3[e][n0 .. n0 + 15][0 .. G - 1] is one contiguous run of 16 G pairs (32 G words); a lane past it reads
-  // zeros without a memory access (an offset past the buffer), as do columns past the expert
-  const int n0 = ob * kTileOut + kMfWCols * wave;
-  const int ncols = valid ? N - n0 : 0;
-  const uint32_t rs_bytes = ncols > 0 ? static_cast<uint32_t>(ncols) * G * 8u : 0u;
-  const __amdgpu_buffer_rsrc_t r_rs =
-      make_rsrc(p.row_pack3 + (static_cast<int64_t>(e) * N + (ncols > 0 ? n0 : 0)) * G, rs_bytes);
-  const int rs_words = kMfWCols * 2 * G;
-#pragma unroll
-  for (int i = 0; i < MfWaveWords<kCompact>::kRsCopies; ++i) {
-    const int w = i * kWave + lane;
-    dma32(r_rs, wb.rs + i * kWave, w < rs_words ? static_cast<uint32_t>(w) * 4u : rs_bytes, 0u);
+    for (int i = 0; i < kWords; ++i) dst[i] = bload32(r, voff + 4u * i, 0u);
+  } else if constexpr (kWords == 4) {
+    const uint4 v = bload128(r, voff, 0u);
+    dst[0] = v.x, dst[1] = v.y, dst[2] = v.z, dst[3] = v.w;
+  } else {
+    const auto v = __builtin_amdgcn_raw_buffer_load_b64(r, voff, 0u, 0);
+    dst[0] = v[0], dst[1] = v[1];
   }
 }
 
-// One projection over one staged chunk and output tile [n0, n0 + 64): accumulates rows 4 * kg + v,
-// column n0 + 16 * wave + lane % 16 of x . W^T into acc.  xrow is the staged activation row this
-// lane's A operand reads.
-// Exact B operand of the lane's column for packed row j: the 8 weights k = kg + 4m.  Per packed row the
-// lane builds nibble selectors: bit 1 = this term is used, bit 3 = the column's qweight1 bit (shared by both
-// terms; the unused term is a signed zero); with the staged factors negated, w = fma(sd, fp16(-C_d * R_d),
-// sn * fp16(-C_nd * R_nd)) is -fp16(C_j * R_j) where the bit is clear and +fp16(C_j * R_j) where it is set.
+// Issues the wavefront's loads of its 16 columns of output tile ob: one 16-byte load a lane for the packed rows'
+// qweight1 words, one for their split words, one for the row scales (16 / 16 / 8 or 16 bytes; kSingle: a word at a time).
+// Nothing is masked: an offset past its buffer reads zeros, and what lies inside it but past the chunk's rows, the
+// groups or column N (the next row's words, the next tile's block) only feeds packed rows the compute skips, scales it
+// does not read or output columns that are not stored.  valid = false (a prefetch with no tile to fetch, wave-uniform)
+// empties the buffers, so every load reads zeros without a memory access: a workgroup does not fetch the tile after
+// its run, which another workgroup reads (likely through another XCD's L2).
+template <bool kCompact, bool kSingle>
+__device__ __forceinline__ void mf_wave_tile_issue(const MfWaveSrc& w, int G, int ob, int lane,
+                                                   MfWaveRegs<kCompact>& r, bool valid = true) {
+  constexpr int kRsLane = MfWaveWords<kCompact>::kRsLane;
+  const uint32_t col = static_cast<uint32_t>(ob) * kTileOut;
+  const __amdgpu_buffer_rsrc_t r_q1 = make_rsrc(w.q1 + col, valid ? w.q1_bytes - col * 4u : 0u);
+  const __amdgpu_buffer_rsrc_t r_dec =
+      make_rsrc(w.dec + static_cast<uint32_t>(ob) * kGrWords, valid ? w.dec_bytes - static_cast<uint32_t>(ob) * kGrWords * 4u : 0u);
+  const int ncols = valid ? w.rs_cols - static_cast<int>(col) : 0;  // the wavefront's columns to the expert's last
+  const __amdgpu_buffer_rsrc_t r_rs = make_rsrc(w.rs + (ncols > 0 ? static_cast<int64_t>(col) * 2 * G : 0),
+                                                ncols > 0 ? static_cast<uint32_t>(ncols) * G * 8u : 0u);
+  bload_words<4, kSingle>(r_q1, w.v_q1, r.q);
+  bload_words<4, kSingle>(r_dec, w.v_dec, r.g);
+  bload_words<kRsLane, kSingle>(r_rs, static_cast<uint32_t>(lane * kRsLane) * 4u, r.rs);
+}
+
+// Writes the loaded words to the wavefront's LDS words wb of that tile (this waits for the loads).
+template <bool kCompact>
+__device__ __forceinline__ void mf_wave_tile_write(const MfWaveRegs<kCompact>& r, int lane, uint32_t* wb) {
+  constexpr int kRsLane = MfWaveWords<kCompact>::kRsLane;
+  const int row = lane / 4;
+  uint32_t* dst = wb + kMfWw + ((row >> 1) * kMfWCols + 4 * (lane % 4)) * 4 + (row & 1) * 2;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) *reinterpret_cast<uint2*>(dst + 4 * i) = make_uint2(r.q[i], r.g[i]);
+  if constexpr (kRsLane == 4) {
+    *reinterpret_cast<uint4*>(wb + kMfWrs + lane * 4) = make_uint4(r.rs[0], r.rs[1], r.rs[2], r.rs[3]);
+  } else {
+    *reinterpret_cast<uint2*>(wb + kMfWrs + lane * 2) = make_uint2(r.rs[0], r.rs[1]);
+  }
+}
+
+// Exact B operand of the lane's column for packed row j: the 8 weights k = kg + 4 i and kg + 4 i + 16 (i < 4).  Per pair
+// a 16-bit mask of the two split bits (shifted to each half's top bit, then an arithmetic shift) picks fp16(-C_d * R_d)
+// or fp16(-C_nd * R_nd), and the two qweight1 bits, at each half's bit 0, times 0x8000 are added to the halves: the sum
+// mod 2^16 flips the sign where the bit is set, to +fp16(C * R).  left = 3 - kg; right = kg.
+// Bound by VALU issue.  Picking the terms by fp4 selectors (two v_cvt_scalef32_pk_f16_fp4, a product and a
+// fused multiply-add a pair) took 148 cycles a packed row with three wavefronts a SIMD, this form 132.
 __device__ __forceinline__ f16x8 mf_row_b(uint32_t qw, uint32_t gw, const uint4& cdv, const uint4& cnv, uint32_t rs2,
-                                          uint32_t shl, uint32_t rot) {
-  const f16x2 rd2 = u32_as_f16x2(__builtin_amdgcn_perm(rs2, rs2, 0x01000100u));
-  const f16x2 rn2 = u32_as_f16x2(__builtin_amdgcn_perm(rs2, rs2, 0x03020302u));
+                                          uint32_t left, uint32_t right) {
+  const f16x2 r = u32_as_f16x2(rs2);
+  const f16x2 rd2 = __builtin_shufflevector(r, r, 0, 0);  // (operand selects of the packed products)
+  const f16x2 rn2 = __builtin_shufflevector(r, r, 1, 1);
   const uint32_t cd[4] = {cdv.x, cdv.y, cdv.z, cdv.w};
   const uint32_t cn[4] = {cnv.x, cnv.y, cnv.z, cnv.w};
-  const uint32_t sgn3 = (qw << shl) & 0x88888888u;  // fp4 -1.0 on a negated factor where the bit is set
-  const uint32_t sd = (__builtin_rotateright32(gw, rot) & 0x22222222u) | sgn3;  // d term: fp4 +-1.0, else +-0
-  const uint32_t sn = sd ^ 0x22222222u;                                        // nd term: the others
+  const uint32_t g = gw << left;
+  const uint32_t q = qw >> right;
   uint32_t b[4];
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
-    const f16x2 pd = u32_as_f16x2(cd[i]) * rd2;
-    const f16x2 pn = u32_as_f16x2(cn[i]) * rn2;
-    const f16x2 tn = fp4x2_to_f16x2(sn, i) * pn;
-    b[i] = f16x2_as_u32(__builtin_elementwise_fma(fp4x2_to_f16x2(sd, i), pd, tn));
+    const uint32_t pd = f16x2_as_u32(u32_as_f16x2(cd[i]) * rd2);
+    const uint32_t pn = f16x2_as_u32(u32_as_f16x2(cn[i]) * rn2);
+    uint32_t m, w;
+    asm("v_pk_ashrrev_i16 %0, 15, %1 op_sel_hi:[0,1]" : "=v"(m) : "v"(g << (12 - 4 * i)));
+    w = ((pd ^ pn) & m) ^ pn;
+    asm("v_pk_mad_u16 %0, %1, %2, %0" : "+v"(w) : "v"(q >> (4 * i)), "s"(0x80008000u));
+    b[i] = w;
   }
   return __builtin_bit_cast(f16x8, make_uint4(b[0], b[1], b[2], b[3]));
 }
@@ -659,8 +729,9 @@ __device__ __forceinline__ uint32_t spread8(uint32_t b) {
 // spread to one nibble each.
 __device__ __forceinline__ f16x8 mf_row_b_nat(uint32_t qw, uint32_t gw, const uint4& cdv, const uint4& cnv,
                                               uint32_t rs2, int kg) {
-  const f16x2 rd2 = u32_as_f16x2(__builtin_amdgcn_perm(rs2, rs2, 0x01000100u));
-  const f16x2 rn2 = u32_as_f16x2(__builtin_amdgcn_perm(rs2, rs2, 0x03020302u));
+  const f16x2 r = u32_as_f16x2(rs2);
+  const f16x2 rd2 = __builtin_shufflevector(r, r, 0, 0);  // (operand selects of the packed products)
+  const f16x2 rn2 = __builtin_shufflevector(r, r, 1, 1);
   const uint32_t cd[4] = {cdv.x, cdv.y, cdv.z, cdv.w};
   const uint32_t cn[4] = {cnv.x, cnv.y, cnv.z, cnv.w};
   const uint32_t q4 = spread8(__builtin_amdgcn_ubfe(qw, 8u * kg, 8u));
@@ -707,202 +778,224 @@ __device__ __forceinline__ void mf_salient_weights(const MfChunk& ch, const MfTi
 }
 
 // Both MFMA operands of the salient window starting at slot w0, built in registers: lane (i16, kg) takes window
-// slots 8 kg .. 8 kg + 7.  bv holds the exact fp16 weights of its column, w = fp16(+-fp16(C0 * R0) +-
-// fp16(C1 * R1)) (both products in one packed multiply), and av its activation row xr at those slots'
+// slots 8 kg .. 8 kg + 7.  bv[b] holds the exact fp16 weights of its column of tile b, w = fp16(+-fp16(C0 * R0) +-
+// fp16(C1 * R1)) (both products in one packed multiply), and av[m] its activation row xr[m] at those slots'
 // columns.  The staged slot words carry every column-dependent offset, so a slot costs three LDS reads (its
 // qweight1 word, its group's R0 | R1, its activation) and no masking: padding slots read zero factors and the
 // zero activation column.  q1_lane / rs_lane: the byte offsets of the lane's column in the wavefront's qweight1
-// rows and in its row-scale block; q2w: the lane's qweight2_sparse words of rows (sbase0 + w0) / 32 and the next
+// words and in its row-scale block (of wb, kStride words a tile); q2w: the lane's qweight2_sparse words of rows (sbase0 + w0) / 32 and the next
 // (a window spans at most two), q2off = (sbase0 + w0) % 32 + 8 kg the bit of slot 0 in q2w[0] | q2w[1] << 32.
-__device__ __forceinline__ void mf_salient_operands(const MfChunk& ch, const MfWaveBuf& tb, const uint16_t* xr,
-                                                    uint32_t q1_lane, uint32_t rs_lane, int kg, int w0, int q2off,
-                                                    const uint32_t q2w[2], f16x8& av, f16x8& bv) {
+template <int kNs, int kRt, int kStride>
+__device__ __forceinline__ void mf_salient_operands(const MfChunk& ch, const uint32_t* wb,
+                                                    const uint16_t* const (&xr)[kRt], uint32_t q1_lane,
+                                                    uint32_t rs_lane, int kg, int w0, int q2off,
+                                                    const uint32_t (&q2w)[kNs][2], f16x8 (&av)[kRt],
+                                                    f16x8 (&bv)[kNs]) {
   const int s0 = w0 + 8 * kg;  // a multiple of 8: the slot vectors are 16-byte aligned
   const uint4 swa = *reinterpret_cast<const uint4*>(&ch.sal_w[s0]);
   const uint4 swb = *reinterpret_cast<const uint4*>(&ch.sal_w[s0 + 4]);
   const uint4 xov = *reinterpret_cast<const uint4*>(&ch.sal_xo[s0]);
   const uint32_t sw[8] = {swa.x, swa.y, swa.z, swa.w, swb.x, swb.y, swb.z, swb.w};
   const uint32_t xo[4] = {xov.x, xov.y, xov.z, xov.w};
-  const unsigned char* q1b = reinterpret_cast<const unsigned char*>(tb.q1) + q1_lane;
-  const unsigned char* rsb = reinterpret_cast<const unsigned char*>(tb.rs) + rs_lane;
-  const unsigned char* xb = reinterpret_cast<const unsigned char*>(xr);
-  uint32_t w1v[8], rrv[8], a16[8];
+  uint32_t w1v[kNs][8], rrv[kNs][8], a16[kRt][8];
 #pragma unroll
-  for (int u = 0; u < 8; ++u) {  // all 24 reads issued before any is used
-    w1v[u] = *reinterpret_cast<const uint32_t*>(q1b + (sw[u] >> 16));
-    rrv[u] = *reinterpret_cast<const uint32_t*>(rsb + ((sw[u] >> 8) & 0xFFu));
-    a16[u] = *reinterpret_cast<const uint16_t*>(xb + ((xo[u / 2] >> (16 * (u & 1))) & 0xFFFFu));
+  for (int u = 0; u < 8; ++u) {  // every read issued before any is used
+#pragma unroll
+    for (int b = 0; b < kNs; ++b) {
+      const unsigned char* q1b = reinterpret_cast<const unsigned char*>(wb + b * kStride + kMfWw) + q1_lane;
+      const unsigned char* rsb = reinterpret_cast<const unsigned char*>(wb + b * kStride + kMfWrs) + rs_lane;
+      w1v[b][u] = *reinterpret_cast<const uint32_t*>(q1b + (sw[u] >> 16));
+      rrv[b][u] = *reinterpret_cast<const uint32_t*>(rsb + ((sw[u] >> 8) & 0xFFu));
+    }
+#pragma unroll
+    for (int m = 0; m < kRt; ++m) {
+      const unsigned char* xb = reinterpret_cast<const unsigned char*>(xr[m]);
+      a16[m][u] = *reinterpret_cast<const uint16_t*>(xb + ((xo[u / 2] >> (16 * (u & 1))) & 0xFFFFu));
+    }
   }
   const uint4 cpa = *reinterpret_cast<const uint4*>(&ch.sal_cp[s0]);
   const uint4 cpb = *reinterpret_cast<const uint4*>(&ch.sal_cp[s0 + 4]);
   const uint32_t cp[8] = {cpa.x, cpa.y, cpa.z, cpa.w, cpb.x, cpb.y, cpb.z, cpb.w};
-  // qweight2_sparse bits of the 8 slots: bit u of q2lo
-  const uint32_t q2lo = static_cast<uint32_t>(((static_cast<uint64_t>(q2w[1]) << 32) | q2w[0]) >> q2off);
-  uint32_t t[8];
 #pragma unroll
-  for (int u = 0; u < 8; ++u) {
-    // staged factors have both signs flipped; flip back where the qweight1 (bit 15) / qweight2 (bit 31) bit is
-    // set (the positive weights)
-    const uint32_t rot = __builtin_amdgcn_alignbit(w1v[u], w1v[u], sw[u]);  // column's bit at bit 15
-    const uint32_t pos = (rot & 0x8000u) | ((q2lo << (31 - u)) & 0x80000000u);
-    t[u] = f16x2_as_u32(u32_as_f16x2(cp[u]) * u32_as_f16x2(rrv[u])) ^ pos;
-  }
-  uint32_t wb[4], ab[4];
+  for (int b = 0; b < kNs; ++b) {
+    // qweight2_sparse bits of the 8 slots: bit u of q2lo
+    const uint32_t q2lo = static_cast<uint32_t>(((static_cast<uint64_t>(q2w[b][1]) << 32) | q2w[b][0]) >> q2off);
+    uint32_t t[8];
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const uint32_t lo = __builtin_amdgcn_perm(t[2 * i + 1], t[2 * i], 0x05040100u);  // the C0 R0 terms
-    const uint32_t hi = __builtin_amdgcn_perm(t[2 * i + 1], t[2 * i], 0x07060302u);  // the C1 R1 terms
-    wb[i] = f16x2_as_u32(u32_as_f16x2(lo) + u32_as_f16x2(hi));
-    ab[i] = a16[2 * i] | (a16[2 * i + 1] << 16);
+    for (int u = 0; u < 8; ++u) {
+      // staged factors have both signs flipped; flip back where the qweight1 (bit 15) / qweight2 (bit 31) bit is
+      // set (the positive weights)
+      const uint32_t rot = __builtin_amdgcn_alignbit(w1v[b][u], w1v[b][u], sw[u]);  // column's bit at bit 15
+      const uint32_t pos = (rot & 0x8000u) | ((q2lo << (31 - u)) & 0x80000000u);
+      t[u] = f16x2_as_u32(u32_as_f16x2(cp[u]) * u32_as_f16x2(rrv[b][u])) ^ pos;
+    }
+    uint32_t wb[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const uint32_t lo = __builtin_amdgcn_perm(t[2 * i + 1], t[2 * i], 0x05040100u);  // the C0 R0 terms
+      const uint32_t hi = __builtin_amdgcn_perm(t[2 * i + 1], t[2 * i], 0x07060302u);  // the C1 R1 terms
+      wb[i] = f16x2_as_u32(u32_as_f16x2(lo) + u32_as_f16x2(hi));
+    }
+    bv[b] = __builtin_bit_cast(f16x8, make_uint4(wb[0], wb[1], wb[2], wb[3]));
   }
-  av = __builtin_bit_cast(f16x8, make_uint4(ab[0], ab[1], ab[2], ab[3]));
-  bv = __builtin_bit_cast(f16x8, make_uint4(wb[0], wb[1], wb[2], wb[3]));
+#pragma unroll
+  for (int m = 0; m < kRt; ++m) {
+    uint32_t ab[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) ab[i] = a16[m][2 * i] | (a16[m][2 * i + 1] << 16);
+    av[m] = __builtin_bit_cast(f16x8, make_uint4(ab[0], ab[1], ab[2], ab[3]));
+  }
 }
 
 // The lane's qweight2_sparse words of the chunk's first salient window (a window of kMfSalWin salient
 // columns spans at most two qweight2_sparse rows), for output column n.  Issued before the next tile's
 // LDS copies so that waiting for them does not wait for the copies.
-// A staged chunk's metadata in scalar registers: the group of each K tile (-1: none), the chunk's first
-// salient index and its salient count.  One LDS round trip.
+// A staged chunk's first salient index and its salient count, in scalar registers, the count held to the slots staged.
 struct MfChunkMeta {
-  int g[kMfTiles];
   int sbase0, num_sal;
 };
-__device__ __forceinline__ MfChunkMeta mf_chunk_meta(const MfChunk& ch) {
-  const int4 m0 = *reinterpret_cast<const int4*>(&ch.meta[0]);
-  const int4 m1 = *reinterpret_cast<const int4*>(&ch.meta[4]);
-  const int4 m2 = *reinterpret_cast<const int4*>(&ch.meta[8]);
-  const int gv[kMfTiles] = {m0.x, m0.y, m0.z, m0.w, m1.x, m1.y, m1.z, m1.w};
-  MfChunkMeta m;
-#pragma unroll
-  for (int t = 0; t < kMfTiles; ++t) m.g[t] = __builtin_amdgcn_readfirstlane(gv[t]);
-  m.sbase0 = __builtin_amdgcn_readfirstlane(m2.x);
-  m.num_sal = __builtin_amdgcn_readfirstlane(m2.y) - m.sbase0;
-  return m;
+__device__ __forceinline__ MfChunkMeta mf_chunk_meta(const MfColRegs& R, int sal_cap) {
+  MfChunkMeta r;
+  r.sbase0 = __builtin_amdgcn_readfirstlane(R.sbase0);
+  const int n = __builtin_amdgcn_readfirstlane(R.send) - r.sbase0;
+  r.num_sal = n < 0 ? 0 : (n < sal_cap ? n : sal_cap);
+  return r;
 }
 
-__device__ __forceinline__ void mf_q2_issue(const MfmaProj& pa, int e, int n, const MfChunkMeta& cm,
-                                            uint32_t q2w[2]) {
-  const tris_compact3_payload& p = pa.p;
-  const int N = p.outfeatures;
-  const int sbase0 = cm.sbase0;
-  const int num_sal = cm.num_sal;
-  const int q2rows = p.qweight2_sparse_rows;
-  const uint32_t q2_bytes = static_cast<uint32_t>(q2rows) * N * 4u;
-  const __amdgpu_buffer_rsrc_t r_q2 = make_rsrc(p.qweight2_sparse + static_cast<int64_t>(e) * q2rows * N, q2_bytes);
-  const uint32_t v_q2 = n < N ? static_cast<uint32_t>(n) * 4u : q2_bytes;
+// q2: the expert's qweight2_sparse [q2rows][N].
+__device__ __forceinline__ void mf_q2_issue(const uint32_t* q2, int q2rows, int N, int n, const MfChunkMeta& cm,
+                                            uint32_t (&q2w)[2]) {
+  const uint32_t v_q2 = n < N ? static_cast<uint32_t>(n) * 4u : kMfOob;
 #pragma unroll
   for (int h = 0; h < 2; ++h) {
-    const int row = (sbase0 >> 5) + h;
-    const bool rv = num_sal > 0 && row < q2rows;
-    q2w[h] = bload32(r_q2, rv ? v_q2 : q2_bytes, static_cast<uint32_t>(rv ? row : 0) * N * 4u);
+    // a row past the last: an empty resource
+    const int row = (cm.sbase0 >> 5) + h;
+    const bool rv = cm.num_sal > 0 && row < q2rows;
+    const __amdgpu_buffer_rsrc_t r_q2 = make_rsrc(q2 + (rv ? static_cast<int64_t>(row) * N : 0),
+                                                  rv ? static_cast<uint32_t>(N) * 4u : 0u);
+    q2w[h] = bload32(r_q2, v_q2, 0u);
   }
 }
 
-__device__ __forceinline__ f32x4 mf_compute(const MfmaProj& pa, int e, int kc, int n0, int xrow, int utid,
-                                            const MfChunk& ch, const MfChunkMeta& cm, const MfWaveBuf& tb,
-                                            const uint32_t q2w0[2], f32x4 acc) {
-  const tris_compact3_payload& p = pa.p;
-  const int N = p.outfeatures;
-  const int rank = p.rank;
-  const int G = p.num_groups;
-  const int wave = __builtin_amdgcn_readfirstlane(utid / kWave);  // wave-uniform
-  const int lane = utid % kWave;
+// kNs output tiles over one staged chunk: adds rows 16 m + 4 kg + v, column n[b] of x . W^T to acc[b][m].  Every
+// activation and column-factor read from LDS feeds all kNs tiles and every weight built all kRt row sub-tiles.
+// xr[m]: the staged activation row this lane's A operand of sub-tile m reads.
+//
+// The K loop stays rolled, two packed rows (a K tile) an iteration.  A launch starts with a cold instruction cache, and
+// its workgroups share few passes over the code: unrolled over the chunk, a pass was about 8 KB of instructions a tile
+// and the first one of each wavefront took 20000 cycles against 8400 for the next (T = 16 gate/up; timestamps
+// in the kernel), the difference being instruction fetch.
+template <int kNs, int kRt, int kStride>
+__device__ __forceinline__ void mf_compute(const uint32_t* q2, int q2rows, int N, int rank, int G, int kc,
+                                           const int (&n)[kNs], const uint16_t* const (&xr)[kRt], int lane,
+                                           const MfChunk& ch, const MfChunkMeta& cm, const uint32_t* wb,
+                                           const uint32_t (&q2w0)[kNs][2], f32x4 (&acc)[kNs][kRt]) {
   const int i16 = lane % 16;   // MFMA column within the wave's 16 outputs / A row
   const int kg = lane / 16;    // MFMA k group: columns k = kg (mod 4) of every packed row
-  const int tc = 16 * wave + i16;
-  const int n = n0 + tc;
-  const int packed_rows = rank / 32;
-  const int pr0 = kc / 32;
-  const int npr = (packed_rows - pr0) < kMfPR ? (packed_rows - pr0) : kMfPR;
-  const uint16_t* xr = ch.xs + xrow * kMfXStride;
+  const int nt = (rank - kc) / kTileK < kMfTiles ? (rank - kc) / kTileK : kMfTiles;  // K tiles (rank % 64 == 0)
 
-  // salient columns of the chunk; the first window's qweight2_sparse words come in q2w0
-  const int sbase0 = cm.sbase0;
-  const int num_sal = cm.num_sal;
-  const int q2rows = p.qweight2_sparse_rows;
-  const uint32_t q2_bytes = static_cast<uint32_t>(q2rows) * N * 4u;
-  const __amdgpu_buffer_rsrc_t r_q2 =
-      make_rsrc(p.qweight2_sparse + static_cast<int64_t>(e) * q2rows * N, q2_bytes);
-  const uint32_t v_q2 = n < N ? static_cast<uint32_t>(n) * 4u : q2_bytes;
-
-  // ---- MFMA over the chunk's packed rows (salient columns have zero factors here).  Per packed row
-  // the lane builds the nibble selectors of its 8 columns k = kg + 4m: bit 1 = this term is used,
-  // bit 3 = negative (shared by both terms; the unused term is a signed zero).  The LDS reads of row
-  // j + 1 are issued before row j is computed.
-  const uint32_t rot = static_cast<uint32_t>(kg - 1) & 31u;  // rotate right: bit kg + 4m -> 4m + 1
-  const uint32_t shl = static_cast<uint32_t>(3 - kg);        // shift left:   bit kg + 4m -> 4m + 3
+  // ---- MFMA over the chunk's packed rows (salient columns have zero factors here).  Each packed row's LDS reads
+  // are issued as soon as the same row of the K tile before is computed.
   // the lane's column in the wavefront's row-scale block [16 columns][G][R0 | R1, R_d | R_nd]
   const uint32_t rs_lane = static_cast<uint32_t>(i16 * G * 8);
-  // R_d | R_nd << 16 of each K tile's group for this column; a tile without a group reads the buffer's zero
-  // word.  The offsets are selected, not the pointers, so every read is known to address this buffer and
-  // need not wait for copies into the other.
-  uint32_t rdn[kMfTiles];
-  const uint32_t zero_off = static_cast<uint32_t>(reinterpret_cast<const unsigned char*>(tb.zero) -
-                                                  reinterpret_cast<const unsigned char*>(tb.rs));
+  const uint32_t* wp = wb + kMfWw + i16 * 4;
+  const uint16_t* cp = ch.cds + 8 * kg;  // C_nd follows C_d
+  const uint16_t* xp[kRt];
 #pragma unroll
-  for (int t = 0; t < kMfTiles; ++t) {
-    const int g = cm.g[t];
-    const uint32_t off = g >= 0 ? rs_lane + static_cast<uint32_t>(g) * 8u + 4u : zero_off;
-    rdn[t] = *reinterpret_cast<const uint32_t*>(reinterpret_cast<const unsigned char*>(tb.rs) + off);
-  }
+  for (int m = 0; m < kRt; ++m) xp[m] = xr[m] + 8 * kg;
   struct Row {
-    uint32_t qw, gw;
-    uint4 av, cd, cn;
+    uint2 w[kNs];
+    uint4 av[kRt], cd, cn;
   };
-  auto load_row = [&](int j) {
+  auto load_row = [&](int h) {
     Row r;
-    const int kl = j * 32 + 8 * kg;
-    r.qw = tb.q1[j * kMfWCols + i16];
-    r.gw = tb.gw[j * kMfWCols + i16];
-    r.av = *reinterpret_cast<const uint4*>(&xr[kl]);
-    r.cd = *reinterpret_cast<const uint4*>(&ch.cds[kl]);
-    r.cn = *reinterpret_cast<const uint4*>(&ch.cns[kl]);
+#pragma unroll
+    for (int b = 0; b < kNs; ++b) r.w[b] = *reinterpret_cast<const uint2*>(wp + b * kStride + 2 * h);
+#pragma unroll
+    for (int m = 0; m < kRt; ++m) r.av[m] = *reinterpret_cast<const uint4*>(xp[m] + 32 * h);
+    r.cd = *reinterpret_cast<const uint4*>(cp + 32 * h);
+    r.cn = *reinterpret_cast<const uint4*>(cp + kMfChunk + 32 * h);
     return r;
   };
-  auto row_mfma = [&](const Row& r, uint32_t rs2) {
-    acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, r.av),
-                                                 mf_row_b(r.qw, r.gw, r.cd, r.cn, rs2, shl, rot), acc, 0, 0, 0);
+  auto row_mfma = [&](const Row& r, const uint32_t (&rs2)[kNs]) {
+#pragma unroll
+    for (int b = 0; b < kNs; ++b) {
+      const f16x8 bv = mf_row_b(r.w[b].x, r.w[b].y, r.cd, r.cn, rs2[b], static_cast<uint32_t>(3 - kg), static_cast<uint32_t>(kg));
+#pragma unroll
+      for (int m = 0; m < kRt; ++m) {
+        acc[b][m] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, r.av[m]), bv, acc[b][m], 0, 0, 0);
+      }
+    }
   };
-  if (npr == kMfPR) {  // a full chunk
-    Row cur = load_row(0);
+  // R_d | R_nd << 16 of a K tile's group for this lane's columns
+  auto load_rs = [&](uint2 go, uint32_t (&rs2)[kNs]) {
+    const uint32_t off = (rs_lane & go.y) + go.x;
 #pragma unroll
-    for (int j = 0; j < kMfPR; ++j) {
-      Row nxt = cur;
-      if (j + 1 < kMfPR) nxt = load_row(j + 1);  // compile-time condition
-      row_mfma(cur, rdn[j / 2]);
-      cur = nxt;
+    for (int b = 0; b < kNs; ++b) {
+      rs2[b] = *reinterpret_cast<const uint32_t*>(reinterpret_cast<const unsigned char*>(wb + b * kStride) + off);
     }
-  } else {
+  };
+  uint32_t rs2[kNs];
+  load_rs(ch.goff[0], rs2);
+  uint2 go = ch.goff[nt > 1 ? 1 : 0];
+  Row r0 = load_row(0), r1 = load_row(1);
+#pragma unroll 1
+  for (int t = 0; t < nt; ++t) {
+    const int step = t + 1 < nt ? 1 : 0;  // the last iteration reads its own K tile again (not used)
+    wp += step * 2 * kMfWCols * 2;
+    cp += step * kTileK;
 #pragma unroll
-    for (int j = 0; j < kMfPR; ++j) {
-      if (j < npr) row_mfma(load_row(j), rdn[j / 2]);  // uniform
-    }
+    for (int m = 0; m < kRt; ++m) xp[m] += step * kTileK;
+    uint32_t rn[kNs];
+    load_rs(go, rn);
+    go = ch.goff[t + 2 < nt ? t + 2 : nt - 1];
+    row_mfma(r0, rs2);
+    r0 = load_row(0);
+    row_mfma(r1, rs2);
+    r1 = load_row(1);
+#pragma unroll
+    for (int b = 0; b < kNs; ++b) rs2[b] = rn[b];
   }
 
-  // ---- salient columns, kMfSalWin at a time: both operands in registers (mf_salient_operands), one MFMA.
-  // The first window uses the words loaded with the tile (no copy of them is made, so nothing waits for them
-  // before the window); later windows load their own.
-  if (num_sal > 0) {
-    f16x8 av, bv;
-    mf_salient_operands(ch, tb, xr, static_cast<uint32_t>(i16 * 4), rs_lane, kg, 0, (sbase0 & 31) + 8 * kg, q2w0, av,
-                        bv);
-    acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(av, bv, acc, 0, 0, 0);
-  }
-  for (int w0 = kMfSalWin; w0 < num_sal; w0 += kMfSalWin) {
-    const int q2b = (sbase0 + w0) >> 5;  // qweight2_sparse row of the window's first salient column
-    uint32_t q2w[2];
+  // ---- salient columns, kMfSalWin at a time: both operands in registers (mf_salient_operands).
+  // The first window uses the words loaded with the tile; later windows load their own.
+  const int sbase0 = cm.sbase0;
+  const int num_sal = cm.num_sal;
+  auto window = [&](int w0, const uint32_t (&q2w)[kNs][2]) {
+    f16x8 av[kRt], bv[kNs];
+    mf_salient_operands<kNs, kRt, kStride>(ch, wb, xr, static_cast<uint32_t>(i16 * 16), rs_lane, kg, w0,
+                                  ((sbase0 + w0) & 31) + 8 * kg, q2w, av, bv);
 #pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      const bool rv = q2b + h < q2rows;
-      q2w[h] = bload32(r_q2, rv ? v_q2 : q2_bytes, static_cast<uint32_t>(rv ? q2b + h : 0) * N * 4u);
+    for (int b = 0; b < kNs; ++b) {
+#pragma unroll
+      for (int m = 0; m < kRt; ++m) acc[b][m] = __builtin_amdgcn_mfma_f32_16x16x32_f16(av[m], bv[b], acc[b][m], 0, 0, 0);
     }
-    f16x8 av, bv;
-    mf_salient_operands(ch, tb, xr, static_cast<uint32_t>(i16 * 4), rs_lane, kg, w0,
-                        ((sbase0 + w0) & 31) + 8 * kg, q2w, av, bv);
-    acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(av, bv, acc, 0, 0, 0);
+  };
+  if (num_sal > 0) {
+    const __amdgpu_buffer_rsrc_t r_q2 = make_rsrc(q2, static_cast<uint32_t>(q2rows) * N * 4u);
+    uint32_t q2w[kNs][2];
+#pragma unroll
+    for (int b = 0; b < kNs; ++b) {
+      q2w[b][0] = q2w0[b][0];
+      q2w[b][1] = q2w0[b][1];
+    }
+#pragma unroll 1
+    for (int w0 = 0;;) {
+      window(w0, q2w);
+      w0 += kMfSalWin;
+      if (w0 >= num_sal) break;
+      const int q2b = (sbase0 + w0) >> 5;  // qweight2_sparse row of the window's first salient column
+#pragma unroll
+      for (int b = 0; b < kNs; ++b) {
+        const uint32_t v_q2 = n[b] < N ? static_cast<uint32_t>(n[b]) * 4u : kMfOob;
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+          const bool rv = q2b + h < q2rows;
+          q2w[b][h] = bload32(r_q2, rv ? v_q2 : kMfOob, static_cast<uint32_t>(rv ? q2b + h : 0) * N * 4u);
+        }
+      }
+    }
   }
-  return acc;
 }
 
 // Workgroup = kUnits units of 4 wavefronts.  The grid is sized to what the GPU holds at once, and the
@@ -912,27 +1005,47 @@ __device__ __forceinline__ f32x4 mf_compute(const MfmaProj& pa, int e, int kc, i
 // kUnits == 1: one projection (blockIdx.z picks it when two are given, unfused).
 // kUnits == 2: unit 0 computes the gate and unit 1 the up projection of the same tiles, side by side;
 // the output is fp16(silu(g) * u).
-// Along a run the units compute from one weight buffer while the next tile's weight words are copied into
-// the other.  With more than one 512-column chunk (rank > 512) the chunk data is restaged per tile and
+// Along a run the units compute two output tiles at a time (mf_compute) while the next two tiles' weight words are
+// in flight to registers.  With more than one 512-column chunk (rank > 512) the chunk data is restaged per tile and
 // nothing is prefetched.
 // Registers are capped at what the LDS lets reside anyway: one unit with 4 staged rows fits four workgroups per CU
 // (128 VGPRs), with 16 rows three.
-// Every LDS array is a static object of its own (kRows activation rows staged: 4 when the batch has at most 4
-// rows, else 16).  The compiler then tells the arrays apart from the copy buffers, and an LDS read waits only
-// for copies into the buffer it reads; a read from dynamic LDS would wait for every copy in flight, the
-// prefetch included.
-template <int kUnits, int kRows, bool kCompact>
+// a / b for 0 <= a < 2^22 and b > 0 (wave-uniform): a reciprocal estimate corrected by one (the general 32-bit division
+// is some 20 dependent instructions, and every wavefront does three of these before its first load).
+__device__ __forceinline__ int mf_div(int a, int b) {
+  int q = static_cast<int>(static_cast<float>(a) * __builtin_amdgcn_rcpf(static_cast<float>(b)));
+  const int r = a - q * b;
+  q += r >= b ? 1 : 0;
+  q -= r < 0 ? 1 : 0;
+  return __builtin_amdgcn_readfirstlane(q);
+}
+
+template <int kUnits, int kRows, bool kCompact, bool kGeneral>
 __global__ __launch_bounds__(kUnits * kMfThreads)
-__attribute__((amdgpu_waves_per_eu(kUnits == 2 ? 2 : (kRows == kMfRows && !kCompact ? 3 : 4), 8)))
+__attribute__((amdgpu_waves_per_eu(kUnits == 2 ? 2 : 3, 8)))
 void grouped_mfma_kernel(MfmaArgs a) {
   using WW = MfWaveWords<kCompact>;
   constexpr int kSal = mf_sal_slots(kCompact);
+  constexpr int kRuns = kRows / 4;
   const int unit = kUnits == 2 ? __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) / kMfThreads) : 0;
-  const int utid = static_cast<int>(threadIdx.x) % kMfThreads;
-  const MfmaProj& pa = a.proj[kUnits == 2 ? unit : blockIdx.z];
+  const int which = kUnits == 2 ? unit : static_cast<int>(blockIdx.z);
+  const MfmaProj& pa = a.proj[which];
   const tris_compact3_payload& p = pa.p;
-  const int N = p.outfeatures;
-  const int nob = ceil_div(N, kTileOut);
+  // the launch's scalars and pointers, all asked for at once (left alone, the compiler loads each where it is first
+  // used, and the workgroup waits for one scalar load after another before its first weight load)
+  const int num_experts = p.num_experts;
+  const int64_t* const row_index = pa.row_index;
+  asm volatile("" ::"s"(p.outfeatures), "s"(num_experts), "s"(p.rank), "s"(p.num_groups), "s"(row_index), "s"(pa.hidden), "s"(pa.out),
+               "s"(pa.decoded), "s"(p.qweight1), "s"(p.qweight2_sparse), "s"(p.qweight2_sparse_prefix), "s"(p.c_map),
+               "s"(p.g_idx), "s"(p.col_pack3), "s"(p.row_pack3), "s"(pa.hidden_rows), "s"(p.qweight2_sparse_rows),
+               "s"(a.segment_offsets), "s"(a.expert_ids), "s"(a.num_segments), "s"(a.batch), "s"(a.decoded_by_expert),
+               "s"(a.comb_out));
+  const int nob = ceil_div(p.outfeatures, kTileOut);
+  // with at most 64 routed rows, every row's index in the segments' round trip (lane i: row i)
+  const int lane = static_cast<int>(threadIdx.x) % kWave;
+  // (without one, any readable words)
+  const int64_t* const any_index = row_index != nullptr ? row_index : reinterpret_cast<const int64_t*>(p.col_pack3);
+  const int64_t early = any_index[row_index != nullptr ? (lane < a.batch ? lane : a.batch - 1) : 0];
   const MfSegScan sc = mf_scan_segments(a.segment_offsets, a.expert_ids, a.num_segments, kMfRows);
   const int R = __builtin_amdgcn_readfirstlane(sc.total);
   if (R == 0) return;  // no rows
@@ -942,32 +1055,20 @@ void grouped_mfma_kernel(MfmaArgs a) {
   const int Rm = comb ? 1 : R;
   const int W = static_cast<int>(gridDim.x);
   const int w = static_cast<int>(blockIdx.x);
+  // workgroup w is the (w / Rm)-th of row tile w % Rm (its activations and column data stay with few XCDs); that tile's
+  // workgroups split its output tiles into runs, and those past its output tiles, the last of the grid, are idle.  With
+  // more row tiles than workgroups, each takes row tiles w, w + W, ... whole.
   int rt_first = w, rt_step = W, ob_lo = 0, ob_hi = nob;
-  if (static_cast<int64_t>(Rm) * nob <= W) {
-    // at least one workgroup per (row tile, output tile): workgroup w takes pair w, and the idle ones are the
-    // last of the grid, so the busy ones are spread evenly over the CUs as the hardware deals them out
-    if (w >= Rm * nob) return;
-    rt_first = w / nob;
-    ob_lo = w - rt_first * nob;
-    ob_hi = ob_lo + 1;
-    rt_step = Rm;  // one row tile
-  } else if (Rm <= W) {
-    const int per = W / Rm;
-    const int extra = W % Rm;
-    int sub, cnt;
-    if (w < extra * (per + 1)) {
-      rt_first = w / (per + 1);
-      sub = w % (per + 1);
-      cnt = per + 1;
-    } else {
-      rt_first = extra + (w - extra * (per + 1)) / per;
-      sub = (w - extra * (per + 1)) % per;
-      cnt = per;
-    }
+  if (Rm <= W) {
+    const int per = mf_div(W, Rm);
+    const int sub = mf_div(w, Rm);
+    rt_first = w - sub * Rm;
+    int cnt = per + (rt_first < W - per * Rm ? 1 : 0);
     cnt = cnt < nob ? cnt : nob;
-    if (sub >= cnt) return;  // more workgroups than output tiles for this row tile
-    ob_lo = static_cast<int>(static_cast<int64_t>(sub) * nob / cnt);
-    ob_hi = static_cast<int>(static_cast<int64_t>(sub + 1) * nob / cnt);
+    if (sub >= cnt) return;
+    const int run = mf_div(nob, cnt), more = nob - run * cnt;  // the first `more` runs have one output tile more
+    ob_lo = sub * run + (sub < more ? sub : more);
+    ob_hi = ob_lo + run + (sub < more ? 1 : 0);
     rt_step = Rm;  // one row tile
   }
   // the combine's weights by row (w_row[inverse_perm[s]] = w[s]); a route that is not one token on two experts,
@@ -980,61 +1081,57 @@ void grouped_mfma_kernel(MfmaArgs a) {
       int cs = 0, cr0 = 0, crc = 0, ce = -1;
       mf_map_scanned(sc, a.segment_offsets, a.expert_ids, a.num_segments, t, kMfRows, &cs, &cr0, &crc, &ce);
       ce = __builtin_amdgcn_readfirstlane(ce);
-      ok = __builtin_amdgcn_readfirstlane(crc) == 1 && ce >= 0 && ce < p.num_experts;
+      ok = __builtin_amdgcn_readfirstlane(crc) == 1 && ce >= 0 && ce < num_experts;
     }
     if (!ok) {
       if (unit == 0) {
-        for (int n = ob_lo * kTileOut + utid; n < ob_hi * kTileOut && n < N; n += kMfThreads) a.comb_out[n] = 0;
+        const int t0 = static_cast<int>(threadIdx.x) % kMfThreads;
+        for (int n = ob_lo * kTileOut + t0; n < ob_hi * kTileOut && n < p.outfeatures; n += kMfThreads) a.comb_out[n] = 0;
       }
       return;
     }
     wr0 = a.comb_w[inv0 == 0 ? 0 : 1];
     wr1 = a.comb_w[inv0 == 0 ? 1 : 0];
   }
-  const int lane = utid % kWave;
   uint16_t* out = kUnits == 2 ? a.proj[0].out : pa.out;
   __shared__ __attribute__((aligned(16))) uint16_t mf_xs[kUnits][kRows * kMfXStride];
-  __shared__ __attribute__((aligned(16))) uint16_t mf_cds[kUnits][kMfChunk];
-  __shared__ __attribute__((aligned(16))) uint16_t mf_cns[kUnits][kMfChunk];
-  __shared__ __attribute__((aligned(16))) uint32_t mf_salw[kUnits][kSal];
-  __shared__ __attribute__((aligned(16))) uint16_t mf_salxo[kUnits][kSal];
-  __shared__ __attribute__((aligned(16))) uint32_t mf_salcp[kUnits][kSal];
-  __shared__ __attribute__((aligned(16))) int32_t mf_meta[kUnits][16];
-  __shared__ __attribute__((aligned(16))) float mf_exch[kUnits == 2 ? kMfThreads * 4 : 4];
+  __shared__ __attribute__((aligned(16))) uint16_t mf_cds[kUnits][2 * kMfChunk];  // C_d, then C_nd
+  __shared__ __attribute__((aligned(16))) uint2 mf_goff[kUnits][kMfTiles];
+  __shared__ __attribute__((aligned(16))) uint32_t mf_salw[kUnits][kSal + 4];  // (one spare slot)
+  __shared__ __attribute__((aligned(16))) uint16_t mf_salxo[kUnits][kSal + 8];
+  __shared__ __attribute__((aligned(16))) uint32_t mf_salcp[kUnits][kSal + 4];
+  __shared__ __attribute__((aligned(16))) float mf_exch[kUnits == 2 ? kMfThreads * 4 * 2 : 4];
   MfChunk ch;
   ch.xs = &mf_xs[unit][0];
   ch.cds = &mf_cds[unit][0];
-  ch.cns = &mf_cns[unit][0];
+  ch.cns = &mf_cds[unit][kMfChunk];
+  ch.goff = &mf_goff[unit][0];
   ch.col_sal = nullptr;
   ch.sal_col = nullptr;
   ch.sal_xi = nullptr;
   ch.sal_w = &mf_salw[unit][0];
   ch.sal_xo = &mf_salxo[unit][0];
   ch.sal_cp = &mf_salcp[unit][0];
-  ch.meta = &mf_meta[unit][0];
-  // each wavefront's two copy buffers (two objects, so reads of one do not wait for copies into the other)
-  __shared__ __attribute__((aligned(16))) uint32_t mf_wb0[kUnits * kMfWaves][WW::kAlloc];
-  __shared__ __attribute__((aligned(16))) uint32_t mf_wb1[kUnits * kMfWaves][WW::kAlloc];
-  const int wave = __builtin_amdgcn_readfirstlane(utid / kWave);
-  const int wslot = unit * kMfWaves + wave;
-  const MfWaveBuf tb0{&mf_wb0[wslot][kMfWq1], &mf_wb0[wslot][kMfWgw], &mf_wb0[wslot][kMfWrs],
-                      &mf_wb0[wslot][WW::kWords]};
-  const MfWaveBuf tb1{&mf_wb1[wslot][kMfWq1], &mf_wb1[wslot][kMfWgw], &mf_wb1[wslot][kMfWrs],
-                      &mf_wb1[wslot][WW::kWords]};
-  if (lane == 0) {  // the zero words (the first row tile's barrier orders these writes before any read)
-    *tb0.zero = 0u;
-    *tb1.zero = 0u;
-  }
+  ch.meta = nullptr;
+  // each wavefront's words of the two tiles it computes together
+  __shared__ __attribute__((aligned(16))) uint32_t mf_wb[kUnits * kMfWaves][2][WW::kAlloc];
+  const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) % kMfThreads / kWave);
+  uint32_t* const wb = &mf_wb[unit * kMfWaves + wave][0][0];
+  if (lane < 2) wb[lane * WW::kAlloc] = 0u;  // the zero words (the first row tile's barrier orders these writes)
   float* exch = mf_exch;
-  const int i16 = lane % 16;
-  const int rank = p.rank;
-  const bool one_chunk = rank <= kMfChunk;
-  const int kg = lane / 16;
 
   for (int rt_i = rt_first; rt_i < Rm; rt_i += rt_step) {
+  // the lane index and sizes of this row tile: opaque, so that the many addresses and conditions made of them are not
+  // computed ahead of the loop and held across it (most launches run it once, and the held registers spill)
+  int ln = lane, N = p.outfeatures, rank = p.rank, G = p.num_groups, nseg = a.num_segments;
+  int ob_begin = ob_lo, ob_end = ob_hi;
+  asm volatile("" : "+v"(ln), "+s"(N), "+s"(rank), "+s"(G), "+s"(nseg), "+s"(ob_begin), "+s"(ob_end));
+  const int utid = wave * kWave + ln;
+  const int i16 = ln % 16;
+  const int kg = ln / 16;
   const int rt = comb ? unit : rt_i;  // the combine's units: row tiles 0 and 1
   int s = 0, row0 = 0, rc = 0, e = -1;
-  mf_map_scanned(sc, a.segment_offsets, a.expert_ids, a.num_segments, rt, kMfRows, &s, &row0, &rc, &e);
+  mf_map_scanned(sc, a.segment_offsets, a.expert_ids, nseg, rt, kMfRows, &s, &row0, &rc, &e);
   s = __builtin_amdgcn_readfirstlane(s);  // the mapping is the same in every lane
   row0 = __builtin_amdgcn_readfirstlane(row0);
   rc = __builtin_amdgcn_readfirstlane(rc);
@@ -1043,9 +1140,7 @@ void grouped_mfma_kernel(MfmaArgs a) {
   // activations from partial sums: only the 4-row instances carry that staging (the host sends at most 4 rows),
   // so the others keep no register for it across their tile loop
   const bool part = kRows == 4 && pa.partials != nullptr;
-  const int ob_begin = ob_lo;
-  const int ob_end = ob_hi;
-  if (e < 0 || e >= p.num_experts) {  // rows routed to no expert: zero output
+  if (e < 0 || e >= num_experts) {  // rows routed to no expert: zero output
     if (unit == 0) {
       const int span = (ob_end - ob_begin) * kTileOut;
       for (int idx = utid; idx < rc * span; idx += kMfThreads) {
@@ -1058,130 +1153,152 @@ void grouped_mfma_kernel(MfmaArgs a) {
   if (rt_i != rt_first) __syncthreads();  // the previous row tile's LDS readers are done
   // A operand row of this lane: rows past rc feed output rows that are not stored, so they read row 0 (the same
   // LDS words as lane 0's rows: broadcast reads instead of bank conflicts; T = 16 gate/up launch 33.2 -> 32.5 us)
-  const int xrow = i16 < rc ? i16 : 0;
-  const MfWaveOffsets wo = mf_wave_offsets(pa, 0, wave, lane);
-  {  // chunk 0 and the first tile's weights
-    MfRegs regs;
-    mf_wave_tile_issue<kCompact>(pa, ds, e, ob_begin, wo, lane, wave, tb0);
-    mf_chunk_issue(pa, e, row0, rc, 0, utid, regs, part);
-    mf_chunk_write(pa, rc, 0, utid, ch, regs, false, kSal, part);
+  const uint16_t* const xr[1] = {ch.xs + (i16 < rc ? i16 : 0) * kMfXStride};
+  const MfWaveSrc src = mf_wave_src(pa, ds, e, 0, wave, ln);
+  const uint32_t* q2 = reinterpret_cast<const uint32_t*>(p.qweight2_sparse) +
+                       static_cast<int64_t>(e) * p.qweight2_sparse_rows * N;
+  const int q2rows = p.qweight2_sparse_rows;
+  MfWaveRegs<kCompact> wr[2];  // the next two tiles' words in flight
+  int64_t entry = early;
+  int tok0 = row0;
+  if (row_index == nullptr) {
+    entry = ln;
+    tok0 = 0;
+  } else if (a.batch > kWave) {  // more rows than lanes: this row tile's own
+    entry = row_index[row0 + (ln < rc ? ln : rc - 1)];
+    tok0 = 0;
+  }
+  const int hidden_rows = row_index != nullptr ? pa.hidden_rows : rc;
+  const uint32_t roff = entry >= 0 && entry < hidden_rows && ln - tok0 < rc
+                            ? static_cast<uint32_t>(entry) * static_cast<uint32_t>(rank) * 2u : kMfOob;
+  const __amdgpu_buffer_rsrc_t r_hid =
+      make_rsrc(pa.hidden + (row_index != nullptr ? 0 : static_cast<int64_t>(row0) * rank),
+                part ? 0u : static_cast<uint32_t>(hidden_rows) * rank * 2u);
+  MfChunkMeta cm;
+  {  // chunk 0 and the first tiles' weights
+    MfColRegs cols;
+    MfRowRegs<kRuns> rows;
+    mf_cols_issue(pa, e, 0, utid, cols);
+    mf_rows_issue<kRuns>(r_hid, rank, 0, wave, ln, roff, tok0, rows);
+    mf_wave_tile_issue<kCompact, kGeneral>(src, G, ob_begin, ln, wr[0]);
+    mf_wave_tile_issue<kCompact, kGeneral>(src, G, ob_begin + 1, ln, wr[1], !kGeneral && ob_begin + 1 < ob_end);
+    mf_cols_write(pa, rc, 0, utid, ch, cols, kSal);
+    if (!part) mf_rows_write<kRuns>(rows, rc, wave, ln, ch.xs);
     if (part) mf_partials_stage(pa, row0, rc, utid, ch);  // one chunk (host-checked)
-    __builtin_amdgcn_s_waitcnt(0);  // LDS copies landed (all counters zero)
+    cm = mf_chunk_meta(cols, kSal);
+    mf_wave_tile_write<kCompact>(wr[0], ln, wb);
+    mf_wave_tile_write<kCompact>(wr[1], ln, wb + WW::kAlloc);
     __syncthreads();
   }
-  // One output tile, computed from `cur`; with one chunk each wavefront copies its columns of the next tile
-  // into `nxt` meanwhile.  Called with the two buffers in alternation, so every instance knows which object it
-  // reads and which it fills.  With one chunk and one unit the wavefronts do not wait for each other, and a
-  // tile's four output stores are issued by the next tile (or after the last), once that tile has issued its
-  // own loads and copies: nothing then waits for a store that has just been issued.  Each tile issues, after
-  // the copies of `cur` (the previous tile's prefetch), at least its two qweight2_sparse loads, its prefetch
-  // and the previous tile's stores, so waiting until no more than those are outstanding leaves `cur`'s copies
-  // landed (vector memory operations complete in issue order).  The first tile of a row tile finds its copies
-  // landed already.
-  constexpr int kAfterCopies = 2 + WW::kDma + (kUnits == 1 ? 4 : 0);
-  // the staged chunk's metadata, its salient count held to the slots staged (a payload whose prefix counts
-  // disagree with its salient map reads no slot past them)
-  const auto chunk_meta = [&]() {
-    MfChunkMeta m = mf_chunk_meta(ch);
-    m.num_sal = m.num_sal < 0 ? 0 : (m.num_sal < kSal ? m.num_sal : kSal);
-    return m;
-  };
-  // one unit: the last tile's outputs (fp16 pairs of rows 4 kg .. 4 kg + 3) and the tile they belong to
-  uint32_t held01 = 0u, held23 = 0u;
-  int held_ob = -1;
-  const uint32_t out_bytes = static_cast<uint32_t>(rc) * N * 2u;
-  const __amdgpu_buffer_rsrc_t r_out = make_rsrc(out + static_cast<int64_t>(row0) * N, out_bytes);
-  auto store_held = [&]() {
-    const int hn = held_ob * kTileOut + 16 * wave + i16;
-    const uint32_t hv[4] = {held01 & 0xFFFFu, held01 >> 16, held23 & 0xFFFFu, held23 >> 16};
+  // The outputs of tile ob, from its accumulators.  Stores go through a buffer resource over the tile's rows from its
+  // first column: rows past rc have an offset past it and are dropped, so every lane issues all four; only the
+  // expert's last tile can have columns past N.
+  uint16_t* const out0 = out + static_cast<int64_t>(row0) * N;
+  uint32_t orow[4];
+#pragma unroll
+  for (int v = 0; v < 4; ++v) {
+    orow[v] = 4 * kg + v < rc ? static_cast<uint32_t>((4 * kg + v) * N + 16 * wave + i16) * 2u : kMfOob;
+  }
+  auto store = [&](int ob, const f32x4& acc, const float* ex) {
+    const int n = ob * kTileOut + 16 * wave + i16;
+    if (kUnits == 2 && comb) {
+      // row 0 of each unit's tile (one row a tile): the combine of the token's two rows at column n, the products
+      // rounded to fp16 (the asm keeps them from being fused into the sum) and added in fp32 (two terms: the
+      // pick order does not matter), rounded once to the output dtype
+      if (kg == 0 && n < N) {
+        const float up0 = ex[utid * 4];
+        uint16_t p0 = hmul_bits(f2h_bits(acc[0]), wr0);
+        uint16_t p1 = hmul_bits(f2h_bits(up0), wr1);
+        asm volatile("" : "+v"(p0), "+v"(p1));
+        const float y = h2f(p0) + h2f(p1);
+        a.comb_out[n] = a.comb_bf16 ? f32_to_bf16_rne(y) : f2h_bits(y);
+      }
+      return;
+    }
+    f32x4 up = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    if (kUnits == 2) up = *reinterpret_cast<const f32x4*>(&ex[utid * 4]);
+    const __amdgpu_buffer_rsrc_t r_out = make_rsrc(out0 + ob * kTileOut, static_cast<uint32_t>(rc * N - ob * kTileOut) * 2u);
+    const bool edge = (ob + 1) * kTileOut > N;  // uniform
 #pragma unroll
     for (int v = 0; v < 4; ++v) {
-      const int r = 4 * kg + v;
-      __builtin_amdgcn_raw_buffer_store_b16(static_cast<uint16_t>(hv[v]), r_out,
-                                            hn < N && r < rc ? static_cast<uint32_t>(r * N + hn) * 2u : out_bytes,
-                                            0u, 0);
+      // two units: g and u rounded to fp16 as the two outputs would be.  One unit: no output scale or bias here, the
+      // host sends none (launch_grouped_mfma rejects payloads with them)
+      const uint16_t y = kUnits == 2 ? swiglu_bits(f2h_bits(acc[v]), f2h_bits(up[v])) : f2h_bits(acc[v]);
+      uint32_t vo = orow[v];
+      if (edge) vo = n < N ? vo : kMfOob;
+      __builtin_amdgcn_raw_buffer_store_b16(y, r_out, vo, 0u, 0);
     }
   };
-  auto tile = [&](int ob, const MfWaveBuf& cur, const MfWaveBuf& nxt) {
-    const int n = ob * kTileOut + 16 * wave + i16;
-    f32x4 acc = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-    // (the two cases keep separate qweight2_sparse words: a variable shared by both would be copied at their join,
-    // and the copy waits for the loads)
-    if (one_chunk) {
-      const MfChunkMeta cm = chunk_meta();
-      uint32_t q2w[2];
-      mf_q2_issue(pa, e, n, cm, q2w);
-      mf_wave_tile_issue<kCompact>(pa, ds, e, ob + 1, wo, lane, wave, nxt, ob + 1 < ob_end);  // prefetch
-      if (kUnits == 1 && held_ob >= 0) store_held();  // the previous tile's outputs (wave-uniform condition)
-      wait_vmcnt<kAfterCopies>();  // this wavefront's copies into `cur` landed
-      acc = mf_compute(pa, e, 0, ob * kTileOut, xrow, utid, ch, cm, cur, q2w, acc);
+  // kNs output tiles from `ob`, whose words are in wb; with one chunk the next tiles' words are loaded to registers
+  // meanwhile and written to wb after the last read of this pass (one wavefront's LDS operations stay in order).
+  auto tiles = [&](auto ns, int ob) {
+    constexpr int kNs = decltype(ns)::value;
+    f32x4 acc[kNs][1];
+    int n[kNs];
+    uint32_t q2w[kNs][2];
+#pragma unroll
+    for (int b = 0; b < kNs; ++b) {
+      acc[b][0] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+      n[b] = (ob + b) * kTileOut + 16 * wave + i16;
+    }
+    if constexpr (!kGeneral) {
+#pragma unroll
+      for (int b = 0; b < kNs; ++b) mf_q2_issue(q2, q2rows, N, n[b], cm, q2w[b]);
+#pragma unroll
+      for (int b = 0; b < 2; ++b) {
+        mf_wave_tile_issue<kCompact, kGeneral>(src, G, ob + kNs + b, ln, wr[b], ob + kNs + b < ob_end);
+      }
+      __builtin_amdgcn_sched_barrier(0);  // the loads stay ahead of the pass they overlap
+      mf_compute<kNs, 1, WW::kAlloc>(q2, q2rows, N, rank, G, 0, n, xr, ln, ch, cm, wb, q2w, acc);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int b = 0; b < 2; ++b) mf_wave_tile_write<kCompact>(wr[b], ln, wb + b * WW::kAlloc);
     } else {
       for (int kc = 0; kc < rank; kc += kMfChunk) {
         if (ob > ob_begin || kc > 0) {
           __syncthreads();  // the previous chunk's readers are done
-          MfRegs regs;
-          mf_wave_tile_issue<kCompact>(pa, ds, e, ob, mf_wave_offsets(pa, kc, wave, lane), lane, wave, cur);
-          mf_chunk_issue(pa, e, row0, rc, kc, utid, regs);
-          mf_chunk_write(pa, rc, kc, utid, ch, regs, false, kSal);
-          __builtin_amdgcn_s_waitcnt(0);
+          MfColRegs cols;
+          MfRowRegs<kRuns> rows;
+          mf_wave_tile_issue<kCompact, kGeneral>(mf_wave_src(pa, ds, e, kc, wave, ln), G, ob, ln, wr[0]);
+          mf_cols_issue(pa, e, kc, utid, cols);
+          mf_rows_issue<kRuns>(r_hid, rank, kc, wave, ln, roff, tok0, rows);
+          mf_cols_write(pa, rc, kc, utid, ch, cols, kSal);
+          mf_rows_write<kRuns>(rows, rc, wave, ln, ch.xs);
+          cm = mf_chunk_meta(cols, kSal);
+          mf_wave_tile_write<kCompact>(wr[0], ln, wb);
           __syncthreads();
         }
-        const MfChunkMeta cm = chunk_meta();
-        uint32_t q2w[2];
-        mf_q2_issue(pa, e, n, cm, q2w);
-        acc = mf_compute(pa, e, kc, ob * kTileOut, xrow, utid, ch, cm, cur, q2w, acc);
+        mf_q2_issue(q2, q2rows, N, n[0], cm, q2w[0]);
+        mf_compute<kNs, 1, WW::kAlloc>(q2, q2rows, N, rank, G, kc, n, xr, ln, ch, cm, wb, q2w, acc);
       }
     }
-
-    // stores through a buffer resource over the tile's rows: rows past rc and columns past N go past its end and
-    // are dropped, so every lane issues all four
-    const bool nv = n < N;
     if (kUnits == 2) {
-      if (unit == 1) *reinterpret_cast<f32x4*>(&exch[utid * 4]) = acc;
+      if (unit == 1) {
+#pragma unroll
+        for (int b = 0; b < kNs; ++b) *reinterpret_cast<f32x4*>(&exch[(b * kMfThreads + utid) * 4]) = acc[b][0];
+      }
       __syncthreads();
-      if (unit == 0 && comb) {
-        // row 0 of each unit's tile (one row a tile): the combine of the token's two rows at column n, the products
-        // rounded to fp16 (the asm keeps them from being fused into the sum) and added in fp32 (two terms: the
-        // pick order does not matter), rounded once to the output dtype
-        if (kg == 0 && nv) {
-          const float up0 = exch[utid * 4];
-          uint16_t p0 = hmul_bits(f2h_bits(acc[0]), wr0);
-          uint16_t p1 = hmul_bits(f2h_bits(up0), wr1);
-          asm volatile("" : "+v"(p0), "+v"(p1));
-          const float y = h2f(p0) + h2f(p1);
-          a.comb_out[n] = a.comb_bf16 ? f32_to_bf16_rne(y) : f2h_bits(y);
-        }
-      } else if (unit == 0) {
-        const f32x4 up = *reinterpret_cast<const f32x4*>(&exch[utid * 4]);
+      if (unit == 0) {
 #pragma unroll
-        for (int v = 0; v < 4; ++v) {
-          const int r = 4 * kg + v;
-          // g and u rounded to fp16 as the two outputs would be
-          __builtin_amdgcn_raw_buffer_store_b16(swiglu_bits(f2h_bits(acc[v]), f2h_bits(up[v])), r_out,
-                                                nv && r < rc ? static_cast<uint32_t>(r * N + n) * 2u : out_bytes,
-                                                0u, 0);
-        }
+        for (int b = 0; b < kNs; ++b) store(ob + b, acc[b][0], exch + b * kMfThreads * 4);
       }
-      __syncthreads();  // exch is rewritten by the next tile
+      __syncthreads();  // exch is rewritten by the next tiles
     } else {
-      // no output scale or bias here: the host sends none (launch_grouped_mfma rejects payloads with them)
-      uint32_t hv[4];
 #pragma unroll
-      for (int v = 0; v < 4; ++v) hv[v] = f2h_bits(acc[v]);
-      held01 = hv[0] | (hv[1] << 16);
-      held23 = hv[2] | (hv[3] << 16);
-      held_ob = ob;
-      if (!one_chunk) {
-        store_held();
-        held_ob = -1;
-      }
+      for (int b = 0; b < kNs; ++b) store(ob + b, acc[b][0], exch);
     }
   };
-  for (int ob = ob_begin; ob < ob_end; ob += 2) {
-    tile(ob, tb0, tb1);
-    if (ob + 1 < ob_end) tile(ob + 1, tb1, tb0);
+  for (int ob = ob_begin; ob < ob_end;) {
+    if constexpr (!kGeneral) {
+      if (ob + 1 < ob_end) {
+        tiles(std::integral_constant<int, 2>{}, ob);
+        ob += 2;
+        continue;
+      }
+    }
+    tiles(std::integral_constant<int, 1>{}, ob);
+    ob += 1;
   }
-  if (kUnits == 1 && held_ob >= 0) store_held();  // the row tile's last outputs
   }  // row tiles
 }
 
@@ -1366,6 +1483,7 @@ __global__ __launch_bounds__(kUnits * kMfThreads) __attribute__((amdgpu_waves_pe
   ch.sal_cp = reinterpret_cast<uint32_t*>(lbase + L.sal_cp);
   ch.sal_w = nullptr;
   ch.sal_xo = nullptr;
+  ch.goff = nullptr;
   ch.meta = reinterpret_cast<int32_t*>(lbase + L.meta);
   uint16_t* const xsb0 = reinterpret_cast<uint16_t*>(lbase + L.xs[0]);
   uint16_t* const xsb1 = reinterpret_cast<uint16_t*>(lbase + L.xs[1]);
@@ -1421,8 +1539,8 @@ __global__ __launch_bounds__(kUnits * kMfThreads) __attribute__((amdgpu_waves_pe
       }
       if (it == it0) {  // the segment's column data
         MfRegs regs;
-        mf_chunk_issue(pa, e, seg_lo, 0, 0, utid, regs);  // rc = 0: no activation rows
-        mf_chunk_write(pa, 0, 0, utid, ch, regs, true);  // natural column order
+        mf_chunk_issue(pa, e, 0, utid, regs);
+        mf_chunk_write(pa, 0, utid, ch, regs);
       }
       __builtin_amdgcn_s_waitcnt(0);
       __syncthreads();
@@ -1697,6 +1815,13 @@ static bool ws_fits(const tris_compact3_payload* p) {
   return p->rank <= kMfChunk && p->qweight2_sparse_rows <= kWsSalWindows && !p->has_output_scale && !p->has_bias;
 }
 
+// The decode kernel may load a projection's weight words 16 bytes at a time: 16-byte aligned tensors and a column
+// count that is a multiple of 4, so that no load straddles a row's or the tensor's end.
+static bool mf_wide(const MfmaProj& p) {
+  const auto al = [](const void* q) { return reinterpret_cast<uintptr_t>(q) % 16 == 0; };
+  return p.p.outfeatures % 4 == 0 && al(p.p.qweight1) && al(p.p.row_pack3) && al(p.decoded);
+}
+
 int launch_grouped_mfma(const uint16_t* hidden_a, const uint16_t* hidden_b, int batch, const int32_t* expert_ids,
                         const int32_t* segment_offsets, int num_segments, const int32_t* decoded_a,
                         const int32_t* decoded_b, const tris_compact3_payload* pa, const tris_compact3_payload* pb,
@@ -1754,6 +1879,7 @@ int launch_grouped_mfma(const uint16_t* hidden_a, const uint16_t* hidden_b, int 
   args.expert_ids = expert_ids;
   args.segment_offsets = segment_offsets;
   args.num_segments = num_segments;
+  args.batch = batch;
   args.decoded_by_expert = decoded_by_expert ? 1 : 0;
   if (comb_out != nullptr) {  // both units run the one projection, on row tiles 0 and 1
     args.proj[1] = args.proj[0];
@@ -1783,12 +1909,16 @@ int launch_grouped_mfma(const uint16_t* hidden_a, const uint16_t* hidden_b, int 
            p->rank <= kMfChunk / 2;
   };
   const bool compact = compact_ok(pa) && (!pb || compact_ok(pb));
-  const int lds_total = mf_static_lds_bytes(units, rows, compact);
+  // more than one chunk (rank > 512), or columns that 16-byte loads do not fit: the general instance, which computes
+  // a tile at a time and loads nothing ahead
+  const bool general = pa->rank > kMfChunk || !mf_wide(args.proj[0]) ||
+                       (pb && (pb->rank > kMfChunk || !mf_wide(args.proj[1])));
+  const int lds_total = mf_static_lds_bytes(units, general ? kMfRows : rows, compact && !general);
   TRIS_REQUIRE(lds_total <= 160 * 1024, "%s: LDS request %d exceeds a CU", who, lds_total);
   // Workgroups: as many as the GPU holds at once (LDS and the kernel's 128 VGPRs per lane, 4 wavefronts
   // per SIMD for one unit, bound them), shared by the projections of an unfused pair.
   int wgs_per_cu = (160 * 1024) / lds_total;
-  const int by_regs = units == 1 ? 4 : 1;
+  const int by_regs = units == 1 ? 3 : 1;
   wgs_per_cu = wgs_per_cu < by_regs ? wgs_per_cu : by_regs;
   wgs_per_cu = wgs_per_cu > 0 ? wgs_per_cu : 1;
   int wgs = (kMfCus * wgs_per_cu) / nproj;
@@ -1799,19 +1929,19 @@ int launch_grouped_mfma(const uint16_t* hidden_a, const uint16_t* hidden_b, int 
   if (comb_out != nullptr && ceil_div(max_n, kTileOut) < wgs) wgs = ceil_div(max_n, kTileOut);  // output tiles only
   const dim3 grid(wgs > 0 ? wgs : 1, 1, nproj);
   const dim3 block(units * kMfThreads);
-#define TRIS_MF_LAUNCH(U, ROWS, C) hipLaunchKernelGGL((grouped_mfma_kernel<U, ROWS, C>), grid, block, 0, s, args)
+#define TRIS_MF_LAUNCH(U, ROWS, C, M) hipLaunchKernelGGL((grouped_mfma_kernel<U, ROWS, C, M>), grid, block, 0, s, args)
   if (units == 2) {
-    if (rows == 4) {
-      if (compact) TRIS_MF_LAUNCH(2, 4, true); else TRIS_MF_LAUNCH(2, 4, false);
-    } else {
-      if (compact) TRIS_MF_LAUNCH(2, kMfRows, true); else TRIS_MF_LAUNCH(2, kMfRows, false);
-    }
+    if (general) TRIS_MF_LAUNCH(2, kMfRows, false, true);
+    else if (rows == 4 && compact) TRIS_MF_LAUNCH(2, 4, true, false);
+    else if (rows == 4) TRIS_MF_LAUNCH(2, 4, false, false);
+    else if (compact) TRIS_MF_LAUNCH(2, kMfRows, true, false);
+    else TRIS_MF_LAUNCH(2, kMfRows, false, false);
   } else {
-    if (rows == 4) {
-      if (compact) TRIS_MF_LAUNCH(1, 4, true); else TRIS_MF_LAUNCH(1, 4, false);
-    } else {
-      if (compact) TRIS_MF_LAUNCH(1, kMfRows, true); else TRIS_MF_LAUNCH(1, kMfRows, false);
-    }
+    if (general) TRIS_MF_LAUNCH(1, kMfRows, false, true);
+    else if (rows == 4 && compact) TRIS_MF_LAUNCH(1, 4, true, false);
+    else if (rows == 4) TRIS_MF_LAUNCH(1, 4, false, false);
+    else if (compact) TRIS_MF_LAUNCH(1, kMfRows, true, false);
+    else TRIS_MF_LAUNCH(1, kMfRows, false, false);
   }
 #undef TRIS_MF_LAUNCH
   return check_launch(who);
