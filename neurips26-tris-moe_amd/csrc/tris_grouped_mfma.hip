@@ -52,7 +52,6 @@ constexpr int kMfWaves = 4;
 constexpr int kMfThreads = kMfWaves * kWave;
 constexpr int kMfRows = 16;         // segment rows per workgroup tile
 constexpr int kMfChunk = 512;       // K columns staged per pass
-constexpr int kMfXStride = kMfChunk + 8;  // fp16 elements per staged row (pad breaks bank aliasing)
 constexpr int kMfSalWin = 32;             // salient columns per MFMA pass
 constexpr int kMfSalStride = kMfSalWin + 8;
 
@@ -204,13 +203,16 @@ constexpr int kMfTbRs = kMfTbGw + kMfPR * kTileOut;
 constexpr int kMfTbWords = kMfTbRs + kTileOut * kMfMaxGroups * 2;
 static_assert(kMfTbGw % 4 == 0 && kMfTbRs % 4 == 0, "tile buffer pieces must be 16-byte aligned");
 constexpr int kMfCus = 256;  // MI355X compute units
+constexpr int kMfTallMinRows = 12;  // mean rows a segment from which the decode kernel takes 32- or 64-row tiles
 // Decode kernel: row-scale groups and salient slots per chunk its LDS holds; the compact variant (at most 4
 // groups and 64 salient columns per expert) fits four workgroups per CU.
 constexpr int mf_groups_cap(bool compact) { return compact ? 4 : kMfMaxGroups; }
 constexpr int mf_sal_slots(bool compact) { return compact ? 64 : kMfChunk; }
+constexpr int mf_chunk(bool compact) { return compact ? kMfChunk / 2 : kMfChunk; }  // K columns staged
+constexpr int mf_xstride(bool compact) { return mf_chunk(compact) + 8; }  // fp16 elements per staged row (pad breaks bank aliasing)
 // per wavefront and tile: a zero word, the qweight1 and split words of 16 columns and their row-scale block
 constexpr int mf_wave_alloc_bytes(bool compact) {
-  return (4 + 2 * (kMfChunk / 32) * 16 + 16 * mf_groups_cap(compact) * 2) * 4;
+  return (4 + 2 * (mf_chunk(compact) / 32) * 16 + 16 * mf_groups_cap(compact) * 2) * 4;
 }
 constexpr int kMfRuns = kMfRows * (kMfChunk / 8) / kMfThreads;  // activation runs per thread of a unit
 
@@ -225,13 +227,14 @@ __host__ __device__ inline int mf_take(int* o, int b) {
 
 // Static LDS of the decode kernel with `units` units and `rows` staged activation rows (as declared there).
 constexpr int mf_static_lds_bytes(int units, int rows, bool compact) {
-  return units * (rows * kMfXStride * 2 + kMfChunk * (2 + 2) + mf_sal_slots(compact) * (4 + 2 + 4) + 48 + (kMfChunk / kTileK) * 8 +
+  return units * (rows * mf_xstride(compact) * 2 + mf_chunk(compact) * (2 + 2) + mf_sal_slots(compact) * (4 + 2 + 4) + 48 +
+                  (mf_chunk(compact) / kTileK) * 8 +
                   2 * kMfWaves * mf_wave_alloc_bytes(compact)) +
-         (units == 2 ? 2 * kMfExchBytes : 16);
+         (units == 2 ? 2 * (rows > kMfRows ? rows / kMfRows : 1) * kMfExchBytes : 16);
 }
 
 struct MfChunk {       // a unit's staged chunk
-  uint16_t* xs;        // [rows][kMfXStride] activations, staged column order; column kMfChunk is zero (decode)
+  uint16_t* xs;        // [rows][mf_xstride] activations, staged column order; the column past the chunk is zero (decode)
   uint16_t* cds;       // -C_d, staged column order (0 for salient columns); decode: -C_nd follows
   uint16_t* cns;       // weight-stationary: -C_nd (0 for salient columns)
   // Weight-stationary kernel (natural column order):
@@ -261,14 +264,15 @@ struct MfTileBuf {     // one output tile's weight words
 // qweight1 and split word each; the row-scale block [16 columns][G][R0 | R1, R_d | R_nd].
 constexpr int kMfWCols = 16;
 constexpr int kMfWw = 4;                            // word offset of the weight words (the zero word is word 0)
-constexpr int kMfWrs = kMfWw + 2 * kMfPR * kMfWCols;  // word offset of the row scales
 template <bool kCompact>
 struct MfWaveWords {
+  static constexpr int kPR = mf_chunk(kCompact) / 32;            // packed rows
+  static constexpr int kRs = kMfWw + 2 * kPR * kMfWCols;         // word offset of the row scales
   static constexpr int kRsLane = kMfWCols * mf_groups_cap(kCompact) * 2 / kWave;  // row-scale words a lane loads
-  static constexpr int kAlloc = kMfWrs + kRsLane * kWave;
+  static constexpr int kAlloc = kRs + kRsLane * kWave;
   static_assert(kRsLane * kWave == kMfWCols * mf_groups_cap(kCompact) * 2 && (kRsLane == 2 || kRsLane == 4),
                 "one 8- or 16-byte row-scale load a lane");
-  static_assert(kAlloc * 4 == mf_wave_alloc_bytes(kCompact) && kMfWrs % 4 == 0, "LDS accounting");
+  static_assert(kAlloc * 4 == mf_wave_alloc_bytes(kCompact) && kRs % 4 == 0, "LDS accounting");
 };
 template <bool kCompact>
 struct MfWaveRegs {    // a tile's words in flight: lane l holds columns 4 (l % 4) .. + 3 of packed row l / 4, and
@@ -377,11 +381,12 @@ struct MfColRegs {
   int sbase0;    // salient prefix at the chunk's first packed row (the same in every lane)
   int send;      // salient prefix at the chunk's end (the same in every lane)
 };
+template <bool kCompact>
 __device__ __forceinline__ void mf_cols_issue(const MfmaProj& pa, int e, int kc, int utid, MfColRegs& R) {
   const tris_compact3_payload& p = pa.p;
   const int rank = p.rank;
   const int packed_rows = rank / 32;  // rank % 64 == 0
-  const int end = kc + kMfChunk < rank ? kc + kMfChunk : rank;
+  const int end = kc + mf_chunk(kCompact) < rank ? kc + mf_chunk(kCompact) : rank;
   const __amdgpu_buffer_rsrc_t r_col =
       make_rsrc(p.col_pack3 + static_cast<int64_t>(e) * rank, static_cast<uint32_t>(rank) * 8u);
   const __amdgpu_buffer_rsrc_t r_cm =
@@ -403,8 +408,10 @@ __device__ __forceinline__ void mf_cols_issue(const MfmaProj& pa, int e, int kc,
 // exactly -fp16(C * R), so a set qweight1 bit is the selectors' sign bit) and zero for salient columns, whatever their
 // selector bits; the salient slots; the K tiles' row-scale offsets; the zero columns of the rc staged rows.  sal_cap:
 // the slots staged (a payload whose prefix counts disagree with its salient map writes no slot past them).
+template <bool kCompact>
 __device__ __forceinline__ void mf_cols_write(const MfmaProj& pa, int rc, int kc, int utid, const MfChunk& ch,
                                               const MfColRegs& R, int sal_cap) {
+  constexpr int kChunk = mf_chunk(kCompact);
   const int rank = pa.p.rank;
   const int G = pa.p.num_groups;
   const int j = 2 * utid;
@@ -413,30 +420,32 @@ __device__ __forceinline__ void mf_cols_write(const MfmaProj& pa, int rc, int kc
   const int bit = j & 31;
   const uint32_t sal = kc + j < rank ? (R.cm >> bit) & 3u : 0u;
   const uint32_t cdn[2] = {R.cp.y ^ 0x80008000u, R.cp.w ^ 0x80008000u};  // C_d | C_nd << 16
+  if (j < kChunk) {  // wave-uniform
 #pragma unroll
-  for (int h = 0; h < 2; ++h) {
-    const uint32_t v = (sal >> h) & 1u ? 0u : cdn[h];
-    ch.cds[pos + 8 * h] = static_cast<uint16_t>(v);
-    ch.cds[kMfChunk + pos + 8 * h] = static_cast<uint16_t>(v >> 16);
-  }
-  // (a column that is not salient writes the spare slot sal_cap, so that no load is put off into a branch and waited
-  // for there, with every load issued after it)
-  int q = R.q2t - R.sbase0 + __popc(R.cm & ((1u << bit) - 1u));
+    for (int h = 0; h < 2; ++h) {
+      const uint32_t v = (sal >> h) & 1u ? 0u : cdn[h];
+      ch.cds[pos + 8 * h] = static_cast<uint16_t>(v);
+      ch.cds[kChunk + pos + 8 * h] = static_cast<uint16_t>(v >> 16);
+    }
+    // (a column that is not salient writes the spare slot sal_cap, so that no load is put off into a branch and waited
+    // for there, with every load issued after it)
+    int q = R.q2t - R.sbase0 + __popc(R.cm & ((1u << bit) - 1u));
 #pragma unroll
-  for (int h = 0; h < 2; ++h) {
-    // the column's group as the main pass takes it (uniform 64-column groups); an invalid group gives
-    // zero factors, as a K tile without a group does
-    const bool is = ((sal >> h) & 1u) != 0u;
-    const int at = is && q >= 0 && q < sal_cap ? q : sal_cap;
-    ch.sal_w[at] = (static_cast<uint32_t>((j >> 6) * kMfWCols * 16 + ((j >> 5) & 1) * 8) << 16) |
-                   (static_cast<uint32_t>((gv ? R.g : 0) * 8) << 8) | (static_cast<uint32_t>(bit + h - 15) & 31u);
-    ch.sal_xo[at] = static_cast<uint16_t>((pos + 8 * h) * 2);
-    ch.sal_cp[at] = (gv ? (h ? R.cp.z : R.cp.x) : 0u) ^ 0x80008000u;
-    q += is ? 1 : 0;
-  }
-  if ((utid & 31) == 0) {  // the first column of K tile utid / 32
-    ch.goff[utid >> 5] = kc + j < rank && gv ? make_uint2(static_cast<uint32_t>(kMfWrs * 4 + R.g * 8 + 4), ~0u)
-                                             : make_uint2(0u, 0u);
+    for (int h = 0; h < 2; ++h) {
+      // the column's group as the main pass takes it (uniform 64-column groups); an invalid group gives
+      // zero factors, as a K tile without a group does
+      const bool is = ((sal >> h) & 1u) != 0u;
+      const int at = is && q >= 0 && q < sal_cap ? q : sal_cap;
+      ch.sal_w[at] = (static_cast<uint32_t>((j >> 6) * kMfWCols * 16 + ((j >> 5) & 1) * 8) << 16) |
+                     (static_cast<uint32_t>((gv ? R.g : 0) * 8) << 8) | (static_cast<uint32_t>(bit + h - 15) & 31u);
+      ch.sal_xo[at] = static_cast<uint16_t>((pos + 8 * h) * 2);
+      ch.sal_cp[at] = (gv ? (h ? R.cp.z : R.cp.x) : 0u) ^ 0x80008000u;
+      q += is ? 1 : 0;
+    }
+    if ((utid & 31) == 0) {  // the first column of K tile utid / 32
+      ch.goff[utid >> 5] = kc + j < rank && gv ? make_uint2(static_cast<uint32_t>(MfWaveWords<kCompact>::kRs * 4 + R.g * 8 + 4), ~0u)
+                                               : make_uint2(0u, 0u);
+    }
   }
   if (utid < kMfSalWin) {
     // padding slots up to the last window's end read the zero activation column with zero factors
@@ -444,47 +453,61 @@ __device__ __forceinline__ void mf_cols_write(const MfmaProj& pa, int rc, int kc
     const int q = nsal + utid;
     if (q >= 0 && q < sal_cap && q < ((nsal + kMfSalWin - 1) & ~(kMfSalWin - 1))) {
       ch.sal_w[q] = 0u;
-      ch.sal_xo[q] = static_cast<uint16_t>(kMfChunk * 2);
+      ch.sal_xo[q] = static_cast<uint16_t>(kChunk * 2);
       ch.sal_cp[q] = 0x80008000u;
     }
-    // the zero column (and its neighbour, so that row 0 holds an aligned zero word)
-    if (utid < rc) *reinterpret_cast<uint32_t*>(&ch.xs[utid * kMfXStride + kMfChunk]) = 0u;
   }
+  // the zero column (and its neighbour, so that row 0 holds an aligned zero word)
+  if (utid < rc) *reinterpret_cast<uint32_t*>(&ch.xs[utid * mf_xstride(kCompact) + kChunk]) = 0u;
 }
 
-// Activation rows of a unit's chunk: wavefront `wave` loads rows 4 h + wave, a row's 512 columns 8 a lane.
-template <int kRuns>
+// Activation rows of a unit's chunk, 8 columns a lane: a wavefront's load h takes kRpl rows (one of 512 columns, two of
+// 256), and the four wavefronts neighbouring ones.
+template <int kRows, bool kCompact>
 struct MfRowRegs {
+  static constexpr int kRpl = kMfChunk / mf_chunk(kCompact);  // rows a load
+  static constexpr int kRuns = (kRows + 4 * kRpl - 1) / (4 * kRpl);
   uint4 xv[kRuns];
 };
 
 // Issue the loads of the row tile's rows: lane tok0 + r of roff holds the byte offset of row r in r_hid, or kMfOob (rows
 // past the tile, index entries that name no hidden row: they read zeros, as columns past the rank do).
-template <int kRuns>
+template <int kRows, bool kCompact>
 __device__ __forceinline__ void mf_rows_issue(__amdgpu_buffer_rsrc_t r_hid, int rank, int kc, int wave, int lane,
-                                              uint32_t roff, int tok0, MfRowRegs<kRuns>& R) {
-  const uint32_t col = kc + lane * 8 < rank ? static_cast<uint32_t>(kc + lane * 8) * 2u : kMfOob;
+                                              uint32_t roff, int tok0, MfRowRegs<kRows, kCompact>& R) {
+  constexpr int kRpl = MfRowRegs<kRows, kCompact>::kRpl;
+  const int c = kc + (lane % (kWave / kRpl)) * 8;
+  const uint32_t col = c < rank ? static_cast<uint32_t>(c) * 2u : kMfOob;
 #pragma unroll
-  for (int h = 0; h < kRuns; ++h) {
-    const int at = tok0 + 4 * h + wave;  // wave-uniform
-    const uint32_t ro = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(roff), at & (kWave - 1)));
+  for (int h = 0; h < MfRowRegs<kRows, kCompact>::kRuns; ++h) {
+    const int at = tok0 + kRpl * (4 * h + wave);  // wave-uniform
+    uint32_t ro = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(roff), at & (kWave - 1)));
+    if constexpr (kRpl == 2) {
+      const uint32_t r1 = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(roff), (at + 1) & (kWave - 1)));
+      ro = lane < kWave / 2 ? ro : r1;
+    }
     R.xv[h] = bload128(r_hid, __builtin_elementwise_add_sat(ro, col), 0u);
   }
 }
 
 // Writes the loaded rows to LDS in the staged order.
-template <int kRuns>
-__device__ __forceinline__ void mf_rows_write(const MfRowRegs<kRuns>& R, int rc, int wave, int lane, uint16_t* xs) {
-  const int c = lane * 8;  // run start within the chunk
+template <int kRows, bool kCompact>
+__device__ __forceinline__ void mf_rows_write(const MfRowRegs<kRows, kCompact>& R, int rc, int wave, int lane,
+                                              uint16_t* xs) {
+  constexpr int kRpl = MfRowRegs<kRows, kCompact>::kRpl;
+  const int c = (lane % (kWave / kRpl)) * 8;  // run start within the chunk
   uint16_t* const dst = xs + (c & ~31) + 2 * ((c >> 2) & 3) + ((c >> 4) & 1);
 #pragma unroll
-  for (int h = 0; h < kRuns; ++h) {
-    const int r = 4 * h + wave;
-    if (r < rc) {  // wave-uniform
+  for (int h = 0; h < MfRowRegs<kRows, kCompact>::kRuns; ++h) {
+    const int r0 = kRpl * (4 * h + wave);  // wave-uniform
+    if (r0 < rc) {
+      const int r = kRpl == 2 ? r0 + lane / (kWave / kRpl) : r0;
       const uint32_t w[4] = {R.xv[h].x, R.xv[h].y, R.xv[h].z, R.xv[h].w};
+      if (kRpl == 1 || r < rc) {
 #pragma unroll
-      for (int x = 0; x < 8; ++x) {  // column c + x
-        dst[r * kMfXStride + 8 * (x & 3) + 2 * (x >> 2)] = static_cast<uint16_t>(w[x >> 1] >> (16 * (x & 1)));
+        for (int x = 0; x < 8; ++x) {  // column c + x
+          dst[r * mf_xstride(kCompact) + 8 * (x & 3) + 2 * (x >> 2)] = static_cast<uint16_t>(w[x >> 1] >> (16 * (x & 1)));
+        }
       }
     }
   }
@@ -528,6 +551,7 @@ __device__ __forceinline__ void mf_chunk_write(const MfmaProj& pa, int kc, int u
 // (backbone_reduce_at) writes.  Thread utid of the unit takes columns 2 utid and 2 utid + 1 of each row, with
 // kMfPartialBatch slices' loads in flight.
 constexpr int kMfPartialBatch = 16;
+template <bool kCompact>
 __device__ __forceinline__ void mf_partials_stage(const MfmaProj& pa, int row0, int rc, int utid, const MfChunk& ch) {
   const int rank = pa.p.rank;
   const int c = 2 * utid;
@@ -555,8 +579,8 @@ __device__ __forceinline__ void mf_partials_stage(const MfmaProj& pa, int row0, 
       }
     }
     if (c < rank) {
-      ch.xs[i * kMfXStride + pos0] = f2h_bits(a0);
-      ch.xs[i * kMfXStride + pos1] = f2h_bits(a1);
+      ch.xs[i * mf_xstride(kCompact) + pos0] = f2h_bits(a0);
+      ch.xs[i * mf_xstride(kCompact) + pos1] = f2h_bits(a1);
     }
   }
 }
@@ -613,6 +637,7 @@ struct MfWaveSrc {
   int rs_cols;           // columns from the wavefront's first to the expert's last
   uint32_t v_q1, v_dec;  // lane l: packed row kc / 32 + l / 4, columns 16 wave + 4 (l % 4) ..
 };
+template <bool kCompact>
 __device__ __forceinline__ MfWaveSrc mf_wave_src(const MfmaProj& pa, int s, int e, int kc, int wave, int lane) {
   const tris_compact3_payload& p = pa.p;
   const int N = p.outfeatures;
@@ -629,8 +654,10 @@ __device__ __forceinline__ MfWaveSrc mf_wave_src(const MfmaProj& pa, int s, int 
   w.q1_bytes = static_cast<uint32_t>(packed_rows) * N * 4u;
   w.dec_bytes = static_cast<uint32_t>(nblk) * kGrWords * 4u;
   w.rs_cols = N - kMfWCols * wave;
-  w.v_q1 = (pr * N + c) * 4u;
-  w.v_dec = ((pr >> 1) * nob * kGrWords + (pr & 1u) * kTileOut + c) * 4u;
+  // packed rows past the rank (or past the staged chunk's) read nothing
+  const bool rv = static_cast<int>(pr) < packed_rows && lane / 4 < MfWaveWords<kCompact>::kPR;
+  w.v_q1 = rv ? (pr * N + c) * 4u : kMfOob;
+  w.v_dec = rv ? ((pr >> 1) * nob * kGrWords + (pr & 1u) * kTileOut + c) * 4u : kMfOob;
   return w;
 }
 
@@ -652,9 +679,8 @@ __device__ __forceinline__ void bload_words(__amdgpu_buffer_rsrc_t r, uint32_t v
 
 // Issues the wavefront's loads of its 16 columns of output tile ob: one 16-byte load a lane for the packed rows'
 // qweight1 words, one for their split words, one for the row scales (16 / 16 / 8 or 16 bytes; kSingle: a word at a time).
-// Nothing is masked: an offset past its buffer reads zeros, and what lies inside it but past the chunk's rows, the
-// groups or column N (the next row's words, the next tile's block) only feeds packed rows the compute skips, scales it
-// does not read or output columns that are not stored.  valid = false (a prefetch with no tile to fetch, wave-uniform)
+// An offset past its buffer reads zeros, and what lies inside it but past the groups or column N (the next row's words,
+// the next tile's block) only feeds scales that are not read or output columns that are not stored.  valid = false (a prefetch with no tile to fetch, wave-uniform)
 // empties the buffers, so every load reads zeros without a memory access: a workgroup does not fetch the tile after
 // its run, which another workgroup reads (likely through another XCD's L2).
 template <bool kCompact, bool kSingle>
@@ -679,12 +705,14 @@ __device__ __forceinline__ void mf_wave_tile_write(const MfWaveRegs<kCompact>& r
   constexpr int kRsLane = MfWaveWords<kCompact>::kRsLane;
   const int row = lane / 4;
   uint32_t* dst = wb + kMfWw + ((row >> 1) * kMfWCols + 4 * (lane % 4)) * 4 + (row & 1) * 2;
+  if (!kCompact || row < MfWaveWords<kCompact>::kPR) {
 #pragma unroll
-  for (int i = 0; i < 4; ++i) *reinterpret_cast<uint2*>(dst + 4 * i) = make_uint2(r.q[i], r.g[i]);
+    for (int i = 0; i < 4; ++i) *reinterpret_cast<uint2*>(dst + 4 * i) = make_uint2(r.q[i], r.g[i]);
+  }
   if constexpr (kRsLane == 4) {
-    *reinterpret_cast<uint4*>(wb + kMfWrs + lane * 4) = make_uint4(r.rs[0], r.rs[1], r.rs[2], r.rs[3]);
+    *reinterpret_cast<uint4*>(wb + MfWaveWords<kCompact>::kRs + lane * 4) = make_uint4(r.rs[0], r.rs[1], r.rs[2], r.rs[3]);
   } else {
-    *reinterpret_cast<uint2*>(wb + kMfWrs + lane * 2) = make_uint2(r.rs[0], r.rs[1]);
+    *reinterpret_cast<uint2*>(wb + MfWaveWords<kCompact>::kRs + lane * 2) = make_uint2(r.rs[0], r.rs[1]);
   }
 }
 
@@ -783,14 +811,15 @@ __device__ __forceinline__ void mf_salient_weights(const MfChunk& ch, const MfTi
 // columns.  The staged slot words carry every column-dependent offset, so a slot costs three LDS reads (its
 // qweight1 word, its group's R0 | R1, its activation) and no masking: padding slots read zero factors and the
 // zero activation column.  q1_lane / rs_lane: the byte offsets of the lane's column in the wavefront's qweight1
-// words and in its row-scale block (of wb, kStride words a tile); q2w: the lane's qweight2_sparse words of rows (sbase0 + w0) / 32 and the next
+// words and in its row-scale block (of wb); q2w: the lane's qweight2_sparse words of rows (sbase0 + w0) / 32 and the next
 // (a window spans at most two), q2off = (sbase0 + w0) % 32 + 8 kg the bit of slot 0 in q2w[0] | q2w[1] << 32.
-template <int kNs, int kRt, int kStride>
+template <int kNs, int kRt, bool kCompact>
 __device__ __forceinline__ void mf_salient_operands(const MfChunk& ch, const uint32_t* wb,
                                                     const uint16_t* const (&xr)[kRt], uint32_t q1_lane,
                                                     uint32_t rs_lane, int kg, int w0, int q2off,
                                                     const uint32_t (&q2w)[kNs][2], f16x8 (&av)[kRt],
                                                     f16x8 (&bv)[kNs]) {
+  constexpr int kStride = MfWaveWords<kCompact>::kAlloc;
   const int s0 = w0 + 8 * kg;  // a multiple of 8: the slot vectors are 16-byte aligned
   const uint4 swa = *reinterpret_cast<const uint4*>(&ch.sal_w[s0]);
   const uint4 swb = *reinterpret_cast<const uint4*>(&ch.sal_w[s0 + 4]);
@@ -803,7 +832,7 @@ __device__ __forceinline__ void mf_salient_operands(const MfChunk& ch, const uin
 #pragma unroll
     for (int b = 0; b < kNs; ++b) {
       const unsigned char* q1b = reinterpret_cast<const unsigned char*>(wb + b * kStride + kMfWw) + q1_lane;
-      const unsigned char* rsb = reinterpret_cast<const unsigned char*>(wb + b * kStride + kMfWrs) + rs_lane;
+      const unsigned char* rsb = reinterpret_cast<const unsigned char*>(wb + b * kStride + MfWaveWords<kCompact>::kRs) + rs_lane;
       w1v[b][u] = *reinterpret_cast<const uint32_t*>(q1b + (sw[u] >> 16));
       rrv[b][u] = *reinterpret_cast<const uint32_t*>(rsb + ((sw[u] >> 8) & 0xFFu));
     }
@@ -885,14 +914,16 @@ __device__ __forceinline__ void mf_q2_issue(const uint32_t* q2, int q2rows, int 
 // its workgroups share few passes over the code: unrolled over the chunk, a pass was about 8 KB of instructions a tile
 // and the first one of each wavefront took 20000 cycles against 8400 for the next (T = 16 gate/up; timestamps
 // in the kernel), the difference being instruction fetch.
-template <int kNs, int kRt, int kStride>
+template <int kNs, int kRt, bool kCompact>
 __device__ __forceinline__ void mf_compute(const uint32_t* q2, int q2rows, int N, int rank, int G, int kc,
                                            const int (&n)[kNs], const uint16_t* const (&xr)[kRt], int lane,
                                            const MfChunk& ch, const MfChunkMeta& cm, const uint32_t* wb,
                                            const uint32_t (&q2w0)[kNs][2], f32x4 (&acc)[kNs][kRt]) {
   const int i16 = lane % 16;   // MFMA column within the wave's 16 outputs / A row
   const int kg = lane / 16;    // MFMA k group: columns k = kg (mod 4) of every packed row
-  const int nt = (rank - kc) / kTileK < kMfTiles ? (rank - kc) / kTileK : kMfTiles;  // K tiles (rank % 64 == 0)
+  constexpr int kStride = MfWaveWords<kCompact>::kAlloc;
+  constexpr int kTiles = mf_chunk(kCompact) / kTileK;
+  const int nt = (rank - kc) / kTileK < kTiles ? (rank - kc) / kTileK : kTiles;  // K tiles (rank % 64 == 0)
 
   // ---- MFMA over the chunk's packed rows (salient columns have zero factors here).  Each packed row's LDS reads
   // are issued as soon as the same row of the K tile before is computed.
@@ -914,7 +945,7 @@ __device__ __forceinline__ void mf_compute(const uint32_t* q2, int q2rows, int N
 #pragma unroll
     for (int m = 0; m < kRt; ++m) r.av[m] = *reinterpret_cast<const uint4*>(xp[m] + 32 * h);
     r.cd = *reinterpret_cast<const uint4*>(cp + 32 * h);
-    r.cn = *reinterpret_cast<const uint4*>(cp + kMfChunk + 32 * h);
+    r.cn = *reinterpret_cast<const uint4*>(cp + mf_chunk(kCompact) + 32 * h);
     return r;
   };
   auto row_mfma = [&](const Row& r, const uint32_t (&rs2)[kNs]) {
@@ -963,7 +994,7 @@ __device__ __forceinline__ void mf_compute(const uint32_t* q2, int q2rows, int N
   const int num_sal = cm.num_sal;
   auto window = [&](int w0, const uint32_t (&q2w)[kNs][2]) {
     f16x8 av[kRt], bv[kNs];
-    mf_salient_operands<kNs, kRt, kStride>(ch, wb, xr, static_cast<uint32_t>(i16 * 16), rs_lane, kg, w0,
+    mf_salient_operands<kNs, kRt, kCompact>(ch, wb, xr, static_cast<uint32_t>(i16 * 16), rs_lane, kg, w0,
                                   ((sbase0 + w0) & 31) + 8 * kg, q2w, av, bv);
 #pragma unroll
     for (int b = 0; b < kNs; ++b) {
@@ -1010,23 +1041,29 @@ __device__ __forceinline__ void mf_compute(const uint32_t* q2, int q2rows, int N
 // nothing is prefetched.
 // Registers are capped at what the LDS lets reside anyway: one unit with 4 staged rows fits four workgroups per CU
 // (128 VGPRs), with 16 rows three.
-// a / b for 0 <= a < 2^22 and b > 0 (wave-uniform): a reciprocal estimate corrected by one (the general 32-bit division
-// is some 20 dependent instructions, and every wavefront does three of these before its first load).
-__device__ __forceinline__ int mf_div(int a, int b) {
+// Wavefronts a SIMD each instance is held to: what its LDS lets reside anyway.
+constexpr int mf_waves(int units, int rows, bool compact) {
+  return units == 2 ? 2 : (rows > kMfRows && !compact ? 2 : 3);
+}
+
+// a / b for b > 0 (wave-uniform).  Below 2^22 a reciprocal estimate corrected by one (the general 32-bit division is some
+// 20 dependent instructions, and every wavefront does some of these before its first load).
+__device__ __forceinline__ uint32_t mf_div(uint32_t a, uint32_t b) {
+  if (a >= (1u << 22)) return a / b;  // uniform
   int q = static_cast<int>(static_cast<float>(a) * __builtin_amdgcn_rcpf(static_cast<float>(b)));
-  const int r = a - q * b;
-  q += r >= b ? 1 : 0;
+  const int r = static_cast<int>(a) - q * static_cast<int>(b);
+  q += r >= static_cast<int>(b) ? 1 : 0;
   q -= r < 0 ? 1 : 0;
-  return __builtin_amdgcn_readfirstlane(q);
+  return static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(q));
 }
 
 template <int kUnits, int kRows, bool kCompact, bool kGeneral>
 __global__ __launch_bounds__(kUnits * kMfThreads)
-__attribute__((amdgpu_waves_per_eu(kUnits == 2 ? 2 : 3, 8)))
+__attribute__((amdgpu_waves_per_eu(mf_waves(kUnits, kRows, kCompact), 8)))
 void grouped_mfma_kernel(MfmaArgs a) {
   using WW = MfWaveWords<kCompact>;
   constexpr int kSal = mf_sal_slots(kCompact);
-  constexpr int kRuns = kRows / 4;
+  constexpr int kRowTile = kRows > kMfRows ? kRows : kMfRows;  // rows of a row tile (the 4-row instances have no more)
   const int unit = kUnits == 2 ? __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) / kMfThreads) : 0;
   const int which = kUnits == 2 ? unit : static_cast<int>(blockIdx.z);
   const MfmaProj& pa = a.proj[which];
@@ -1046,7 +1083,7 @@ void grouped_mfma_kernel(MfmaArgs a) {
   // (without one, any readable words)
   const int64_t* const any_index = row_index != nullptr ? row_index : reinterpret_cast<const int64_t*>(p.col_pack3);
   const int64_t early = any_index[row_index != nullptr ? (lane < a.batch ? lane : a.batch - 1) : 0];
-  const MfSegScan sc = mf_scan_segments(a.segment_offsets, a.expert_ids, a.num_segments, kMfRows);
+  const MfSegScan sc = mf_scan_segments(a.segment_offsets, a.expert_ids, a.num_segments, kRowTile);
   const int R = __builtin_amdgcn_readfirstlane(sc.total);
   if (R == 0) return;  // no rows
   // the one-token combine: the two units take row tiles 0 and 1 of the same output tiles, so the workgroups share
@@ -1055,21 +1092,29 @@ void grouped_mfma_kernel(MfmaArgs a) {
   const int Rm = comb ? 1 : R;
   const int W = static_cast<int>(gridDim.x);
   const int w = static_cast<int>(blockIdx.x);
-  // workgroup w is the (w / Rm)-th of row tile w % Rm (its activations and column data stay with few XCDs); that tile's
-  // workgroups split its output tiles into runs, and those past its output tiles, the last of the grid, are idle.  With
-  // more row tiles than workgroups, each takes row tiles w, w + W, ... whole.
-  int rt_first = w, rt_step = W, ob_lo = 0, ob_hi = nob;
-  if (Rm <= W) {
-    const int per = mf_div(W, Rm);
-    const int sub = mf_div(w, Rm);
-    rt_first = w - sub * Rm;
-    int cnt = per + (rt_first < W - per * Rm ? 1 : 0);
-    cnt = cnt < nob ? cnt : nob;
+  // The workgroup's (row tile, output tile) pairs [t_lo, t_hi), row-tile major.  As long as there are enough workgroups,
+  // workgroup w is the (w / Rm)-th of row tile w % Rm (its activations and column data stay with few XCDs); that
+  // tile's workgroups split its output tiles into runs, and those past its output tiles, the last of the grid, are idle.
+  // With fewer than three workgroups a row tile the runs would differ by half or more; where they are long (8 output
+  // tiles and up) all pairs are split evenly instead, and a run may go on in the next row tile, which it stages too
+  // (A3B T = 1024, 257 row tiles on 768 workgroups: down 64 -> 58 us; the gate/up launch's runs of five: 39 -> 40 us).
+  uint32_t t_lo, t_hi;
+  const uint32_t total = static_cast<uint32_t>(Rm) * nob;
+  if (Rm * 3 <= W || (Rm <= W && total < 8u * W)) {
+    const uint32_t per = mf_div(W, Rm);
+    const uint32_t sub = mf_div(w, Rm);
+    const uint32_t rt = w - sub * Rm;
+    uint32_t cnt = per + (rt < W - per * Rm ? 1u : 0u);
+    cnt = cnt < static_cast<uint32_t>(nob) ? cnt : nob;
     if (sub >= cnt) return;
-    const int run = mf_div(nob, cnt), more = nob - run * cnt;  // the first `more` runs have one output tile more
-    ob_lo = sub * run + (sub < more ? sub : more);
-    ob_hi = ob_lo + run + (sub < more ? 1 : 0);
-    rt_step = Rm;  // one row tile
+    const uint32_t run = mf_div(nob, cnt), more = nob - run * cnt;  // the first `more` runs have one output tile more
+    t_lo = rt * nob + sub * run + (sub < more ? sub : more);
+    t_hi = t_lo + run + (sub < more ? 1u : 0u);
+  } else {
+    const uint32_t run = mf_div(total, W), more = total - run * W;
+    t_lo = w * run + (static_cast<uint32_t>(w) < more ? w : more);
+    t_hi = t_lo + run + (static_cast<uint32_t>(w) < more ? 1u : 0u);
+    if (t_hi <= t_lo) return;
   }
   // the combine's weights by row (w_row[inverse_perm[s]] = w[s]); a route that is not one token on two experts,
   // one row each, gets zero outputs (before any barrier, the same in both units)
@@ -1079,14 +1124,14 @@ void grouped_mfma_kernel(MfmaArgs a) {
     bool ok = R == 2 && ((inv0 == 0 && inv1 == 1) || (inv0 == 1 && inv1 == 0));
     for (int t = 0; t < 2 && ok; ++t) {
       int cs = 0, cr0 = 0, crc = 0, ce = -1;
-      mf_map_scanned(sc, a.segment_offsets, a.expert_ids, a.num_segments, t, kMfRows, &cs, &cr0, &crc, &ce);
+      mf_map_scanned(sc, a.segment_offsets, a.expert_ids, a.num_segments, t, kRowTile, &cs, &cr0, &crc, &ce);
       ce = __builtin_amdgcn_readfirstlane(ce);
       ok = __builtin_amdgcn_readfirstlane(crc) == 1 && ce >= 0 && ce < num_experts;
     }
     if (!ok) {
       if (unit == 0) {
         const int t0 = static_cast<int>(threadIdx.x) % kMfThreads;
-        for (int n = ob_lo * kTileOut + t0; n < ob_hi * kTileOut && n < p.outfeatures; n += kMfThreads) a.comb_out[n] = 0;
+        for (int n = t_lo * kTileOut + t0; n < static_cast<int>(t_hi) * kTileOut && n < p.outfeatures; n += kMfThreads) a.comb_out[n] = 0;
       }
       return;
     }
@@ -1094,17 +1139,17 @@ void grouped_mfma_kernel(MfmaArgs a) {
     wr1 = a.comb_w[inv0 == 0 ? 1 : 0];
   }
   uint16_t* out = kUnits == 2 ? a.proj[0].out : pa.out;
-  __shared__ __attribute__((aligned(16))) uint16_t mf_xs[kUnits][kRows * kMfXStride];
-  __shared__ __attribute__((aligned(16))) uint16_t mf_cds[kUnits][2 * kMfChunk];  // C_d, then C_nd
-  __shared__ __attribute__((aligned(16))) uint2 mf_goff[kUnits][kMfTiles];
+  __shared__ __attribute__((aligned(16))) uint16_t mf_xs[kUnits][kRows * mf_xstride(kCompact)];
+  __shared__ __attribute__((aligned(16))) uint16_t mf_cds[kUnits][2 * mf_chunk(kCompact)];  // C_d, then C_nd
+  __shared__ __attribute__((aligned(16))) uint2 mf_goff[kUnits][mf_chunk(kCompact) / kTileK];
   __shared__ __attribute__((aligned(16))) uint32_t mf_salw[kUnits][kSal + 4];  // (one spare slot)
   __shared__ __attribute__((aligned(16))) uint16_t mf_salxo[kUnits][kSal + 8];
   __shared__ __attribute__((aligned(16))) uint32_t mf_salcp[kUnits][kSal + 4];
-  __shared__ __attribute__((aligned(16))) float mf_exch[kUnits == 2 ? kMfThreads * 4 * 2 : 4];
+  __shared__ __attribute__((aligned(16))) float mf_exch[kUnits == 2 ? kMfThreads * 4 * 2 * (kRowTile / kMfRows) : 4];
   MfChunk ch;
   ch.xs = &mf_xs[unit][0];
   ch.cds = &mf_cds[unit][0];
-  ch.cns = &mf_cds[unit][kMfChunk];
+  ch.cns = &mf_cds[unit][mf_chunk(kCompact)];
   ch.goff = &mf_goff[unit][0];
   ch.col_sal = nullptr;
   ch.sal_col = nullptr;
@@ -1120,18 +1165,22 @@ void grouped_mfma_kernel(MfmaArgs a) {
   if (lane < 2) wb[lane * WW::kAlloc] = 0u;  // the zero words (the first row tile's barrier orders these writes)
   float* exch = mf_exch;
 
-  for (int rt_i = rt_first; rt_i < Rm; rt_i += rt_step) {
+  for (uint32_t t = t_lo; t < t_hi;) {
+  const int rt_i = static_cast<int>(mf_div(t, nob));
   // the lane index and sizes of this row tile: opaque, so that the many addresses and conditions made of them are not
   // computed ahead of the loop and held across it (most launches run it once, and the held registers spill)
   int ln = lane, N = p.outfeatures, rank = p.rank, G = p.num_groups, nseg = a.num_segments;
-  int ob_begin = ob_lo, ob_end = ob_hi;
+  int ob_begin = static_cast<int>(t - static_cast<uint32_t>(rt_i) * nob), ob_end = ob_begin + static_cast<int>(t_hi - t);
+  ob_end = ob_end < nob ? ob_end : nob;
+  const bool first = t == t_lo;
+  t += ob_end - ob_begin;
   asm volatile("" : "+v"(ln), "+s"(N), "+s"(rank), "+s"(G), "+s"(nseg), "+s"(ob_begin), "+s"(ob_end));
   const int utid = wave * kWave + ln;
   const int i16 = ln % 16;
   const int kg = ln / 16;
   const int rt = comb ? unit : rt_i;  // the combine's units: row tiles 0 and 1
   int s = 0, row0 = 0, rc = 0, e = -1;
-  mf_map_scanned(sc, a.segment_offsets, a.expert_ids, nseg, rt, kMfRows, &s, &row0, &rc, &e);
+  mf_map_scanned(sc, a.segment_offsets, a.expert_ids, nseg, rt, kRowTile, &s, &row0, &rc, &e);
   s = __builtin_amdgcn_readfirstlane(s);  // the mapping is the same in every lane
   row0 = __builtin_amdgcn_readfirstlane(row0);
   rc = __builtin_amdgcn_readfirstlane(rc);
@@ -1150,11 +1199,8 @@ void grouped_mfma_kernel(MfmaArgs a) {
     }
     continue;
   }
-  if (rt_i != rt_first) __syncthreads();  // the previous row tile's LDS readers are done
-  // A operand row of this lane: rows past rc feed output rows that are not stored, so they read row 0 (the same
-  // LDS words as lane 0's rows: broadcast reads instead of bank conflicts; T = 16 gate/up launch 33.2 -> 32.5 us)
-  const uint16_t* const xr[1] = {ch.xs + (i16 < rc ? i16 : 0) * kMfXStride};
-  const MfWaveSrc src = mf_wave_src(pa, ds, e, 0, wave, ln);
+  if (!first) __syncthreads();  // the previous row tile's LDS readers are done
+  const MfWaveSrc src = mf_wave_src<kCompact>(pa, ds, e, 0, wave, ln);
   const uint32_t* q2 = reinterpret_cast<const uint32_t*>(p.qweight2_sparse) +
                        static_cast<int64_t>(e) * p.qweight2_sparse_rows * N;
   const int q2rows = p.qweight2_sparse_rows;
@@ -1169,7 +1215,7 @@ void grouped_mfma_kernel(MfmaArgs a) {
     tok0 = 0;
   }
   const int hidden_rows = row_index != nullptr ? pa.hidden_rows : rc;
-  const uint32_t roff = entry >= 0 && entry < hidden_rows && ln - tok0 < rc
+  const uint32_t roff = entry >= 0 && entry < hidden_rows && static_cast<uint32_t>(ln - tok0) < static_cast<uint32_t>(rc)
                             ? static_cast<uint32_t>(entry) * static_cast<uint32_t>(rank) * 2u : kMfOob;
   const __amdgpu_buffer_rsrc_t r_hid =
       make_rsrc(pa.hidden + (row_index != nullptr ? 0 : static_cast<int64_t>(row0) * rank),
@@ -1177,29 +1223,24 @@ void grouped_mfma_kernel(MfmaArgs a) {
   MfChunkMeta cm;
   {  // chunk 0 and the first tiles' weights
     MfColRegs cols;
-    MfRowRegs<kRuns> rows;
-    mf_cols_issue(pa, e, 0, utid, cols);
-    mf_rows_issue<kRuns>(r_hid, rank, 0, wave, ln, roff, tok0, rows);
+    MfRowRegs<kRows, kCompact> rows;
+    mf_cols_issue<kCompact>(pa, e, 0, utid, cols);
+    mf_rows_issue<kRows, kCompact>(r_hid, rank, 0, wave, ln, roff, tok0, rows);
     mf_wave_tile_issue<kCompact, kGeneral>(src, G, ob_begin, ln, wr[0]);
     mf_wave_tile_issue<kCompact, kGeneral>(src, G, ob_begin + 1, ln, wr[1], !kGeneral && ob_begin + 1 < ob_end);
-    mf_cols_write(pa, rc, 0, utid, ch, cols, kSal);
-    if (!part) mf_rows_write<kRuns>(rows, rc, wave, ln, ch.xs);
-    if (part) mf_partials_stage(pa, row0, rc, utid, ch);  // one chunk (host-checked)
+    mf_cols_write<kCompact>(pa, rc, 0, utid, ch, cols, kSal);
+    if (!part) mf_rows_write<kRows, kCompact>(rows, rc, wave, ln, ch.xs);
+    if (part) mf_partials_stage<kCompact>(pa, row0, rc, utid, ch);  // one chunk (host-checked)
     cm = mf_chunk_meta(cols, kSal);
     mf_wave_tile_write<kCompact>(wr[0], ln, wb);
     mf_wave_tile_write<kCompact>(wr[1], ln, wb + WW::kAlloc);
     __syncthreads();
   }
-  // The outputs of tile ob, from its accumulators.  Stores go through a buffer resource over the tile's rows from its
-  // first column: rows past rc have an offset past it and are dropped, so every lane issues all four; only the
-  // expert's last tile can have columns past N.
+  // The outputs of rows 16 m .. of tile ob, from their accumulators.  Stores go through a buffer resource over the
+  // tile's rows from its first column: rows past rc have an offset past it and are dropped, so every lane issues all
+  // four; only the expert's last tile can have columns past N.
   uint16_t* const out0 = out + static_cast<int64_t>(row0) * N;
-  uint32_t orow[4];
-#pragma unroll
-  for (int v = 0; v < 4; ++v) {
-    orow[v] = 4 * kg + v < rc ? static_cast<uint32_t>((4 * kg + v) * N + 16 * wave + i16) * 2u : kMfOob;
-  }
-  auto store = [&](int ob, const f32x4& acc, const float* ex) {
+  auto store = [&](int ob, int m, const f32x4& acc, const float* ex) {
     const int n = ob * kTileOut + 16 * wave + i16;
     if (kUnits == 2 && comb) {
       // row 0 of each unit's tile (one row a tile): the combine of the token's two rows at column n, the products
@@ -1218,27 +1259,35 @@ void grouped_mfma_kernel(MfmaArgs a) {
     f32x4 up = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
     if (kUnits == 2) up = *reinterpret_cast<const f32x4*>(&ex[utid * 4]);
     const __amdgpu_buffer_rsrc_t r_out = make_rsrc(out0 + ob * kTileOut, static_cast<uint32_t>(rc * N - ob * kTileOut) * 2u);
-    const bool edge = (ob + 1) * kTileOut > N;  // uniform
+    const int r0 = 16 * m + 4 * kg;  // the lane's rows r0 .. r0 + 3
+    const uint32_t vo = n < N ? static_cast<uint32_t>(r0 * N + 16 * wave + i16) * 2u : kMfOob;
 #pragma unroll
     for (int v = 0; v < 4; ++v) {
       // two units: g and u rounded to fp16 as the two outputs would be.  One unit: no output scale or bias here, the
       // host sends none (launch_grouped_mfma rejects payloads with them)
       const uint16_t y = kUnits == 2 ? swiglu_bits(f2h_bits(acc[v]), f2h_bits(up[v])) : f2h_bits(acc[v]);
-      uint32_t vo = orow[v];
-      if (edge) vo = n < N ? vo : kMfOob;
-      __builtin_amdgcn_raw_buffer_store_b16(y, r_out, vo, 0u, 0);
+      __builtin_amdgcn_raw_buffer_store_b16(y, r_out, r0 + v < rc ? vo + static_cast<uint32_t>(v * N) * 2u : kMfOob, 0u,
+                                            0);
     }
   };
-  // kNs output tiles from `ob`, whose words are in wb; with one chunk the next tiles' words are loaded to registers
-  // meanwhile and written to wb after the last read of this pass (one wavefront's LDS operations stay in order).
-  auto tiles = [&](auto ns, int ob) {
+  // kNs output tiles from `ob`, whose words are in wb, kRt 16-row sub-tiles; with one chunk the next tiles' words are
+  // loaded to registers meanwhile and written to wb after the last read of this pass (one wavefront's LDS operations
+  // stay in order).
+  auto tiles = [&](auto ns, auto nrt, int ob) {
     constexpr int kNs = decltype(ns)::value;
-    f32x4 acc[kNs][1];
+    constexpr int kRt = decltype(nrt)::value;
+    f32x4 acc[kNs][kRt];
     int n[kNs];
     uint32_t q2w[kNs][2];
+    // A operand rows of this lane: rows past rc feed output rows that are not stored, so they read row 0 (the same
+    // LDS words as lane 0's rows: broadcast reads instead of bank conflicts; T = 16 gate/up launch 33.2 -> 32.5 us)
+    const uint16_t* xr[kRt];
+#pragma unroll
+    for (int m = 0; m < kRt; ++m) xr[m] = ch.xs + (16 * m + i16 < rc ? 16 * m + i16 : 0) * mf_xstride(kCompact);
 #pragma unroll
     for (int b = 0; b < kNs; ++b) {
-      acc[b][0] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+      for (int m = 0; m < kRt; ++m) acc[b][m] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
       n[b] = (ob + b) * kTileOut + 16 * wave + i16;
     }
     if constexpr (!kGeneral) {
@@ -1249,7 +1298,7 @@ void grouped_mfma_kernel(MfmaArgs a) {
         mf_wave_tile_issue<kCompact, kGeneral>(src, G, ob + kNs + b, ln, wr[b], ob + kNs + b < ob_end);
       }
       __builtin_amdgcn_sched_barrier(0);  // the loads stay ahead of the pass they overlap
-      mf_compute<kNs, 1, WW::kAlloc>(q2, q2rows, N, rank, G, 0, n, xr, ln, ch, cm, wb, q2w, acc);
+      mf_compute<kNs, kRt, kCompact>(q2, q2rows, N, rank, G, 0, n, xr, ln, ch, cm, wb, q2w, acc);
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
       for (int b = 0; b < 2; ++b) mf_wave_tile_write<kCompact>(wr[b], ln, wb + b * WW::kAlloc);
@@ -1258,46 +1307,67 @@ void grouped_mfma_kernel(MfmaArgs a) {
         if (ob > ob_begin || kc > 0) {
           __syncthreads();  // the previous chunk's readers are done
           MfColRegs cols;
-          MfRowRegs<kRuns> rows;
-          mf_wave_tile_issue<kCompact, kGeneral>(mf_wave_src(pa, ds, e, kc, wave, ln), G, ob, ln, wr[0]);
-          mf_cols_issue(pa, e, kc, utid, cols);
-          mf_rows_issue<kRuns>(r_hid, rank, kc, wave, ln, roff, tok0, rows);
-          mf_cols_write(pa, rc, kc, utid, ch, cols, kSal);
-          mf_rows_write<kRuns>(rows, rc, wave, ln, ch.xs);
+          MfRowRegs<kRows, kCompact> rows;
+          mf_wave_tile_issue<kCompact, kGeneral>(mf_wave_src<kCompact>(pa, ds, e, kc, wave, ln), G, ob, ln, wr[0]);
+          mf_cols_issue<kCompact>(pa, e, kc, utid, cols);
+          mf_rows_issue<kRows, kCompact>(r_hid, rank, kc, wave, ln, roff, tok0, rows);
+          mf_cols_write<kCompact>(pa, rc, kc, utid, ch, cols, kSal);
+          if (!part) mf_rows_write<kRows, kCompact>(rows, rc, wave, ln, ch.xs);  // (partial sums: one chunk, staged already)
           cm = mf_chunk_meta(cols, kSal);
           mf_wave_tile_write<kCompact>(wr[0], ln, wb);
           __syncthreads();
         }
         mf_q2_issue(q2, q2rows, N, n[0], cm, q2w[0]);
-        mf_compute<kNs, 1, WW::kAlloc>(q2, q2rows, N, rank, G, kc, n, xr, ln, ch, cm, wb, q2w, acc);
+        mf_compute<kNs, kRt, kCompact>(q2, q2rows, N, rank, G, kc, n, xr, ln, ch, cm, wb, q2w, acc);
       }
     }
     if (kUnits == 2) {
       if (unit == 1) {
 #pragma unroll
-        for (int b = 0; b < kNs; ++b) *reinterpret_cast<f32x4*>(&exch[(b * kMfThreads + utid) * 4]) = acc[b][0];
+        for (int b = 0; b < kNs; ++b) {
+#pragma unroll
+          for (int m = 0; m < kRt; ++m) *reinterpret_cast<f32x4*>(&exch[((b * kRt + m) * kMfThreads + utid) * 4]) = acc[b][m];
+        }
       }
       __syncthreads();
       if (unit == 0) {
 #pragma unroll
-        for (int b = 0; b < kNs; ++b) store(ob + b, acc[b][0], exch + b * kMfThreads * 4);
+        for (int b = 0; b < kNs; ++b) {
+#pragma unroll
+          for (int m = 0; m < kRt; ++m) store(ob + b, m, acc[b][m], exch + (b * kRt + m) * kMfThreads * 4);
+        }
       }
       __syncthreads();  // exch is rewritten by the next tiles
     } else {
 #pragma unroll
-      for (int b = 0; b < kNs; ++b) store(ob + b, acc[b][0], exch);
-    }
-  };
-  for (int ob = ob_begin; ob < ob_end;) {
-    if constexpr (!kGeneral) {
-      if (ob + 1 < ob_end) {
-        tiles(std::integral_constant<int, 2>{}, ob);
-        ob += 2;
-        continue;
+      for (int b = 0; b < kNs; ++b) {
+#pragma unroll
+        for (int m = 0; m < kRt; ++m) store(ob + b, m, acc[b][m], exch);
       }
     }
-    tiles(std::integral_constant<int, 1>{}, ob);
-    ob += 1;
+  };
+  // the run's output tiles, two at a time, with as many row sub-tiles as the row tile's rows need
+  auto run = [&](auto nrt) {
+    for (int ob = ob_begin; ob < ob_end;) {
+      if constexpr (!kGeneral) {
+        if (ob + 1 < ob_end) {
+          tiles(std::integral_constant<int, 2>{}, nrt, ob);
+          ob += 2;
+          continue;
+        }
+      }
+      tiles(std::integral_constant<int, 1>{}, nrt, ob);
+      ob += 1;
+    }
+  };
+  if (kRows <= 16 || rc <= 16) {  // uniform
+    run(std::integral_constant<int, 1>{});
+  } else if constexpr (kRows > 16) {
+    if (kRows <= 32 || rc <= 32) {
+      run(std::integral_constant<int, 2>{});
+    } else if constexpr (kRows > 32) {
+      run(std::integral_constant<int, 4>{});
+    }
   }
   }  // row tiles
 }
@@ -1312,7 +1382,14 @@ void grouped_mfma_kernel(MfmaArgs a) {
 // of LDS reads per clock on a CU (4 SIMDs), twice what the LDS delivers.  kUnits == 2 runs the gate and up
 // projections of the same item side by side and writes fp16(silu(g) * u).
 constexpr int kWsSalWindows = 2;  // salient columns per item <= 64
-constexpr int kWsMinRows = 64;    // mean rows per active segment from which the host picks this kernel
+// Mean rows per active segment from which the host picks this kernel: below, the decode kernel's row tiles of 32 rows
+// (64 at rank <= 256), which rebuild the operands for each row tile but start at once, are faster.  Gate/up + down
+// launches, decode against weight-stationary: rank 512 (Mixtral) at 83 rows 109 against 130 us, 112 rows 135 / 142, 130
+// rows 153 / 149, 150 rows 167 / 155; rank 256 (OLMoE) at 75 rows 63 / 109, 125 rows 83 / 129, 250 rows 132 / 171, 500
+// rows 240 / 243.  The general decode instance (16-row tiles) hands over earlier.
+constexpr int kWsMinRows = 120;
+constexpr int kWsMinRowsCompact = 500;
+constexpr int kWsMinRowsGeneral = 64;
 #ifndef TRIS_WS_SUB
 #define TRIS_WS_SUB 2
 #endif
@@ -1891,19 +1968,8 @@ int launch_grouped_mfma(const uint16_t* hidden_a, const uint16_t* hidden_b, int 
   const int units = (swiglu || comb_out != nullptr) ? 2 : 1;
   const int nproj = (pb && !swiglu) ? 2 : 1;
   hipStream_t s = static_cast<hipStream_t>(stream);
-  // long segments: keep each output tile's weights in registers and stream the segment's rows through them
-  // (its buffer resources address a segment's rows in 32-bit byte offsets: the whole batch must stay below 2 GiB)
-  if (partials == nullptr && num_segments <= kWave &&
-      static_cast<int64_t>(batch) >= static_cast<int64_t>(kWsMinRows) * num_segments &&
-      ws_fits(pa) && (!pb || ws_fits(pb)) && static_cast<int64_t>(batch) * max_n * 2 < (int64_t{1} << 31) &&
-      static_cast<int64_t>(batch) * kMfChunk * 2 < (int64_t{1} << 31)) {
-    return launch_grouped_mfma_ws(args, units, nproj, max_n, batch, s, who);
-  }
-  const int rows = batch <= 4 ? 4 : kMfRows;  // staged activation rows: a row tile has at most min(16, batch)
-  // the compact LDS layout (four workgroups per CU): at most 4 row-scale groups and 64 salient columns per expert,
-  // and rank <= 256, where a tile's work is short enough that the fourth workgroup's latency hiding pays (at
-  // rank 512 the 128-register cap and the coarser tile split cost more: measured on MI355X, OLMoE T=16 77 -> 73 us,
-  // Mixtral T=16 92.9 -> 95.5 us)
+  // the compact LDS layout: a chunk of 256 columns (rank <= 256), at most 4 row-scale groups and 64 salient columns per
+  // expert.  The 64-row tiles fit in it three workgroups a CU
   const auto compact_ok = [](const tris_compact3_payload* p) {
     return p->num_groups <= mf_groups_cap(true) && p->qweight2_sparse_rows * kMfSalWin <= mf_sal_slots(true) &&
            p->rank <= kMfChunk / 2;
@@ -1913,33 +1979,54 @@ int launch_grouped_mfma(const uint16_t* hidden_a, const uint16_t* hidden_b, int 
   // a tile at a time and loads nothing ahead
   const bool general = pa->rank > kMfChunk || !mf_wide(args.proj[0]) ||
                        (pb && (pb->rank > kMfChunk || !mf_wide(args.proj[1])));
-  const int lds_total = mf_static_lds_bytes(units, general ? kMfRows : rows, compact && !general);
+  const int ws_min = general ? kWsMinRowsGeneral : (compact ? kWsMinRowsCompact : kWsMinRows);
+  // long segments: keep each output tile's weights in registers and stream the segment's rows through them
+  // (its buffer resources address a segment's rows in 32-bit byte offsets: the whole batch must stay below 2 GiB)
+  if (partials == nullptr && num_segments <= kWave &&
+      static_cast<int64_t>(batch) >= static_cast<int64_t>(ws_min) * num_segments &&
+      ws_fits(pa) && (!pb || ws_fits(pb)) && static_cast<int64_t>(batch) * max_n * 2 < (int64_t{1} << 31) &&
+      static_cast<int64_t>(batch) * kMfChunk * 2 < (int64_t{1} << 31)) {
+    return launch_grouped_mfma_ws(args, units, nproj, max_n, batch, s, who);
+  }
+  // Staged activation rows: a row tile has at most min(row tile, batch).  From kMfTallMinRows rows a segment on average,
+  // row tiles of 32 rows (64 at rank <= 256, where they take half the LDS): a segment then rarely needs two, and its
+  // weights are built once, not once every 16 rows.
+  const bool tall = !general && partials == nullptr &&
+                    static_cast<int64_t>(batch) >= static_cast<int64_t>(kMfTallMinRows) * num_segments;
+  const int rows = general ? (partials != nullptr ? 4 : kMfRows) : (batch <= 4 ? 4 : (!tall ? kMfRows : (compact ? 64 : 32)));
+  const int lds_total = mf_static_lds_bytes(units, rows, compact && !general);
   TRIS_REQUIRE(lds_total <= 160 * 1024, "%s: LDS request %d exceeds a CU", who, lds_total);
-  // Workgroups: as many as the GPU holds at once (LDS and the kernel's 128 VGPRs per lane, 4 wavefronts
-  // per SIMD for one unit, bound them), shared by the projections of an unfused pair.
+  // Workgroups: as many as the GPU holds at once (LDS and the kernel's registers, mf_waves, bound them), shared by the
+  // projections of an unfused pair.
   int wgs_per_cu = (160 * 1024) / lds_total;
-  const int by_regs = units == 1 ? 3 : 1;
+  const int by_regs = units == 1 ? mf_waves(units, rows, compact) : 1;
   wgs_per_cu = wgs_per_cu < by_regs ? wgs_per_cu : by_regs;
   wgs_per_cu = wgs_per_cu > 0 ? wgs_per_cu : 1;
   int wgs = (kMfCus * wgs_per_cu) / nproj;
-  // no more than the (row tile, output tile) pairs there can be: row tiles <= batch / 16 + min(segments, batch)
-  const int64_t pairs =
-      (static_cast<int64_t>(batch) / kMfRows + (num_segments < batch ? num_segments : batch)) * ceil_div(max_n, kTileOut);
+  // no more than the (row tile, output tile) pairs there can be: row tiles <= batch / row tile + min(segments, batch)
+  const int64_t pairs = (static_cast<int64_t>(batch) / (rows > kMfRows ? rows : kMfRows) +
+                         (num_segments < batch ? num_segments : batch)) * ceil_div(max_n, kTileOut);
   if (pairs < wgs) wgs = static_cast<int>(pairs);
   if (comb_out != nullptr && ceil_div(max_n, kTileOut) < wgs) wgs = ceil_div(max_n, kTileOut);  // output tiles only
   const dim3 grid(wgs > 0 ? wgs : 1, 1, nproj);
   const dim3 block(units * kMfThreads);
 #define TRIS_MF_LAUNCH(U, ROWS, C, M) hipLaunchKernelGGL((grouped_mfma_kernel<U, ROWS, C, M>), grid, block, 0, s, args)
   if (units == 2) {
-    if (general) TRIS_MF_LAUNCH(2, kMfRows, false, true);
+    if (general && rows == 4) TRIS_MF_LAUNCH(2, 4, false, true);
+    else if (general) TRIS_MF_LAUNCH(2, kMfRows, false, true);
     else if (rows == 4 && compact) TRIS_MF_LAUNCH(2, 4, true, false);
     else if (rows == 4) TRIS_MF_LAUNCH(2, 4, false, false);
+    else if (rows == 64) TRIS_MF_LAUNCH(2, 64, true, false);
+    else if (rows == 32) TRIS_MF_LAUNCH(2, 32, false, false);
     else if (compact) TRIS_MF_LAUNCH(2, kMfRows, true, false);
     else TRIS_MF_LAUNCH(2, kMfRows, false, false);
   } else {
-    if (general) TRIS_MF_LAUNCH(1, kMfRows, false, true);
+    if (general && rows == 4) TRIS_MF_LAUNCH(1, 4, false, true);
+    else if (general) TRIS_MF_LAUNCH(1, kMfRows, false, true);
     else if (rows == 4 && compact) TRIS_MF_LAUNCH(1, 4, true, false);
     else if (rows == 4) TRIS_MF_LAUNCH(1, 4, false, false);
+    else if (rows == 64) TRIS_MF_LAUNCH(1, 64, true, false);
+    else if (rows == 32) TRIS_MF_LAUNCH(1, 32, false, false);
     else if (compact) TRIS_MF_LAUNCH(1, kMfRows, true, false);
     else TRIS_MF_LAUNCH(1, kMfRows, false, false);
   }

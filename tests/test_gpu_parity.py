@@ -730,6 +730,50 @@ def test_predecoded_long_segments(tris, oracle_mod, cuda, drop):
         assert not got[offs[drop]:offs[drop + 1]].any()
 
 
+@pytest.mark.parametrize("rank,n,segs", [
+    (256, 320, [1, 15, 16, 17, 32, 33, 48, 63, 64, 65, 0, 100]),   # 64-row tiles: every sub-tile count, a tile and a row
+    (192, 132, [64, 31, 33, 1]),                                   # a chunk that is not full
+    (512, 192, [16, 17, 31, 32, 33, 65, 0, 2]),                    # 32-row tiles
+    (448, 68, [20, 40, 1, 33]),
+    (512, 66, [20, 40, 1, 33]),                                    # columns no multiple of 4: the general instance
+    (576, 128, [5, 33, 20]),                                       # more than one chunk
+], ids=lambda v: str(v) if isinstance(v, int) else f"{len(v)}seg")
+def test_predecoded_row_tiles(tris, oracle_mod, cuda, rank, n, segs):
+    """Segments around the decode GEMM's row tiles (16, 32 and 64 rows, chosen by the mean rows a segment and the
+    rank), output columns that leave a partial tile and an odd tile of a pair, and the instance that takes column
+    counts 16-byte loads do not fit: against the oracle, and rows read through an index equal to the same rows
+    materialised, bit for bit."""
+    note(f"predecoded row tiles rank={rank} n={n} segs={segs}")
+    ext = tris["ext"]
+    E = len(segs)
+    pa = make_projection(tris, 91 + rank, E, n, rank)
+    pb = make_projection(tris, 92 + rank, E, n, rank)
+    da, db = (tris["qlinear"].payload_to_device(p, cuda) for p in (pa, pb))
+    ids, offs = _segments(segs, E)
+    prob = np.concatenate([[0], np.cumsum((np.diff(offs) + 3) // 4)]).astype(np.int32)
+    rng = np.random.default_rng(21)
+    rows = int(offs[-1])
+    tokens = rows // 2 + 1
+    ha, hb = ((rng.standard_normal((tokens, rank)) * 1.5).astype(np.float16) for _ in range(2))
+    idx = rng.integers(0, tokens, rows)
+    args = (t_i32(ids, cuda), t_i32(offs, cuda), t_i32(prob, cuda), int(prob[-1]))
+    nblk = tris["synthetic"].packing.num_gr_blocks(rank, n)
+    names = ("qweight1", "qweight2_sparse", "qweight2_sparse_prefix", "c_map", "g_idx", "col_pack3", "row_pack3")
+    dec = [ext.compact3_tris_precomputed_grouped_block_gr_predecode(
+        torch.empty((ids.size, nblk, 128), dtype=torch.int32, device=cuda), t_i32(ids, cuda), d["q_gmap_gr_words"],
+        d["q_gmap_gr_offsets"], d["q_gmap_gr_meta"], rank // 32, n) for d in (da, db)]
+    hd = [torch.from_numpy(h).to(cuda) for h in (ha, hb)]
+    got = ext.compact3_tris_precomputed_grouped_dual_forward_block_gr_predecoded(
+        hd[0], hd[1], *args, dec[0], *[da[k] for k in names], dec[1], *[db[k] for k in names], True,
+        row_index=torch.from_numpy(idx).to(cuda))
+    for y, p, d, b, h in zip(got, (pa, pb), (da, db), dec, (ha, hb)):
+        want = oracle_grouped(oracle_mod, p, h[idx], ids, offs, True)
+        assert_close(y.cpu().numpy().astype(np.float32), want.astype(np.float32), f"row tiles rank={rank} n={n}")
+        one = ext.compact3_tris_precomputed_grouped_forward_block_gr_predecoded(
+            torch.from_numpy(h[idx]).to(cuda), *args, b, *[d[k] for k in names], True)
+        assert torch.equal(one, y)
+
+
 @pytest.mark.parametrize("seg", [[3, 21, 0, 9], [90, 150, 0, 70]], ids=["short", "long"])
 def test_swiglu_fused_matches_dual_then_silu(tris, oracle_mod, cuda, seg):
     """The fused gate/up GEMM + SwiGLU equals silu(g) * u computed from the dual kernel's own fp16
