@@ -686,6 +686,21 @@ int tris_compact3_dual_linear_forward(const uint16_t* input, int32_t batch, cons
                                       void* stream);
 
 /*
+ * One to TRIS_MAX_LINEARS non-expert compact3 linears of one input (no reference counterpart: batches
+ * compact3_linear_forward calls, TriSMoE_cuda.cpp:497-700) on the matrix cores: tris_compact3_linear_forward's results
+ * up to the order of the fp32 sums, for any g_idx (K tiles of several groups take a scalar loop on the device).  Every
+ * payload has num_experts == 1 and the same rank, a multiple of 64; input and workspace are 16-byte aligned; input_scale
+ * applies to all, addend to the first; outputs[i] fp16 [batch, outfeatures of payload i].  The workspace (of
+ * tris_compact3_linears_workspace_bytes bytes) holds the decoded split bitmaps and fp32 partial sums.  A matrix gives the
+ * same bits alone and beside others of its output width (the split of K follows the widest).
+ */
+#define TRIS_MAX_LINEARS 3
+int64_t tris_compact3_linears_workspace_bytes(int32_t batch, int32_t rank, const int32_t* outfeatures, int32_t count);
+int tris_compact3_linears_forward(const uint16_t* input, int32_t batch, const tris_compact3_payload* payloads,
+                                  int32_t count, const uint16_t* input_scale, const float* addend,
+                                  uint16_t* const* outputs, void* workspace, int64_t workspace_bytes, void* stream);
+
+/*
  * output[b][n] = sum_k input[b][k] * weight[n][k] in fp32, no rounding; input fp16 (input_f16) or fp32
  * (input_f32, exactly one non-NULL), weight fp16 [out, in].  The non-expert linear's null-space term
  * C1 . (C2 . x) from the dequantised packed matrices, kept in fp32 as the reference's kernel does

@@ -408,7 +408,7 @@ __device__ __forceinline__ void mf_cols_issue(const MfmaProj& pa, int e, int kc,
 // exactly -fp16(C * R), so a set qweight1 bit is the selectors' sign bit) and zero for salient columns, whatever their
 // selector bits; the salient slots; the K tiles' row-scale offsets; the zero columns of the rc staged rows.  sal_cap:
 // the slots staged (a payload whose prefix counts disagree with its salient map writes no slot past them).
-template <bool kCompact>
+template <bool kCompact, bool kByTile = false>
 __device__ __forceinline__ void mf_cols_write(const MfmaProj& pa, int rc, int kc, int utid, const MfChunk& ch,
                                               const MfColRegs& R, int sal_cap) {
   constexpr int kChunk = mf_chunk(kCompact);
@@ -416,7 +416,9 @@ __device__ __forceinline__ void mf_cols_write(const MfmaProj& pa, int rc, int kc
   const int G = pa.p.num_groups;
   const int j = 2 * utid;
   const int pos = (j & ~31) + mf_perm32(j & 31);  // the second column's is pos + 8
-  const bool gv = R.g >= 0 && R.g < G;
+  // the column's place in the row-scale block: its group, or (kByTile: the block holds a pair per K tile) its K tile
+  const bool gv = kByTile || (R.g >= 0 && R.g < G);
+  const int place = kByTile ? j >> 6 : (gv ? R.g : 0);
   const int bit = j & 31;
   const uint32_t sal = kc + j < rank ? (R.cm >> bit) & 3u : 0u;
   const uint32_t cdn[2] = {R.cp.y ^ 0x80008000u, R.cp.w ^ 0x80008000u};  // C_d | C_nd << 16
@@ -437,13 +439,13 @@ __device__ __forceinline__ void mf_cols_write(const MfmaProj& pa, int rc, int kc
       const bool is = ((sal >> h) & 1u) != 0u;
       const int at = is && q >= 0 && q < sal_cap ? q : sal_cap;
       ch.sal_w[at] = (static_cast<uint32_t>((j >> 6) * kMfWCols * 16 + ((j >> 5) & 1) * 8) << 16) |
-                     (static_cast<uint32_t>((gv ? R.g : 0) * 8) << 8) | (static_cast<uint32_t>(bit + h - 15) & 31u);
+                     (static_cast<uint32_t>(place * 8) << 8) | (static_cast<uint32_t>(bit + h - 15) & 31u);
       ch.sal_xo[at] = static_cast<uint16_t>((pos + 8 * h) * 2);
       ch.sal_cp[at] = (gv ? (h ? R.cp.z : R.cp.x) : 0u) ^ 0x80008000u;
       q += is ? 1 : 0;
     }
     if ((utid & 31) == 0) {  // the first column of K tile utid / 32
-      ch.goff[utid >> 5] = kc + j < rank && gv ? make_uint2(static_cast<uint32_t>(MfWaveWords<kCompact>::kRs * 4 + R.g * 8 + 4), ~0u)
+      ch.goff[utid >> 5] = kc + j < rank && gv ? make_uint2(static_cast<uint32_t>(MfWaveWords<kCompact>::kRs * 4 + place * 8 + 4), ~0u)
                                                : make_uint2(0u, 0u);
     }
   }
@@ -684,18 +686,23 @@ __device__ __forceinline__ void bload_words(__amdgpu_buffer_rsrc_t r, uint32_t v
 // empties the buffers, so every load reads zeros without a memory access: a workgroup does not fetch the tile after
 // its run, which another workgroup reads (likely through another XCD's L2).
 template <bool kCompact, bool kSingle>
-__device__ __forceinline__ void mf_wave_tile_issue(const MfWaveSrc& w, int G, int ob, int lane,
-                                                   MfWaveRegs<kCompact>& r, bool valid = true) {
-  constexpr int kRsLane = MfWaveWords<kCompact>::kRsLane;
+__device__ __forceinline__ void mf_wave_words_issue(const MfWaveSrc& w, int ob, MfWaveRegs<kCompact>& r, bool valid) {
   const uint32_t col = static_cast<uint32_t>(ob) * kTileOut;
   const __amdgpu_buffer_rsrc_t r_q1 = make_rsrc(w.q1 + col, valid ? w.q1_bytes - col * 4u : 0u);
   const __amdgpu_buffer_rsrc_t r_dec =
       make_rsrc(w.dec + static_cast<uint32_t>(ob) * kGrWords, valid ? w.dec_bytes - static_cast<uint32_t>(ob) * kGrWords * 4u : 0u);
+  bload_words<4, kSingle>(r_q1, w.v_q1, r.q);
+  bload_words<4, kSingle>(r_dec, w.v_dec, r.g);
+}
+template <bool kCompact, bool kSingle>
+__device__ __forceinline__ void mf_wave_tile_issue(const MfWaveSrc& w, int G, int ob, int lane,
+                                                   MfWaveRegs<kCompact>& r, bool valid = true) {
+  constexpr int kRsLane = MfWaveWords<kCompact>::kRsLane;
+  const uint32_t col = static_cast<uint32_t>(ob) * kTileOut;
+  mf_wave_words_issue<kCompact, kSingle>(w, ob, r, valid);
   const int ncols = valid ? w.rs_cols - static_cast<int>(col) : 0;  // the wavefront's columns to the expert's last
   const __amdgpu_buffer_rsrc_t r_rs = make_rsrc(w.rs + (ncols > 0 ? static_cast<int64_t>(col) * 2 * G : 0),
                                                 ncols > 0 ? static_cast<uint32_t>(ncols) * G * 8u : 0u);
-  bload_words<4, kSingle>(r_q1, w.v_q1, r.q);
-  bload_words<4, kSingle>(r_dec, w.v_dec, r.g);
   bload_words<kRsLane, kSingle>(r_rs, static_cast<uint32_t>(lane * kRsLane) * 4u, r.rs);
 }
 
@@ -1373,6 +1380,222 @@ void grouped_mfma_kernel(MfmaArgs a) {
 }
 
 // ----------------------------------------------------------------------------------------------------
+// Non-expert linears: one matrix over the full input width (thousands of columns, a row-scale group each 128), any
+// batch, up to three of them on one input.  A workgroup takes one 64-output tile, kRows rows and a run of 512-column
+// chunks (blockIdx.y = row tile x slice), stages each chunk as the decode kernel does, and leaves fp32 partial sums
+// [slice][batch][N]; linear_finish_kernel adds the slices in order, then the addend, scale and bias.  Slices are taken
+// until the launch fills the GPU.  The row scales are staged per K tile (the decode kernel's per group would not fit), and
+// whether every K tile of a chunk lies in one group is found on the way: a chunk where one does not takes a scalar loop
+// over its columns instead, so no launch waits for the host to look at g_idx.
+// Q, K and V of 2048 x 2048 at 16 rows: 10.0 us, the finish 3.4 and the bitmaps 9.5, against 504 us of the exact VALU
+// kernel (two launches) and seven host round trips to read g_idx.
+struct LinProj {
+  tris_compact3_payload p;
+  const int32_t* decoded;  // [packed rows / 2][tiles][128]
+  float* part;             // [slices][batch][N]
+  const float* addend;     // [batch][N] or null
+  uint16_t* out;           // [batch][N]
+};
+struct LinArgs {
+  LinProj proj[TRIS_MAX_LINEARS];
+  const uint16_t* x;         // [batch][rank]
+  const uint16_t* in_scale;  // [rank] or null
+  int batch, slices, chunks;
+};
+
+// The exact weight of column k (of the whole matrix) for output n, from memory (chunks with split K tiles).
+__device__ __forceinline__ float lin_weight(const LinProj& a, int k, int n) {
+  const tris_compact3_payload& p = a.p;
+  const int N = p.outfeatures;
+  const int pr = k >> 5, bit = k & 31;
+  const int g = p.g_idx[k];
+  const uint64_t rp = g >= 0 && g < p.num_groups
+                          ? static_cast<uint64_t>(p.row_pack3[static_cast<int64_t>(n) * p.num_groups + g]) : 0ull;
+  const uint64_t cp = static_cast<uint64_t>(p.col_pack3[k]);
+  const uint32_t q1 = static_cast<uint32_t>(p.qweight1[static_cast<int64_t>(pr) * N + n]);
+  const uint32_t cm = static_cast<uint32_t>(p.c_map[pr]);
+  const auto prod = [&](int h) { return hmul_bits(static_cast<uint16_t>(cp >> (16 * h)), static_cast<uint16_t>(rp >> (16 * h))); };
+  const uint16_t neg1 = (q1 >> bit) & 1u ? 0u : 0x8000u;
+  if ((cm >> bit) & 1u) {
+    const int idx = p.qweight2_sparse_prefix[pr] + __popc(cm & ((1u << bit) - 1u));
+    const int row = idx >> 5;
+    const uint32_t q2 = row >= 0 && row < p.qweight2_sparse_rows
+                            ? static_cast<uint32_t>(p.qweight2_sparse[static_cast<int64_t>(row) * N + n]) : 0u;
+    const uint16_t neg2 = (q2 >> (idx & 31)) & 1u ? 0u : 0x8000u;
+    return h2f(hadd_bits(prod(0) ^ neg1, prod(1) ^ neg2));
+  }
+  const uint32_t gw = static_cast<uint32_t>(
+      a.decoded[(static_cast<int64_t>(pr >> 1) * ceil_div(N, kTileOut) + n / kTileOut) * kGrWords + (pr & 1) * kTileOut +
+                n % kTileOut]);
+  return h2f(((gw >> bit) & 1u ? prod(2) : prod(3)) ^ neg1);
+}
+
+template <int kRows, bool kSingle>
+__global__ __launch_bounds__(kMfThreads) __attribute__((amdgpu_waves_per_eu(3, 8))) void linear_mfma_kernel(LinArgs a) {
+  constexpr int kRt = kRows / kMfRows;
+  const LinProj& lp = a.proj[blockIdx.z];
+  const tris_compact3_payload& p = lp.p;
+  const int N = p.outfeatures, rank = p.rank, G = p.num_groups;
+  const int ob = static_cast<int>(blockIdx.x);
+  if (ob * kTileOut >= N) return;  // uniform, before any barrier
+  const int sl = static_cast<int>(blockIdx.y) % a.slices;
+  const int row0 = static_cast<int>(blockIdx.y) / a.slices * kRows;
+  const int rc = a.batch - row0 < kRows ? a.batch - row0 : kRows;
+  const int c_lo = static_cast<int>(static_cast<int64_t>(sl) * a.chunks / a.slices);
+  const int c_hi = static_cast<int>(static_cast<int64_t>(sl + 1) * a.chunks / a.slices);
+  __shared__ __attribute__((aligned(16))) uint16_t xs[kRows * mf_xstride(false)];
+  __shared__ __attribute__((aligned(16))) uint16_t cds[2 * kMfChunk];
+  __shared__ __attribute__((aligned(16))) uint2 goff[kMfTiles];
+  __shared__ __attribute__((aligned(16))) uint32_t salw[kMfChunk + 4];
+  __shared__ __attribute__((aligned(16))) uint16_t salxo[kMfChunk + 8];
+  __shared__ __attribute__((aligned(16))) uint32_t salcp[kMfChunk + 4];
+  __shared__ __attribute__((aligned(16))) uint32_t wbuf[kMfWaves][MfWaveWords<false>::kAlloc];
+  MfChunk ch{};
+  ch.xs = xs;
+  ch.cds = cds;
+  ch.goff = goff;
+  ch.sal_w = salw;
+  ch.sal_xo = salxo;
+  ch.sal_cp = salcp;
+  const int utid = static_cast<int>(threadIdx.x);
+  const int wave = __builtin_amdgcn_readfirstlane(utid / kWave);
+  const int lane = utid % kWave;
+  const int i16 = lane % 16, kg = lane / 16;
+  uint32_t* const wb = wbuf[wave];
+  MfmaProj pa{};
+  pa.decoded = lp.decoded;
+  pa.p = p;
+  const uint32_t roff = lane < rc ? static_cast<uint32_t>(lane) * static_cast<uint32_t>(rank) * 2u : kMfOob;
+  const __amdgpu_buffer_rsrc_t r_x =
+      make_rsrc(a.x + static_cast<int64_t>(row0) * rank, static_cast<uint32_t>(rc) * rank * 2u);
+  const __amdgpu_buffer_rsrc_t r_sc = make_rsrc(a.in_scale, a.in_scale != nullptr ? static_cast<uint32_t>(rank) * 2u : 0u);
+  const __amdgpu_buffer_rsrc_t r_g = make_rsrc(p.g_idx, static_cast<uint32_t>(rank) * 4u);
+  const int n0w = ob * kTileOut + kMfWCols * wave;  // the wavefront's first column
+  const __amdgpu_buffer_rsrc_t r_rs = make_rsrc(p.row_pack3 + (n0w < N ? static_cast<int64_t>(n0w) * G : 0),
+                                                n0w < N ? static_cast<uint32_t>(N - n0w) * G * 8u : 0u);
+  const uint32_t* q2 = reinterpret_cast<const uint32_t*>(p.qweight2_sparse);
+  const uint16_t* xr[kRt];
+#pragma unroll
+  for (int m = 0; m < kRt; ++m) xr[m] = xs + (16 * m + i16 < rc ? 16 * m + i16 : 0) * mf_xstride(false);
+  const int n[1] = {n0w + i16};
+  f32x4 acc[1][kRt];
+  float scalar[kRows / kMfWaves];  // the scalar loop's sums: rows wave + 4 i, column ob * 64 + lane
+  bool any_split = false;
+#pragma unroll
+  for (int m = 0; m < kRt; ++m) acc[0][m] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+  for (int i = 0; i < kRows / kMfWaves; ++i) scalar[i] = 0.0f;
+  for (int c = c_lo; c < c_hi; ++c) {
+    const int kc = c * kMfChunk;
+    if (c > c_lo) __syncthreads();  // the previous chunk's readers are done
+    MfColRegs cols;
+    MfRowRegs<kRows, false> rows;
+    MfWaveRegs<false> wr;
+    int gt[2];  // the groups of K tiles lane / 16 and lane / 16 + 4
+#pragma unroll
+    for (int h = 0; h < 2; ++h) gt[h] = static_cast<int>(bload32(r_g, static_cast<uint32_t>(kc + (kg + 4 * h) * kTileK) * 4u, 0u));
+    const uint64_t gp = bload64(r_g, static_cast<uint32_t>(kc + 2 * utid) * 4u, 0u);  // of the thread's two columns
+    mf_cols_issue<false>(pa, 0, kc, utid, cols);
+    mf_rows_issue<kRows, false>(r_x, rank, kc, wave, lane, roff, 0, rows);
+    mf_wave_words_issue<false, kSingle>(mf_wave_src<false>(pa, 0, 0, kc, wave, lane), ob, wr, true);
+    uint64_t rp[2];
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      rp[h] = bload64(r_rs, gt[h] >= 0 && gt[h] < G ? static_cast<uint32_t>(i16 * G + gt[h]) * 8u : kMfOob, 0u);
+    }
+    const int first = __shfl(static_cast<int>(gp), lane & 32);  // the group of the K tile's first column
+    const bool split = kc + 2 * utid < rank && (static_cast<int>(gp) != first || static_cast<int>(gp >> 32) != first);
+    if (a.in_scale != nullptr) {
+      const uint4 sc = bload128(r_sc, static_cast<uint32_t>(kc + lane * 8) * 2u, 0u);
+      const uint32_t sv[4] = {sc.x, sc.y, sc.z, sc.w};
+#pragma unroll
+      for (int h = 0; h < MfRowRegs<kRows, false>::kRuns; ++h) {
+        uint32_t v[4] = {rows.xv[h].x, rows.xv[h].y, rows.xv[h].z, rows.xv[h].w};
+#pragma unroll
+        for (int i = 0; i < 4; ++i) v[i] = f16x2_as_u32(u32_as_f16x2(v[i]) * u32_as_f16x2(sv[i]));
+        rows.xv[h] = make_uint4(v[0], v[1], v[2], v[3]);
+      }
+    }
+    mf_cols_write<false, true>(pa, rc, kc, utid, ch, cols, kMfChunk);
+    mf_rows_write<kRows, false>(rows, rc, wave, lane, xs);
+    const MfChunkMeta cm = mf_chunk_meta(cols, kMfChunk);
+    {
+      const int row = lane / 4;
+      uint32_t* dst = wb + kMfWw + ((row >> 1) * kMfWCols + 4 * (lane % 4)) * 4 + (row & 1) * 2;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) *reinterpret_cast<uint2*>(dst + 4 * i) = make_uint2(wr.q[i], wr.g[i]);
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        *reinterpret_cast<uint2*>(wb + MfWaveWords<false>::kRs + (i16 * kMfMaxGroups + kg + 4 * h) * 2) =
+            make_uint2(static_cast<uint32_t>(rp[h]), static_cast<uint32_t>(rp[h] >> 32));
+      }
+    }
+    if (!__syncthreads_or(split ? 1 : 0)) {
+      uint32_t q2w[1][2];
+      mf_q2_issue(q2, p.qweight2_sparse_rows, N, n[0], cm, q2w[0]);
+      mf_compute<1, kRt, false>(q2, p.qweight2_sparse_rows, N, rank, kMfMaxGroups, kc, n, xr, lane, ch, cm, wb, q2w, acc);
+    } else {  // uniform over the workgroup
+      any_split = true;
+      const int ns = ob * kTileOut + lane;
+      const int kn = rank - kc < kMfChunk ? rank - kc : kMfChunk;
+      for (int k = 0; k < kn && ns < N; ++k) {
+        const float w = lin_weight(lp, kc + k, ns);
+        const int pos = (k & ~31) + mf_perm32(k & 31);
+#pragma unroll
+        for (int i = 0; i < kRows / kMfWaves; ++i) {
+          const int r = wave + kMfWaves * i;
+          if (r < rc) scalar[i] = fmaf(h2f(xs[r * mf_xstride(false) + pos]), w, scalar[i]);
+        }
+      }
+    }
+  }
+  if (any_split) {  // uniform: the scalar sums join the accumulators through LDS (the staged rows are done with)
+    static_assert(kRows * kTileOut * 4 <= sizeof(xs), "the scalar sums fit the staged rows");
+    float* const ex = reinterpret_cast<float*>(xs);
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < kRows / kMfWaves; ++i) ex[(wave + kMfWaves * i) * kTileOut + lane] = scalar[i];
+    __syncthreads();
+#pragma unroll
+    for (int m = 0; m < kRt; ++m) {
+#pragma unroll
+      for (int v = 0; v < 4; ++v) acc[0][m][v] += ex[(16 * m + 4 * kg + v) * kTileOut + kMfWCols * wave + i16];
+    }
+  }
+  float* const part = lp.part + (static_cast<int64_t>(sl) * a.batch + row0) * N;
+#pragma unroll
+  for (int m = 0; m < kRt; ++m) {
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+      const int r = 16 * m + 4 * kg + v;
+      if (r < rc && n[0] < N) part[static_cast<int64_t>(r) * N + n[0]] = acc[0][m][v];
+    }
+  }
+}
+
+// out[b][n] = fp16((sum of the slices, in order, + addend) * scale + bias), as the exact kernel ends.
+__global__ __launch_bounds__(256) void linear_finish_kernel(LinArgs a) {
+  const LinProj& lp = a.proj[blockIdx.z];
+  const tris_compact3_payload& p = lp.p;
+  const int N = p.outfeatures;
+  const int n = static_cast<int>(blockIdx.x) * 256 + static_cast<int>(threadIdx.x);
+  if (n >= N) return;
+  const float scale = p.has_output_scale ? h2f(p.output_scale[n]) : 1.0f;
+  const float bias = p.has_bias ? h2f(p.bias[n]) : 0.0f;
+  for (int b = static_cast<int>(blockIdx.y); b < a.batch; b += static_cast<int>(gridDim.y)) {
+    const int64_t at = static_cast<int64_t>(b) * N + n;
+    const int64_t step = static_cast<int64_t>(a.batch) * N;
+    float v = 0.0f;
+#pragma unroll 4
+    for (int s = 0; s < a.slices; ++s) v += lp.part[s * step + at];
+    if (lp.addend != nullptr) v += lp.addend[at];
+    if (p.has_output_scale) v = v * scale;
+    if (p.has_bias) v = v + bias;
+    lp.out[at] = f2h_bits(v);
+  }
+}
+
+// ----------------------------------------------------------------------------------------------------
 // Weight-stationary variant for long segments (prefill).  A work item is (active segment, kSub 64-column
 // output tiles): the unit copies the tiles' weight words, builds the exact B operands of its columns over the
 // whole K (rank <= 512: 16 packed rows, 4 registers each per tile, plus at most two 32-column salient windows)
@@ -2034,6 +2257,126 @@ int launch_grouped_mfma(const uint16_t* hidden_a, const uint16_t* hidden_b, int 
   return check_launch(who);
 }
 
+// Slices of a linear's K: chunks are split until one matrix's launch has about three workgroups a CU (whatever the number
+// of matrices, so that each gives the same bits alone and beside others of its width).
+static int lin_slices(int batch, int rank, int max_n) {
+  const int chunks = ceil_div(rank, kMfChunk);
+  const int64_t tiles = static_cast<int64_t>(ceil_div(max_n, kTileOut)) * ceil_div(batch, batch <= kMfRows ? kMfRows : 32);
+  const int64_t want = tiles > 0 ? (3 * kMfCus + tiles - 1) / tiles : 1;
+  return static_cast<int>(want < chunks ? want : chunks);
+}
+
+static int64_t lin_decoded_words(int rank, int n) {
+  return static_cast<int64_t>((rank / 32 + 1) / 2) * ceil_div(n, kTileOut) * kGrWords;
+}
+
+int64_t linear_mfma_workspace(int batch, int rank, const int32_t* outfeatures, int count) {
+  int max_n = 0;
+  int64_t words = 0, sums = 0;
+  for (int i = 0; i < count; ++i) {
+    max_n = outfeatures[i] > max_n ? outfeatures[i] : max_n;
+    words += lin_decoded_words(rank, outfeatures[i]);
+    sums += static_cast<int64_t>(batch) * outfeatures[i];
+  }
+  return 4 * (words + sums * lin_slices(batch, rank, max_n));
+}
+
+// The matrix sizes linear_mfma_kernel takes: whole 64-column K tiles, every 32-bit buffer offset below 2 GiB.
+static bool lin_fits(const tris_compact3_payload* p) {
+  const int64_t limit = int64_t{1} << 31;
+  const int64_t n = p->outfeatures;
+  return p->rank > 0 && p->rank % kTileK == 0 && n > 0 && p->num_groups > 0 &&
+         static_cast<int64_t>(p->rank / 32) * n * 4 < limit && int64_t{p->qweight2_sparse_rows} * n * 4 < limit &&
+         n * p->num_groups * 8 < limit && lin_decoded_words(p->rank, p->outfeatures) * 4 < limit &&
+         int64_t{32} * p->rank * 2 < limit && int64_t{p->rank} * 8 < limit;
+}
+
+// Entry 0 of an expert list: the matrix itself.
+__device__ int32_t lin_expert0[4];
+
+int launch_linear_mfma(const uint16_t* input, int batch, const tris_compact3_payload* payloads, int count,
+                       const uint16_t* input_scale, const float* addend, uint16_t* const* outs, void* workspace,
+                       int64_t workspace_bytes, void* stream, const char* who) {
+  TRIS_REQUIRE(batch >= 0 && count >= 1 && count <= TRIS_MAX_LINEARS && payloads && outs, "%s: bad arguments", who);
+  LinArgs args{};
+  int max_n = 0;
+  int32_t widths[TRIS_MAX_LINEARS];
+  bool wide = true;
+  for (int i = 0; i < count; ++i) {
+    const tris_compact3_payload* p = payloads + i;
+    int rc = check_payload(p, true, who);
+    if (rc) return rc;
+    TRIS_REQUIRE(p->num_experts == 1 && p->q_gmap_gr_offsets != nullptr,
+                 "%s: a non-expert payload holds one block-GR matrix", who);
+    TRIS_REQUIRE(p->rank == payloads[0].rank, "%s: the matrices' ranks differ", who);
+    TRIS_REQUIRE(lin_fits(p), "%s: rank must be a multiple of %d and the tensors below 2 GiB", who, kTileK);
+    widths[i] = p->outfeatures;
+    max_n = p->outfeatures > max_n ? p->outfeatures : max_n;
+  }
+  if (batch == 0) return TRIS_OK;
+  TRIS_REQUIRE(input && workspace, "%s: null pointer", who);
+  TRIS_REQUIRE(reinterpret_cast<uintptr_t>(input) % 16 == 0 && reinterpret_cast<uintptr_t>(workspace) % 16 == 0,
+               "%s: input and workspace must be 16-byte aligned", who);
+  const int rank = payloads[0].rank;
+  TRIS_REQUIRE(workspace_bytes >= linear_mfma_workspace(batch, rank, widths, count), "%s: workspace too small", who);
+  void* ids = nullptr;
+  TRIS_REQUIRE(hipGetSymbolAddress(&ids, HIP_SYMBOL(lin_expert0)) == hipSuccess, "%s: no expert list", who);
+  args.x = input;
+  args.in_scale = input_scale;
+  args.batch = batch;
+  args.chunks = ceil_div(rank, kMfChunk);
+  args.slices = lin_slices(batch, rank, max_n);
+  int32_t* words = static_cast<int32_t*>(workspace);
+  tris_gr_predecode_job jobs[TRIS_MAX_LINEARS];
+  for (int i = 0; i < count; ++i) {
+    const tris_compact3_payload& p = payloads[i];
+    TRIS_REQUIRE(outs[i], "%s: null pointer", who);
+    args.proj[i].p = p;
+    args.proj[i].decoded = words;
+    args.proj[i].out = outs[i];
+    args.proj[i].addend = i == 0 ? addend : nullptr;
+    jobs[i] = tris_gr_predecode_job{words, p.q_gmap_gr_words, p.q_gmap_gr_offsets, p.q_gmap_gr_meta, 1,
+                                    p.gr_words_stride, rank / 32, p.outfeatures};
+    words += lin_decoded_words(rank, p.outfeatures);
+    const MfmaProj probe{nullptr, nullptr, args.proj[i].decoded, p, nullptr, 0, nullptr, 0};
+    wide = wide && mf_wide(probe);
+  }
+  float* sums = reinterpret_cast<float*>(words);
+  for (int i = 0; i < count; ++i) {
+    args.proj[i].part = sums;
+    sums += static_cast<int64_t>(args.slices) * batch * widths[i];
+  }
+  int rc = tris_grouped_block_gr_predecode_multi(jobs, count, static_cast<const int32_t*>(ids), 1, stream);
+  if (rc) return rc;
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  const int rows = batch <= kMfRows ? kMfRows : 32;
+  const int64_t y = static_cast<int64_t>(ceil_div(batch, rows)) * args.slices;
+  TRIS_REQUIRE(y < (int64_t{1} << 31), "%s: too many row tiles", who);
+  // (grid.y is limited to 65535: longer batches go in several launches of whole row tiles)
+  const int per = 65535 / args.slices * rows;
+  for (int b0 = 0; b0 < batch; b0 += per) {
+    LinArgs part = args;
+    part.x = input + static_cast<int64_t>(b0) * rank;
+    part.batch = batch - b0 < per ? batch - b0 : per;
+    for (int i = 0; i < count; ++i) {
+      part.proj[i].part = args.proj[i].part + static_cast<int64_t>(args.slices) * b0 * widths[i];
+      part.proj[i].out = args.proj[i].out + static_cast<int64_t>(b0) * widths[i];
+      if (args.proj[i].addend != nullptr) part.proj[i].addend = args.proj[i].addend + static_cast<int64_t>(b0) * widths[i];
+    }
+    const dim3 grid(ceil_div(max_n, kTileOut), ceil_div(part.batch, rows) * args.slices, count);
+    if (rows == kMfRows) {
+      if (wide) hipLaunchKernelGGL((linear_mfma_kernel<kMfRows, false>), grid, dim3(kMfThreads), 0, s, part);
+      else hipLaunchKernelGGL((linear_mfma_kernel<kMfRows, true>), grid, dim3(kMfThreads), 0, s, part);
+    } else {
+      if (wide) hipLaunchKernelGGL((linear_mfma_kernel<32, false>), grid, dim3(kMfThreads), 0, s, part);
+      else hipLaunchKernelGGL((linear_mfma_kernel<32, true>), grid, dim3(kMfThreads), 0, s, part);
+    }
+    const int ty = part.batch < 4096 ? part.batch : 4096;
+    hipLaunchKernelGGL(linear_finish_kernel, dim3(ceil_div(max_n, 256), ty, count), dim3(256), 0, s, part);
+  }
+  return check_launch(who);
+}
+
 // True when the MFMA kernel can run this payload: uniform 64-column groups (so
 // a 64-column K tile has one row scale) and a rank that is a whole number of
 // 64-column tiles, with 16-byte aligned activations (8-column loads).
@@ -2052,3 +2395,17 @@ bool grouped_mfma_supported(const tris_compact3_payload* p, const uint16_t* hidd
 }
 
 }  // namespace tris
+
+extern "C" int64_t tris_compact3_linears_workspace_bytes(int32_t batch, int32_t rank, const int32_t* outfeatures,
+                                                         int32_t count) {
+  if (batch < 0 || rank <= 0 || count < 1 || count > TRIS_MAX_LINEARS || outfeatures == nullptr) return 0;
+  return tris::linear_mfma_workspace(batch, rank, outfeatures, count);
+}
+
+extern "C" int tris_compact3_linears_forward(const uint16_t* input, int32_t batch, const tris_compact3_payload* payloads,
+                                             int32_t count, const uint16_t* input_scale, const float* addend,
+                                             uint16_t* const* outputs, void* workspace, int64_t workspace_bytes,
+                                             void* stream) {
+  return tris::launch_linear_mfma(input, batch, payloads, count, input_scale, addend, outputs, workspace,
+                                  workspace_bytes, stream, "tris_compact3_linears_forward");
+}

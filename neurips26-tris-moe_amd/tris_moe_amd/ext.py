@@ -1657,12 +1657,45 @@ def _linear_struct(rank, qweight1, qweight2_sparse, qweight2_sparse_prefix, q_gm
         raise RuntimeError(f"{who}: sparse split-bitmap payloads are not accepted; convert them to block-GR at load "
                            "(checkpoint.sparse_gmap_to_dense + gr_encode, as GroupedCheckpoint does)")
     one = lambda t: t.unsqueeze(0) if t is not None else None
+    return make_payload_struct(rank, one(qweight1), one(qweight2_sparse), one(qweight2_sparse_prefix),
+                               one(q_gmap_gr_words), one(q_gmap_gr_offsets), one(q_gmap_gr_meta), one(c_map),
+                               g_idx.reshape(1, -1), one(col_pack3), one(row_pack3),
+                               one(output_scale) if has_output_scale else output_scale, has_output_scale,
+                               one(bias) if has_bias else bias, has_bias, False, device, True, who)
+
+
+def _set_uniform_k64(st, g_idx):
+    """Whether the matrix's 64-column tiles each lie in one group, for the exact kernel (reads g_idx on the host)."""
+    rank = int(st.rank)
     g2 = g_idx.reshape(1, -1)
     uniform = bool(torch.equal(g2[:, (torch.arange(rank, device=g2.device) // 64) * 64], g2)) if rank else True
-    return make_payload_struct(rank, one(qweight1), one(qweight2_sparse), one(qweight2_sparse_prefix),
-                               one(q_gmap_gr_words), one(q_gmap_gr_offsets), one(q_gmap_gr_meta), one(c_map), g2,
-                               one(col_pack3), one(row_pack3), one(output_scale) if has_output_scale else output_scale,
-                               has_output_scale, one(bias) if has_bias else bias, has_bias, uniform, device, True, who)
+    st.use_uniform_k64_groups = 1 if uniform else 0
+
+
+def _linears_ok(x: torch.Tensor, structs) -> bool:
+    """tris_compact3_linears_forward takes these matrices of x's width: whole 64-column K tiles, 16-byte aligned rows,
+    tensors below 2 GiB (any g_idx; it does not read it on the host)."""
+    rank = int(x.size(1))
+    if rank % 64 or x.data_ptr() % 16 or rank * 64 >= 1 << 31:
+        return False
+    for st in structs:
+        n = int(st.outfeatures)
+        if max(rank // 8 * n, 4 * int(st.qweight2_sparse_rows) * n, 8 * int(st.num_groups) * n,
+               rank // 64 * -(-n // 64) * 512) >= 1 << 31 or int(st.num_groups) < 1:
+            return False
+    return True
+
+
+def _linears_forward(x: torch.Tensor, structs, outs, scale, addend, who: str):
+    """The structs' linears of x in one predecode, one GEMM and one finishing launch (outs: fp16 [batch, N] each)."""
+    lib = _lib.load()
+    count, batch = len(structs), int(x.size(0))
+    widths = (ctypes.c_int32 * count)(*[int(st.outfeatures) for st in structs])
+    ws = torch.empty(max(int(lib.tris_compact3_linears_workspace_bytes(batch, int(x.size(1)), widths, count)), 256),
+                     dtype=torch.uint8, device=x.device)
+    _lib.check(lib.tris_compact3_linears_forward(
+        _ptr(x), batch, (TrisPayload * count)(*structs), count, _ptr(scale), _ptr(addend),
+        (ctypes.c_void_p * count)(*[o.data_ptr() for o in outs]), _ptr(ws), int(ws.numel()), _stream(x)), who)
 
 
 def _ns_linear_addend(x16, ns_c1_qweight, ns_c1_qzeros, ns_c1_scales, ns_c1_g_idx, ns_c2_qweight, ns_c2_qzeros,
@@ -1698,7 +1731,7 @@ def compact3_linear_forward(input, qweight1, qweight2_sparse, qweight2_sparse_pr
     [batch, out] = fp16((x' . W^T + ns) * output_scale + bias) for one non-expert compact3 matrix, x' the
     input times input_scale per column (fp16), ns the matrix-mode null-space term in fp32.  Block-GR payloads;
     split_k_slices, request_prefill_tensor_core and use_uniform_k64_groups are the reference's launch hints
-    (one exact kernel serves every shape here)."""
+    (not needed here: the matrix-core path finds uniform tiles on the device, and the exact kernel takes the rest)."""
     who = "compact3_linear_forward"
     _check_cuda("input", input, torch.float16, 2)
     dev = input.device
@@ -1710,9 +1743,9 @@ def compact3_linear_forward(input, qweight1, qweight2_sparse, qweight2_sparse_pr
                         q_gmap_gr_meta, c_map, g_idx, col_pack3, row_pack3, output_scale, has_output_scale, bias,
                         has_bias, dev, who)
     batch = int(input.size(0))
-    out = torch.zeros((batch, outfeatures), dtype=torch.float16, device=dev)
     if batch == 0 or rank == 0 or outfeatures == 0:
-        return out
+        return torch.zeros((batch, outfeatures), dtype=torch.float16, device=dev)
+    out = torch.empty((batch, outfeatures), dtype=torch.float16, device=dev)
     scale = None
     if has_input_scale:
         _check_cuda("input_scale", input_scale, torch.float16, 1, dev)
@@ -1723,6 +1756,10 @@ def compact3_linear_forward(input, qweight1, qweight2_sparse, qweight2_sparse_pr
     if has_ns_matrix:
         addend = _ns_linear_addend(input, ns_c1_qweight, ns_c1_qzeros, ns_c1_scales, ns_c1_g_idx, ns_c2_qweight,
                                    ns_c2_qzeros, ns_c2_scales, ns_c2_g_idx, outfeatures)
+    if _linears_ok(input, (st,)) and (scale is None or scale.data_ptr() % 16 == 0):
+        _linears_forward(input, (st,), (out,), scale, addend, who)
+        return out
+    _set_uniform_k64(st, g_idx)
     _lib.check(_lib.load().tris_compact3_linear_forward(_ptr(input), batch, ctypes.byref(st), _ptr(scale),
                                                         _ptr(addend), _ptr(out), _stream(input)), who)
     return out
@@ -1750,9 +1787,14 @@ def compact3_dual_linear_forward(input, a_qweight1, a_qweight2_sparse, a_qweight
                         b_gmap_gr_offsets, b_gmap_gr_meta, b_c_map, b_g_idx, b_col_pack3, b_row_pack3, None, False,
                         None, False, dev, who)
     batch = int(input.size(0))
-    out = torch.zeros((2, batch, outfeatures), dtype=torch.float16, device=dev)
     if batch == 0 or rank == 0 or outfeatures == 0:
+        return torch.zeros((2, batch, outfeatures), dtype=torch.float16, device=dev)
+    out = torch.empty((2, batch, outfeatures), dtype=torch.float16, device=dev)
+    if _linears_ok(input, (sa, sb)):
+        _linears_forward(input, (sa, sb), (out[0], out[1]), None, None, who)
         return out
+    _set_uniform_k64(sa, a_g_idx)
+    _set_uniform_k64(sb, b_g_idx)
     _lib.check(_lib.load().tris_compact3_dual_linear_forward(_ptr(input), batch, ctypes.byref(sa), ctypes.byref(sb),
                                                              _ptr(out[0]), _ptr(out[1]), _stream(input)), who)
     return out
@@ -1767,7 +1809,8 @@ def compact3_qkv_linear_forward(input, q_qweight1, q_qweight2_sparse, q_qweight2
                                 split_k_slices: int = 1, use_uniform_k64_groups: bool = False) -> torch.Tensor:
     """The extension's compact3_qkv_linear_forward (TriSMoE_cuda.cpp:564-640, kernel.cu:11457-11740): the
     attention Q / K / V projections of one input, each fp16((x . W^T) + bias), stacked fp16 [3, batch, out]
-    (equal output widths).  Q and K share one launch, V takes a second."""
+    (equal output widths), in one launch on the matrix cores (_linears_forward); outside its sizes Q and K share a
+    launch of the exact kernel and V takes a second."""
     who = "compact3_qkv_linear_forward"
     _check_cuda("input", input, torch.float16, 2)
     dev = input.device
@@ -1787,9 +1830,14 @@ def compact3_qkv_linear_forward(input, q_qweight1, q_qweight2_sparse, q_qweight2
         structs.append(_linear_struct(rank, qw1, qw2, qw2p, grw, gro, grm, cmap, gidx, colp, rowp, None, False, b,
                                       has_bias, dev, who))
     batch = int(input.size(0))
-    out = torch.zeros((3, batch, outfeatures), dtype=torch.float16, device=dev)
     if batch == 0 or rank == 0 or outfeatures == 0:
+        return torch.zeros((3, batch, outfeatures), dtype=torch.float16, device=dev)
+    out = torch.empty((3, batch, outfeatures), dtype=torch.float16, device=dev)
+    if _linears_ok(input, structs):
+        _linears_forward(input, structs, (out[0], out[1], out[2]), None, None, who)
         return out
+    for st, gidx in zip(structs, (q_g_idx, k_g_idx, v_g_idx)):
+        _set_uniform_k64(st, gidx)
     lib = _lib.load()
     _lib.check(lib.tris_compact3_dual_linear_forward(_ptr(input), batch, ctypes.byref(structs[0]),
                                                      ctypes.byref(structs[1]), _ptr(out[0]), _ptr(out[1]),

@@ -864,11 +864,6 @@ class Compact3Linear(nn.Module):
                 setattr(self, key, {k: fn(v) for k, v in d.items()})
         return self
 
-    def _compact3_k64_groups_uniform(self) -> bool:
-        g = self.g_idx.reshape(1, -1)
-        rank = int(g.size(1))
-        return bool(torch.equal(g[:, (torch.arange(rank, device=g.device) // 64) * 64], g)) if rank else True
-
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         shape = x.shape[:-1] + (self.outfeatures,)
         x2 = x.reshape(-1, self.infeatures).to(torch.float16).contiguous()
@@ -883,8 +878,7 @@ class Compact3Linear(nn.Module):
             self.bias if self.bias is not None else empty,
             self.input_scale is not None, self.output_scale is not None, self.bias is not None,
             *[c1.get(k, empty) for k in ("qweight", "qzeros", "scales", "g_idx")],
-            *[c2.get(k, empty) for k in ("qweight", "qzeros", "scales", "g_idx")], ns, 1, False,
-            self._compact3_k64_groups_uniform())
+            *[c2.get(k, empty) for k in ("qweight", "qzeros", "scales", "g_idx")], ns, 1, False, False)
         return y.reshape(shape)
 
 
@@ -912,8 +906,7 @@ def run_compact3_qkv_block_gr_forward(q_proj, k_proj, v_proj, hidden_states: tor
     args = []
     for m in (q_proj, k_proj, v_proj):
         args += [getattr(m, key) for key in COMPACT3_MODULE_KEYS] + [m.bias if m.bias is not None else empty]
-    fused = ext.compact3_qkv_linear_forward(x, *args, 1, all(m._compact3_k64_groups_uniform()
-                                                            for m in (q_proj, k_proj, v_proj)))
+    fused = ext.compact3_qkv_linear_forward(x, *args)
     return tuple(fused[i].reshape(shape) for i in range(3))
 
 
@@ -929,9 +922,7 @@ def run_compact3_shared_expert_gate_up_forward(gate_proj, up_proj, hidden_states
     shape = hidden_states.shape[:-1] + (n,)
     x = hidden_states.reshape(-1, hidden_states.shape[-1]).contiguous()
     fused = ext.compact3_dual_linear_forward(x, *[getattr(gate_proj, k) for k in COMPACT3_MODULE_KEYS],
-                                             *[getattr(up_proj, k) for k in COMPACT3_MODULE_KEYS], 1,
-                                             gate_proj._compact3_k64_groups_uniform()
-                                             and up_proj._compact3_k64_groups_uniform())
+                                             *[getattr(up_proj, k) for k in COMPACT3_MODULE_KEYS])
     return fused[0].reshape(shape), fused[1].reshape(shape)
 
 

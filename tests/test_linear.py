@@ -166,3 +166,37 @@ def test_module_and_fused_runners(tris, oracle_mod, cuda):
     g, u = ql.run_compact3_shared_expert_gate_up_forward(*nobias, x)
     assert torch.equal(g, nobias[0](x)) and torch.equal(u, nobias[1](x))
     assert ql.run_compact3_qkv_block_gr_forward(full, plain[1], plain[2], x) is None
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n,k,batch,groups", [
+    (64, 64, 1, "uniform"),         # the smallest matrix
+    (130, 1152, 16, "uniform"),     # columns no multiple of 4; a last chunk of two K tiles
+    (192, 1024, 17, "uniform"),     # 32-row tiles, one row past the 16-row ones
+    (64, 2048, 70, "uniform"),      # more than eight groups; three row tiles, the last ragged
+    (136, 640, 33, "split"),        # groups changing inside a K tile of the second chunk only
+    (68, 192, 5, "shuffled"),       # a group per column
+    (96, 96, 3, "uniform"),         # rank no multiple of 64: the exact kernel
+])
+def test_linear_matrix_core_shapes(tris, oracle_mod, cuda, n, k, batch, groups):
+    """The linears' GEMM at the edges of its tiles, chunks and slices and with g_idx it has to walk column by column,
+    with an input scale, output scale and bias, against the oracle."""
+    from test_gpu_parity import assert_close, note
+
+    note(f"compact3 linear n={n} k={k} batch={batch} groups={groups}")
+    ext = tris["ext"]
+    rng = np.random.default_rng(n + k)
+    gidx = np.arange(k) // 128
+    if groups == "shuffled":
+        gidx = rng.permutation(gidx)
+    elif groups == "split":
+        gidx[600:610] = 0
+    proj = synthetic.make_projection(rng, 1, n, k, 0.15, rng.random(k).astype(np.float32) + 0.5, ext.gr_encode,
+                                     g_idx=gidx.astype(np.int32))
+    m = {key: np.ascontiguousarray(proj[key][0]) for key in MODULE_KEYS}
+    x = (rng.standard_normal((batch, k)) * 1.5).astype(np.float16)
+    s_in, s_out = (rng.random(k) + 0.5).astype(np.float16), (rng.random(n) * 2 + 0.25).astype(np.float16)
+    bias = rng.standard_normal(n).astype(np.float16)
+    t = lambda a: torch.from_numpy(np.ascontiguousarray(a)).to(cuda)
+    got = _linear(ext, t(x), _dev(m, cuda), t(s_in), t(s_out), t(bias))
+    assert_close(got.cpu().numpy(), oracle_mod.compact3_linear(x, m, s_in, s_out, bias), f"linear n={n} k={k}")
