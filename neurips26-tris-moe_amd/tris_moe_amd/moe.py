@@ -502,8 +502,9 @@ def _predecoded_moe_forward(x16, w16, route, payloads, backbones, num_experts, R
                            f"above {FUSED_SWIGLU_MAX_ROWS} routed rows")
     bufs = predecoded if predecoded is not None else {
         name: _predecode_buffer(p, slots, dev) for name, p in (("gate", pg), ("up", pu), ("down", pd))}
-    main = torch.cuda.current_stream(dev)
-    side = _side_stream(dev)
+    # the caller's stream, read only where another one joins it
+    beside = shared_fold is not None or any(v is not None for v in ns.values())
+    main = torch.cuda.current_stream(dev) if beside else None
     n_mlp = int(pg["qweight1"].size(2))
     comp_g = comp_u = None
     ns_side = None
@@ -602,6 +603,7 @@ def _predecoded_moe_forward(x16, w16, route, payloads, backbones, num_experts, R
         # the down compensation beside the down backbone and GEMM; its buffer belongs to the caller's stream,
         # which waits for the side stream before reading or freeing it
         comp_d = torch.empty((R, n_out), dtype=torch.float16, device=dev)
+        side = _side_stream(dev)
         side.wait_stream(main)
         with torch.cuda.stream(side):
             ext.ns_compensation_apply_(comp_d, mlp, eid, seg, ns["down"], accumulate=False)
