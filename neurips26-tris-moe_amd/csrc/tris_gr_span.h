@@ -12,17 +12,24 @@
 // s remainder bits still to read.  For k in {1, 2} two tables describe one
 // byte of stream:
 //   next[k][byte]       four bytes, byte s = the state after the byte from
-//                       entry state s (identity above k).  A map of states in
-//                       this form is a v_perm_b32 selector: composing maps,
-//                       and stepping a state held in all four bytes, is one
-//                       v_perm_b32;
-//   entry[k][s][byte]   64 bits: the low word holds the completed ones' bit
-//                       mask (bit i = a one at F(byte start) - 1 + i; a
-//                       codeword entered mid-remainder whose last bits are
-//                       zero ends at bit 0); the high word holds the F advance
-//                       (bits 0..6) and the number of completed codewords
-//                       (bits 12..15), so a lane's sum of high words holds its
-//                       advance and count sums.
+//                       entry state s (bits 0, 1; identity above k) and the
+//                       byte's F advance from it (bits 2..7, at most 32).  The
+//                       state bits of a map are a v_perm_b32 selector:
+//                       composing maps, and stepping a state held in all four
+//                       bytes, is one v_perm_b32 and a mask;
+//   entry[k][s][byte]   the completed ones' bit mask in bits 0..24 (bit i = a
+//                       one at F(byte start) - 1 + i; a codeword entered
+//                       mid-remainder whose last bits are zero ends at bit 0)
+//                       and the F advance in bits 26..31.
+// The table reads and the emission's ORs hit random LDS banks: at the Mixtral
+// shape (8 experts, 32768 blocks) LDS was busy 61% of the kernel, two thirds
+// of it conflicts, when the walk read 64-bit entries twice.  The advances ride
+// in the words that A reads, an entry is 32 bits and read once, an OR whose
+// word is empty is skipped and the ones are counted in the finished bitmap:
+// LDS busy 44%, 22.3 -> 20.4 us (Mixtral, 16 tokens), 15.9 -> 14.0 us (one
+// token), 24.9 -> 23.2 us (A3B, 32 tokens).  What is left is the latency of
+// the header, words and table chain: fewer VALU (17 instead of 23 a byte) or
+// an even number of items a wavefront changed nothing.
 // Each lane of the block's group of S lanes:
 //   A. reads next[] for every byte of its span (loads that do not wait on
 //      each other) and composes them into its exit-state map;
@@ -69,8 +76,10 @@ namespace tris {
 
 constexpr int kGrEntryStates = 2 + 3;                         // k = 1, 2; s in [0, k]
 constexpr int kGrEntries = kGrEntryStates * 256 + 1;             // + one all-zero entry
-constexpr uint32_t kGrZeroEntryOffset = kGrEntryStates * 256 * 8;  // byte offset of the zero entry
+constexpr uint32_t kGrZeroEntryOffset = kGrEntryStates * 256 * 4;  // byte offset of the zero entry
 constexpr uint32_t kGrIdentityNext = 0x03020100u;               // byte s = s
+constexpr uint32_t kGrStateBits = 0x03030303u;                  // the state bits of a next[] word
+constexpr int kGrAdvanceShift = 26;                             // an entry's F advance
 
 // Decoded-block layout in LDS: four pad words, the 128 bitmap words, eight pad words.  The emission writes the
 // word before the bitmap and up to three words after it.  Rows stay 16-byte aligned, and the 140-word stride
@@ -116,7 +125,7 @@ __host__ __device__ constexpr GrByteStep gr_byte_step(int k, int st, int byte) {
 }
 
 struct alignas(16) GrTables {
-  uint64_t entry[kGrEntries + 1];  // (k, s, byte); then the zero entry and one pad entry
+  uint32_t entry[kGrEntries + 3];  // (k, s, byte); then the zero entry and three pad entries
   uint32_t next[2 * 256];          // (k, byte)
 };
 
@@ -129,9 +138,9 @@ constexpr GrTables gr_make_tables() {
         uint32_t nx = static_cast<uint32_t>(s);
         if (s <= k) {
           const GrByteStep r = gr_byte_step(k, s, byte);
-          nx = r.state;
-          const uint32_t hi = r.advance | (r.count << 12) | (static_cast<uint32_t>(r.mask >> 32) << 23);
-          t.entry[gr_entry_base(k) + s * 256 + byte] = (r.mask & 0xFFFFFFFFull) | (static_cast<uint64_t>(hi) << 32);
+          nx = r.state | (r.advance << 2);
+          t.entry[gr_entry_base(k) + s * 256 + byte] =
+              static_cast<uint32_t>(r.mask) | (r.advance << kGrAdvanceShift);
         }
         fields |= nx << (8 * s);
       }
@@ -140,6 +149,20 @@ constexpr GrTables gr_make_tables() {
   }
   return t;
 }
+
+// The packed fields hold every (k, s, byte): masks below 2^25, advances below 2^6.
+constexpr bool gr_tables_fit() {
+  for (int k = 1; k <= 2; ++k) {
+    for (int s = 0; s <= k; ++s) {
+      for (int byte = 0; byte < 256; ++byte) {
+        const GrByteStep r = gr_byte_step(k, s, byte);
+        if ((r.mask >> 25) != 0 || r.advance > 32 || r.state > 3) return false;
+      }
+    }
+  }
+  return true;
+}
+static_assert(gr_tables_fit(), "a next or entry field overflows");
 
 __constant__ GrTables kGrTables = gr_make_tables();
 constexpr int kGrTableVec4 = static_cast<int>(sizeof(GrTables) / 16);
@@ -325,6 +348,11 @@ __device__ __forceinline__ uint32_t gr_map_compose(uint32_t own, uint32_t earlie
   return __builtin_amdgcn_perm(own, own, earlier);
 }
 
+// The same of a next[] word, whose advances are dropped: a map again.
+__device__ __forceinline__ uint32_t gr_next_compose(uint32_t next, uint32_t earlier) {
+  return __builtin_amdgcn_perm(next, next, earlier) & kGrStateBits;
+}
+
 // Maps of 8 states (Rice k in [4, 7]): byte s of {lo, hi} is the image of s; states above k are never reached.
 struct GrMap8 {
   uint32_t lo, hi;
@@ -451,8 +479,7 @@ __device__ inline void gr_decode_block_group(const GrSpan<S>& sp, const GrTables
   } else if (!serial && k <= 2) {
     const uint32_t* __restrict__ nxt = tab->next + (k - 1) * 256;
     const char* __restrict__ ent = reinterpret_cast<const char*>(tab->entry);
-    const uint32_t kbase = static_cast<uint32_t>(gr_entry_base(k)) * 8u;  // byte offset of k's entries
-    const int nbytes = 4 * sp.nw;
+    const uint32_t kbase = static_cast<uint32_t>(gr_entry_base(k)) * 4u;  // byte offset of k's entries
     // words any lane of the wavefront holds (a group's first lane holds the most): the walks stop there
     const int maxw = wave_max_words<S>(sp.nw);
     // Each phase walks the span a word at a time under a wave-uniform guard, and issues a word's four table
@@ -468,7 +495,7 @@ __device__ inline void gr_decode_block_group(const GrSpan<S>& sp, const GrTables
         for (int b = 0; b < 4; ++b) f[4 * wd + b] = nxt[(sp.w[wd] >> (8 * b)) & 0xFFu];
         uint32_t cw = c;
 #pragma unroll
-        for (int b = 0; b < 4; ++b) cw = gr_map_compose(f[4 * wd + b], cw);
+        for (int b = 0; b < 4; ++b) cw = gr_next_compose(f[4 * wd + b], cw);
         c = wd < sp.nw ? cw : c;
       }
     }
@@ -477,74 +504,75 @@ __device__ inline void gr_decode_block_group(const GrSpan<S>& sp, const GrTables
     const uint32_t prev_map = dpp_mov<0x138, 0xF>(kGrIdentityNext, map);
     // the true entry state in all four bytes (a selector that steps it through a byte's map)
     uint32_t st = j == 0 ? 0u : __builtin_amdgcn_perm(prev_map, prev_map, 0u);
-    // ---- C: entries along the true path (the state chain runs on A's maps); F advance and codeword count
-    // sums from their high words, the masks read again for the emission
+    // ---- C: entry offsets along the true path and the lane's F advance (the chain runs on A's words, no LDS)
     uint32_t off[kBytes];
-    uint32_t hisum = 0u;
+    uint32_t adv4 = 0u;  // four times the advance
 #pragma unroll
     for (int wd = 0; wd < kMaxWords; ++wd) {
       if (wd < maxw) {
-        uint32_t hi[4];
+        const bool own = wd < sp.nw;
+        uint32_t sum = 0u;
 #pragma unroll
         for (int b = 0; b < 4; ++b) {
           const int i = 4 * wd + b;
           // entry index state * 256 + byte: the word's byte b into bits 0..7, the state into bits 8..15
           const uint32_t idx = __builtin_amdgcn_perm(st, sp.w[wd], 0x0C0C0400u | static_cast<uint32_t>(b));
-          off[i] = i < nbytes ? (idx << 3) + kbase : kGrZeroEntryOffset;
-          st = __builtin_amdgcn_perm(f[i], f[i], st);
-          hi[b] = *reinterpret_cast<const uint32_t*>(ent + off[i] + 4);
+          off[i] = own ? (idx << 2) + kbase : kGrZeroEntryOffset;
+          const uint32_t x = __builtin_amdgcn_perm(f[i], f[i], st);
+          sum += x & 0xFCu;
+          st = x & kGrStateBits;
         }
-#pragma unroll
-        for (int b = 0; b < 4; ++b) hisum += hi[b];
+        adv4 += own ? sum : 0u;
       }
     }
-    asm volatile("" ::: "memory");  // the emission reads the entries again rather than keeping 16 of them live
-    // advance sum (< 2^12) and count sum (< 2^9) of the lane, repacked as adv | count << 16 for the group sums
-    const uint32_t packed = (hisum & 0xFFFu) | (((hisum >> 12) & 0x1FFu) << 16);
-    const uint32_t incl = group_incl_sum<S>(packed);
-    const int total = static_cast<int>(group_last<S>(incl) >> 16);
-    serial = total != one_count;
-    if (!serial) {
-      // bit position + 32 of the lane's first mask bit 0 (F at the span start - 1, biased past the front pad)
-      uint32_t posb = ((incl - packed) & 0xFFFFu) + 31u;
-      uint32_t* base = out - 1;
-      // OR a mask (< 2^64) whose bit 0 is at posb - 32 into the bitmap; word 129 and up are the back pads,
-      // where only positions past 4095 land
-      const auto emit = [&](uint64_t m) {
-        const uint32_t rel = posb & 31u;
-        const uint32_t widx = (posb >> 5) < 129u ? (posb >> 5) : 129u;
-        const uint64_t v = m << rel;
-        atomicOr(&base[widx], static_cast<uint32_t>(v));
-        atomicOr(&base[widx + 1], static_cast<uint32_t>(v >> 32));
-        atomicOr(&base[widx + 2], static_cast<uint32_t>((m >> 32) << rel >> 32));
-      };
-      // k <= 2: a byte's mask is below 2^25 and its advance at most 32, so two bytes fit one 64-bit mask
+    const uint32_t adv = adv4 >> 2;
+    const uint32_t incl = group_incl_sum<S>(adv);
+    // bit position + 32 of the lane's first mask bit 0 (F at the span start - 1, biased past the front pad)
+    uint32_t posb = incl - adv + 31u;
+    uint32_t* base = out - 1;
+    // OR a mask (< 2^64) whose bit 0 is at posb - 32 into the bitmap; word 129 and up are the back pads,
+    // where only positions past 4095 land
+    const auto emit = [&](uint64_t m) {
+      const uint32_t rel = posb & 31u;
+      const uint32_t widx = (posb >> 5) < 129u ? (posb >> 5) : 129u;
+      const uint64_t v = m << rel;
+      const uint32_t v1 = static_cast<uint32_t>(v >> 32);
+      const uint32_t v2 = static_cast<uint32_t>((m >> 32) << rel >> 32);
+      atomicOr(&base[widx], static_cast<uint32_t>(v));
+      if (v1 != 0u) atomicOr(&base[widx + 1], v1);
+      if (v2 != 0u) atomicOr(&base[widx + 2], v2);
+    };
+    // k <= 2: a byte's mask is below 2^25 and its advance at most 32, so two bytes fit one 64-bit mask
 #pragma unroll
-      for (int wd = 0; wd < kMaxWords; ++wd) {
-        if (wd < maxw) {
-          uint2 e[4];
+    for (int wd = 0; wd < kMaxWords; ++wd) {
+      if (wd < maxw) {
+        uint32_t e[4];
 #pragma unroll
-          for (int b = 0; b < 4; ++b) e[b] = *reinterpret_cast<const uint2*>(ent + off[4 * wd + b]);
+        for (int b = 0; b < 4; ++b) e[b] = *reinterpret_cast<const uint32_t*>(ent + off[4 * wd + b]);
 #pragma unroll
-          for (int b = 0; b < 4; b += 2) {
-            const uint32_t a0 = e[b].y & 0x7Fu;
-            emit(static_cast<uint64_t>(e[b].x) | (static_cast<uint64_t>(e[b + 1].x) << a0));
-            posb += a0 + (e[b + 1].y & 0x7Fu);
-          }
+        for (int b = 0; b < 4; b += 2) {
+          const uint32_t a0 = e[b] >> kGrAdvanceShift;
+          emit(static_cast<uint64_t>(e[b] & 0x1FFFFFFu) | (static_cast<uint64_t>(e[b + 1] & 0x1FFFFFFu) << a0));
+          posb += a0 + (e[b + 1] >> kGrAdvanceShift);
         }
       }
+    }
+    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    // the completed codewords are the bitmap's ones (positions increase, so no two share a bit) when no pad was
+    // written; a written pad makes the sum differ from any count
+    const uint4* mine = reinterpret_cast<const uint4*>(out) + j * (kGrWords / 4 / S);
+    uint32_t ones = j < 3 && out[kGrWords + j] != 0u ? 1u << 24 : 0u;
+#pragma unroll
+    for (int i = 0; i < kGrWords / 4 / S; ++i) {
+      const uint4 o = mine[i];
+      ones += static_cast<uint32_t>(__popc(o.x) + __popc(o.y) + __popc(o.z) + __popc(o.w));
+    }
+    serial = static_cast<int>(group_last<S>(group_incl_sum<S>(ones))) != one_count;
+    if (serial) {
       __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
       __builtin_amdgcn_wave_barrier();
-      const uint32_t pad = j < 3 ? out[kGrWords + j] : 0u;
-      const uint64_t hit = __ballot(pad != 0u);
-      const uint64_t group_mask = (S == 64 ? ~0ull : ((1ull << S) - 1ull))
-                                  << ((static_cast<int>(__lane_id()) / S) * S);
-      serial = (hit & group_mask) != 0ull;
-      if (serial) {
-        __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        for (int w = j; w < kGrWords; w += S) out[w] = 0u;
-      }
+      for (int w = j; w < kGrWords; w += S) out[w] = 0u;
     }
   } else if (!serial && tab4 != nullptr) {
     // k in [3, 7]: nibble tables
