@@ -509,10 +509,19 @@ __device__ __forceinline__ void route_dispatch(const RouteArgs& ra, int kind, Ro
 }
 
 // The router and the shared backbone projection of the same tokens in one launch (they do not depend on
-// each other): workgroup 0 routes; every other workgroup runs kRbSub blocks of the backbone's grid
+// each other): workgroup 0 routes; every other workgroup runs up to kRbSub blocks of the backbone's grid
 // (backbone_block, 256 threads each, sharing the workgroup's one barrier).  The two roles never share a
 // workgroup, so their LDS is one union.
 constexpr int kRbSub = kRouteThreads / kBbThreads;
+constexpr int kRbFillWgs = 256;  // one workgroup a CU
+
+// Blocks a workgroup runs: kRbSub only when that still covers the CUs.  The backbone's plans aim at 256 to 576 blocks,
+// which four to a workgroup left on half of the CUs (Mixtral, 64 tokens, 20.6 -> 19.8 us; OLMoE, 16 tokens,
+// 7.5 -> 7.1).
+static int route_backbone_subs(int blocks) {
+  const int n = blocks / kRbFillWgs;
+  return n < 1 ? 1 : n < kRbSub ? n : kRbSub;
+}
 
 template <int TT>
 union RouteBackboneSmem {
@@ -523,7 +532,7 @@ union RouteBackboneSmem {
 
 template <int TT, int B>
 __global__ __launch_bounds__(kRouteThreads) void route_backbone_kernel(RouteArgs ra, int kind, BackboneArgs ba,
-                                                                      int bb_blocks, int gx, int gy) {
+                                                                      int bb_blocks, int gx, int gy, int nsub) {
   __shared__ RouteBackboneSmem<TT> sm;
   const int tid = static_cast<int>(threadIdx.x);
   if (blockIdx.x == 0) {
@@ -531,8 +540,8 @@ __global__ __launch_bounds__(kRouteThreads) void route_backbone_kernel(RouteArgs
     return;
   }
   const int sub = tid / kBbThreads;
-  const int vb = (static_cast<int>(blockIdx.x) - 1) * kRbSub + sub;
-  const bool active = vb < bb_blocks;
+  const int vb = (static_cast<int>(blockIdx.x) - 1) * nsub + sub;
+  const bool active = sub < nsub && vb < bb_blocks;
   const int v = active ? vb : 0;
   backbone_block<TT, B>(ba, active, v % gx, (v / gx) % gy, v / (gx * gy), tid % kBbThreads, sm.red[sub]);
 }
@@ -853,7 +862,42 @@ int tris::route_prepare(const float* router_logits, int32_t num_tokens, int32_t 
   return TRIS_OK;
 }
 
+static void launch_route_tokens(const RouteArgs& ra, hipStream_t s) {
+  // every token's wavefront resident at once up to 8192 workgroups (32768 tokens), then a grid-stride loop
+  const int64_t wgs = (static_cast<int64_t>(ra.tokens) + kRouteTokWaves - 1) / kRouteTokWaves;
+  const dim3 grid(static_cast<unsigned>(wgs < 8192 ? wgs : 8192));
+  const int per_lane = ceil_div(ra.num_experts, kWave);
+  if (per_lane <= 1) {
+    hipLaunchKernelGGL((route_topk_tokens_kernel<1>), grid, dim3(kRouteTokThreads), 0, s, ra);
+  } else if (per_lane <= 2) {
+    hipLaunchKernelGGL((route_topk_tokens_kernel<2>), grid, dim3(kRouteTokThreads), 0, s, ra);
+  } else if (per_lane <= 4) {
+    hipLaunchKernelGGL((route_topk_tokens_kernel<4>), grid, dim3(kRouteTokThreads), 0, s, ra);
+  } else if (per_lane <= 8) {
+    hipLaunchKernelGGL((route_topk_tokens_kernel<8>), grid, dim3(kRouteTokThreads), 0, s, ra);
+  } else {
+    hipLaunchKernelGGL((route_topk_tokens_kernel<kRouteSmallMaxExperts / kWave>), grid, dim3(kRouteTokThreads), 0, s,
+                       ra);
+  }
+}
+
+// More than one 64-token chunk: the one-workgroup router routes 16 tokens at a time and scatters a chunk at a time on
+// one CU, so the token-parallel softmax / top-k and the per-expert scatter take over (8 experts, top 2: 64 tokens 7.7
+// against 8.5 us, 333 tokens 26.5 against 9.1, 1000 tokens 71 against 10.6; 128 experts, top 8: 32 tokens 8.7 against
+// 9.6, 250 tokens 44 against 11.4).  The same outputs: both give each expert its tokens in order.
+constexpr int kRouteSmallMaxTokens = 64;
+
 static int launch_route(const RouteArgs& ra, hipStream_t s, const char* who) {
+  if (ra.tokens > kRouteSmallMaxTokens && ra.selected != nullptr) {
+    launch_route_tokens(ra, s);
+    const int rc = check_launch(who);
+    if (rc) return rc;
+    hipLaunchKernelGGL(route_group_scatter_kernel, dim3(ra.num_experts + 1), dim3(kScatterThreads),
+                       static_cast<size_t>(ra.num_experts) * sizeof(int), s, ra.selected, ra.tokens * ra.top_k,
+                       ra.top_k, ra.num_experts, ra.m_tile, ra.expert_ids, ra.segment_offsets, ra.problem_offsets,
+                       ra.counts, ra.perm, ra.token_idx, ra.slots, ra.grouped_expert_ids, ra.inverse_perm);
+    return check_launch(who);
+  }
   switch (route_variant(ra.tokens, ra.num_experts, ra.top_k)) {
     case kRouteWave2: hipLaunchKernelGGL((route_topk_wave_kernel<2>), dim3(1), dim3(kWave), 0, s, ra); break;
     case kRouteWave8: hipLaunchKernelGGL((route_topk_wave_kernel<8>), dim3(1), dim3(kWave), 0, s, ra); break;
@@ -909,28 +953,13 @@ extern "C" int tris_route_topk(const float* router_logits, int32_t num_tokens, i
   ra.weights16 = routing_weights_f16;
   ra.weights32 = routing_weights_f32;
   ra.selected = selected_experts;
-  // every token's wavefront resident at once up to 8192 workgroups (32768 tokens), then a grid-stride loop
-  const int64_t wgs = (static_cast<int64_t>(num_tokens) + kRouteTokWaves - 1) / kRouteTokWaves;
-  const dim3 grid(static_cast<unsigned>(wgs < 8192 ? wgs : 8192));
-  hipStream_t s = static_cast<hipStream_t>(stream);
-  const int per_lane = ceil_div(num_experts, kWave);
-  if (per_lane <= 1) {
-    hipLaunchKernelGGL((route_topk_tokens_kernel<1>), grid, dim3(kRouteTokThreads), 0, s, ra);
-  } else if (per_lane <= 2) {
-    hipLaunchKernelGGL((route_topk_tokens_kernel<2>), grid, dim3(kRouteTokThreads), 0, s, ra);
-  } else if (per_lane <= 4) {
-    hipLaunchKernelGGL((route_topk_tokens_kernel<4>), grid, dim3(kRouteTokThreads), 0, s, ra);
-  } else if (per_lane <= 8) {
-    hipLaunchKernelGGL((route_topk_tokens_kernel<8>), grid, dim3(kRouteTokThreads), 0, s, ra);
-  } else {
-    hipLaunchKernelGGL((route_topk_tokens_kernel<kRouteSmallMaxExperts / kWave>), grid, dim3(kRouteTokThreads), 0, s,
-                       ra);
-  }
+  launch_route_tokens(ra, static_cast<hipStream_t>(stream));
   return check_launch(who);
 }
 
 // Backbone token tiles per workgroup in the merged launch: the 1024-thread workgroup caps the kernel at 128
-// VGPRs, which the 8-step load batches fit with one token tile only.
+// VGPRs, which the 8-step load batches fit with one token tile only; four tiles with 4-step batches spilled 24 of them
+// (64 tokens: 19.8 us, with 2-step batches 16.9).
 constexpr int kRbMaxTokens = 64;
 
 extern "C" int tris_route_topk_backbone(const float* router_logits, int32_t num_tokens, int32_t num_experts,
@@ -964,24 +993,25 @@ extern "C" int tris_route_topk_backbone(const float* router_logits, int32_t num_
   const int gy = pl.token_groups * pl.slices;
   const int64_t blocks = static_cast<int64_t>(gx) * gy * nproj;
   TRIS_REQUIRE(blocks < (int64_t{1} << 28), "%s: backbone grid too large", who);
-  const dim3 grid(static_cast<unsigned>(1 + ceil_div(static_cast<int>(blocks), kRbSub)));
+  const int nsub = route_backbone_subs(static_cast<int>(blocks));
+  const dim3 grid(static_cast<unsigned>(1 + ceil_div(static_cast<int>(blocks), nsub)));
   const int kind = route_variant(num_tokens, num_experts, top_k);
   switch (pl.tt) {
     case 1:
       hipLaunchKernelGGL((route_backbone_kernel<1, 8>), grid, dim3(kRouteThreads), 0, s, ra, kind, ba,
-                         static_cast<int>(blocks), gx, gy);
+                         static_cast<int>(blocks), gx, gy, nsub);
       break;
     case 2:
       hipLaunchKernelGGL((route_backbone_kernel<2, 4>), grid, dim3(kRouteThreads), 0, s, ra, kind, ba,
-                         static_cast<int>(blocks), gx, gy);
+                         static_cast<int>(blocks), gx, gy, nsub);
       break;
     case 3:
       hipLaunchKernelGGL((route_backbone_kernel<3, 4>), grid, dim3(kRouteThreads), 0, s, ra, kind, ba,
-                         static_cast<int>(blocks), gx, gy);
+                         static_cast<int>(blocks), gx, gy, nsub);
       break;
     default:
-      hipLaunchKernelGGL((route_backbone_kernel<4, 4>), grid, dim3(kRouteThreads), 0, s, ra, kind, ba,
-                         static_cast<int>(blocks), gx, gy);
+      hipLaunchKernelGGL((route_backbone_kernel<4, 2>), grid, dim3(kRouteThreads), 0, s, ra, kind, ba,
+                         static_cast<int>(blocks), gx, gy, nsub);
       break;
   }
   rc = check_launch(who);

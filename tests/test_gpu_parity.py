@@ -398,6 +398,13 @@ def test_route_topk_fused_matches_oracle(tris, oracle_mod, cuda, t, k, e, renorm
     np.testing.assert_array_equal(r["perm"].cpu().numpy()[inv], np.arange(t * k))
 
 
+@pytest.mark.parametrize("t,k,e,renorm", [(64, 2, 8, True), (65, 2, 8, True), (65, 8, 128, False), (333, 2, 8, True)])
+def test_route_topk_one_chunk_edge(tris, oracle_mod, cuda, t, k, e, renorm):
+    """The one-workgroup router up to 64 tokens and the two launches of tris_route_topk_grouped above: the same
+    exact route and weights, within the same bounds."""
+    test_route_topk_fused_matches_oracle(tris, oracle_mod, cuda, t, k, e, renorm)
+
+
 @pytest.mark.parametrize("t,k,e,renorm", [(2048, 2, 8, True), (1024, 8, 256, True), (3000, 1, 64, False),
                                           (100, 16, 1024, True), (5, 3, 7, False), (40000, 2, 8, True),
                                           (257, 6, 60, False), (0, 2, 8, True)])
