@@ -1663,9 +1663,11 @@ def _set_uniform_k64(st, g_idx):
 
 def _linears_ok(x: torch.Tensor, structs) -> bool:
     """tris_compact3_linears_forward takes these matrices of x's width: whole 64-column K tiles, 16-byte aligned rows,
-    tensors below 2 GiB (any g_idx; it does not read it on the host)."""
+    tensors below 2 GiB (any g_idx; it does not read it on the host), on the current device (where its list of one expert
+    lies)."""
     rank = int(x.size(1))
-    if rank % 64 or x.data_ptr() % 16 or rank * 64 >= 1 << 31:
+    if (rank % 64 or x.data_ptr() % 16 or rank * 64 >= 1 << 31
+            or torch._C._cuda_getDevice() != x.device.index):
         return False
     for st in structs:
         n = int(st.outfeatures)

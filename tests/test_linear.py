@@ -200,3 +200,16 @@ def test_linear_matrix_core_shapes(tris, oracle_mod, cuda, n, k, batch, groups):
     t = lambda a: torch.from_numpy(np.ascontiguousarray(a)).to(cuda)
     got = _linear(ext, t(x), _dev(m, cuda), t(s_in), t(s_out), t(bias))
     assert_close(got.cpu().numpy(), oracle_mod.compact3_linear(x, m, s_in, s_out, bias), f"linear n={n} k={k}")
+
+
+def test_linears_stay_on_the_current_device(tris, monkeypatch):
+    """The matrix-core linears are refused on any device but the current one (the exact kernel takes those), and only
+    there."""
+    from types import SimpleNamespace
+
+    st = SimpleNamespace(outfeatures=64, qweight2_sparse_rows=1, num_groups=2)
+    x = SimpleNamespace(size=lambda d: (4, 256)[d], data_ptr=lambda: 4096, device=torch.device("cuda", 1))
+    monkeypatch.setattr(torch._C, "_cuda_getDevice", lambda: 1, raising=False)
+    assert tris["ext"]._linears_ok(x, (st,))
+    monkeypatch.setattr(torch._C, "_cuda_getDevice", lambda: 0, raising=False)
+    assert not tris["ext"]._linears_ok(x, (st,))
