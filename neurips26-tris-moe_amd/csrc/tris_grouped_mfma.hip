@@ -46,6 +46,7 @@ namespace tris {
 
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
+typedef uint16_t u16x2 __attribute__((ext_vector_type(2)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 constexpr int kMfWaves = 4;
@@ -1385,8 +1386,8 @@ void grouped_mfma_kernel(MfmaArgs a) {
 // chunks (blockIdx.y = row tile x slice), stages each chunk as the decode kernel does, and leaves fp32 partial sums
 // [slice][batch][N]; linear_finish_kernel adds the slices in order, then the addend, scale and bias.  Slices are taken
 // until the launch fills the GPU.  The row scales are staged per K tile (the decode kernel's per group would not fit), and
-// whether every K tile of a chunk lies in one group is found on the way: a chunk where one does not takes a scalar loop
-// over its columns instead, so no launch waits for the host to look at g_idx.
+// whether every K tile of a chunk lies in one group is found on the way: a chunk where one does not (or with an
+// infinite activation) takes a scalar loop over its columns instead, so no launch waits for the host to look at g_idx.
 // Q, K and V of 2048 x 2048 at 16 rows: 10.0 us, the finish 3.4 and the bitmaps 9.5, against 504 us of the exact VALU
 // kernel (two launches) and seven host round trips to read g_idx.
 struct LinProj {
@@ -1403,7 +1404,7 @@ struct LinArgs {
   int batch, slices, chunks;
 };
 
-// The exact weight of column k (of the whole matrix) for output n, from memory (chunks with split K tiles).
+// The exact weight of column k (of the whole matrix) for output n, from memory (chunks with split K tiles or infinities).
 __device__ __forceinline__ float lin_weight(const LinProj& a, int k, int n) {
   const tris_compact3_payload& p = a.p;
   const int N = p.outfeatures;
@@ -1518,6 +1519,19 @@ __global__ __launch_bounds__(kMfThreads) __attribute__((amdgpu_waves_per_eu(3, 8
     }
     mf_cols_write<false, true>(pa, rc, kc, utid, ch, cols, kMfChunk);
     mf_rows_write<kRows, false>(rows, rc, wave, lane, xs);
+    // an infinite activation: the GEMM multiplies a salient column by its zero factors first (inf * 0), so the chunk walks
+    // its columns.  |v| + 0x83FF (modulo 2^16) is 0xFFFF for an infinity alone; a NaN gives NaN either way.
+    u16x2 top = {0, 0};
+#pragma unroll
+    for (int h = 0; h < MfRowRegs<kRows, false>::kRuns; ++h) {
+      const uint32_t v[4] = {rows.xv[h].x, rows.xv[h].y, rows.xv[h].z, rows.xv[h].w};
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const u16x2 m = __builtin_bit_cast(u16x2, v[i] & 0x7FFF7FFFu) + u16x2{0x83FF, 0x83FF};
+        top = __builtin_elementwise_max(top, m);
+      }
+    }
+    const bool infinite = top[0] == 0xFFFF || top[1] == 0xFFFF;
     const MfChunkMeta cm = mf_chunk_meta(cols, kMfChunk);
     {
       const int row = lane / 4;
@@ -1530,7 +1544,7 @@ __global__ __launch_bounds__(kMfThreads) __attribute__((amdgpu_waves_per_eu(3, 8
             make_uint2(static_cast<uint32_t>(rp[h]), static_cast<uint32_t>(rp[h] >> 32));
       }
     }
-    if (!__syncthreads_or(split ? 1 : 0)) {
+    if (!__syncthreads_or(split || infinite ? 1 : 0)) {
       uint32_t q2w[1][2];
       mf_q2_issue(q2, p.qweight2_sparse_rows, N, n[0], cm, q2w[0]);
       mf_compute<1, kRt, false>(q2, p.qweight2_sparse_rows, N, rank, kMfMaxGroups, kc, n, xr, lane, ch, cm, wb, q2w, acc);

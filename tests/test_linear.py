@@ -202,6 +202,35 @@ def test_linear_matrix_core_shapes(tris, oracle_mod, cuda, n, k, batch, groups):
     assert_close(got.cpu().numpy(), oracle_mod.compact3_linear(x, m, s_in, s_out, bias), f"linear n={n} k={k}")
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("batch", [1, 16, 33])
+def test_linear_infinite_activations(tris, oracle_mod, cuda, batch):
+    """An infinity in a salient column, in a plain one and in none, a row each, and a NaN: the outputs are infinite with
+    the oracle's signs, NaN or finite exactly where the oracle's are."""
+    from test_gpu_parity import assert_close, note
+
+    n, k = 80, 640
+    note(f"compact3 linear with infinities, batch={batch}")
+    ext = tris["ext"]
+    mods, rng = _modules(ext, 1, n, k, 12)
+    m = mods[0]
+    salient = (m["c_map"].view(np.uint32)[np.arange(k) // 32] >> (np.arange(k) % 32)) & 1
+    x = rng.standard_normal((batch, k)).astype(np.float16)
+    x[0, np.flatnonzero(salient)[-1]] = np.inf
+    if batch > 3:
+        x[1, np.flatnonzero(salient == 0)[0]] = -np.inf
+        x[2, 5] = np.nan
+    t = lambda a: torch.from_numpy(np.ascontiguousarray(a)).to(cuda)
+    got = _linear(ext, t(x), _dev(m, cuda)).cpu().numpy()
+    want = oracle_mod.compact3_linear(x, m)
+    assert np.isinf(want[0]).all()
+    np.testing.assert_array_equal(np.isnan(got), np.isnan(want))
+    np.testing.assert_array_equal(np.where(np.isinf(got), got, 0), np.where(np.isinf(want), want, 0))
+    rows = np.isfinite(want).all(1)
+    if rows.any():
+        assert_close(got[rows], want[rows], f"finite rows, batch={batch}")
+
+
 def test_linears_stay_on_the_current_device(tris, monkeypatch):
     """The matrix-core linears are refused on any device but the current one (the exact kernel takes those), and only
     there."""
