@@ -246,7 +246,8 @@ __global__ __launch_bounds__(kSpanThreads) __attribute__((amdgpu_waves_per_eu(5)
 
 // Fills job from one projection's arguments; returns the job's block count (0: nothing to do).
 int make_gr_job(GrJob* job, int32_t* out, const int32_t* words, const int32_t* offsets, const int32_t* meta,
-                int num_experts, int words_stride, int packed_rows, int outfeatures, bool dense, const char* who) {
+                int num_experts, int words_stride, int packed_rows, int outfeatures, bool dense, const char* who,
+                bool no_words_ok = false) {
   TRIS_REQUIRE(packed_rows >= 0 && outfeatures >= 0 && words_stride >= 0 && num_experts >= 0,
                "%s: negative size", who);
   const int nob = ceil_div(outfeatures, kTileOut);
@@ -254,7 +255,7 @@ int make_gr_job(GrJob* job, int32_t* out, const int32_t* words, const int32_t* o
   *job = GrJob{out, words, offsets, meta, num_experts, words_stride, nblk, nob, dense ? packed_rows : 0,
                dense ? outfeatures : 0};
   if (nblk == 0) return TRIS_OK;
-  TRIS_REQUIRE(out && offsets && meta && words, "%s: null pointer", who);
+  TRIS_REQUIRE(out && offsets && meta && (words || (no_words_ok && words_stride == 0)), "%s: null pointer", who);
   return TRIS_OK;
 }
 
@@ -331,6 +332,20 @@ int launch_gr_jobs(const GrJobs& jobs, int num_jobs, const int32_t* expert_ids, 
     hipLaunchKernelGGL((gr_decode_span_kernel<32>), g3, dim3(kSpanThreads), 0, s, jobs, wk, expert_ids, red, rt);
   }
   return check_launch(who);
+}
+
+// The predecode of tris_grouped_block_gr_predecode_multi for non-expert matrices (checked payloads).  One without a
+// split column has no words at all: every block is empty, and the decoder reads none.
+int predecode_linears(const tris_gr_predecode_job* jobs, int num_jobs, const int32_t* expert0, void* stream,
+                      const char* who) {
+  GrJobs g{};
+  for (int q = 0; q < num_jobs; ++q) {
+    const tris_gr_predecode_job& j = jobs[q];
+    int rc = make_gr_job(&g.job[q], j.decoded, j.q_gmap_gr_words, j.q_gmap_gr_offsets, j.q_gmap_gr_meta,
+                         j.num_experts, j.words_stride, j.packed_rows, j.outfeatures, false, who, true);
+    if (rc) return rc;
+  }
+  return launch_gr_jobs(g, num_jobs, expert0, 1, stream, who);
 }
 
 }  // namespace tris

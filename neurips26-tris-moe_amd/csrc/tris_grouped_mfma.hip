@@ -2069,6 +2069,8 @@ __global__ __launch_bounds__(kUnits * kMfThreads) __attribute__((amdgpu_waves_pe
 }
 
 int check_payload(const tris_compact3_payload* p, bool need_gr, const char* who);
+int predecode_linears(const tris_gr_predecode_job* jobs, int num_jobs, const int32_t* expert0, void* stream,
+                      const char* who);
 
 static bool allow_mfma_lds(const void* kernel, int bytes) {
   // dynamic LDS granted so far per kernel (the weight-stationary kernel's two instantiations)
@@ -2360,7 +2362,7 @@ int launch_linear_mfma(const uint16_t* input, int batch, const tris_compact3_pay
     args.proj[i].part = sums;
     sums += static_cast<int64_t>(args.slices) * batch * widths[i];
   }
-  int rc = tris_grouped_block_gr_predecode_multi(jobs, count, static_cast<const int32_t*>(ids), 1, stream);
+  int rc = predecode_linears(jobs, count, static_cast<const int32_t*>(ids), stream, who);
   if (rc) return rc;
   hipStream_t s = static_cast<hipStream_t>(stream);
   const int rows = batch <= kMfRows ? kMfRows : 32;

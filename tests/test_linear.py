@@ -242,3 +242,27 @@ def test_linears_stay_on_the_current_device(tris, monkeypatch):
     assert tris["ext"]._linears_ok(x, (st,))
     monkeypatch.setattr(torch._C, "_cuda_getDevice", lambda: 0, raising=False)
     assert not tris["ext"]._linears_ok(x, (st,))
+
+
+@pytest.mark.gpu
+def test_linear_without_split_columns(tris, oracle_mod, cuda):
+    """A matrix with no split column at all codes to no GR words (an empty tensor): single and Q/K/V calls take it, as
+    the exact kernel does."""
+    from test_gpu_parity import assert_close, note
+
+    note("compact3 linear with an empty GR stream")
+    ext = tris["ext"]
+    n, k, batch = 72, 128, 5
+    rng = np.random.default_rng(31)
+    proj = synthetic.make_projection(rng, 3, n, k, 0.0, rng.random(k).astype(np.float32) + 0.5, ext.gr_encode)
+    mods = [{key: np.ascontiguousarray(proj[key][e]) for key in MODULE_KEYS} for e in range(3)]
+    assert all(m["q_gmap_gr_words"].size == 0 for m in mods)
+    dm = [_dev(m, cuda) for m in mods]
+    x = (rng.standard_normal((batch, k)) * 1.5).astype(np.float16)
+    xd = torch.from_numpy(x).to(cuda)
+    zero = torch.zeros(n, dtype=torch.float16, device=cuda)
+    qkv = ext.compact3_qkv_linear_forward(xd, *(a for m in dm for a in [*(m[key] for key in MODULE_KEYS), zero]))
+    for i in range(3):
+        want = oracle_mod.compact3_linear(x, mods[i])
+        assert_close(_linear(ext, xd, dm[i]).cpu().numpy(), want, f"empty stream {i}")
+        assert_close(qkv[i].cpu().numpy(), want, f"empty stream qkv {i}")
