@@ -1387,7 +1387,7 @@ void grouped_mfma_kernel(MfmaArgs a) {
 // [slice][batch][N]; linear_finish_kernel adds the slices in order, then the addend, scale and bias.  Slices are taken
 // until the launch fills the GPU.  The row scales are staged per K tile (the decode kernel's per group would not fit), and
 // whether every K tile of a chunk lies in one group is found on the way: a chunk where one does not (or with an
-// infinite activation) takes a scalar loop over its columns instead, so no launch waits for the host to look at g_idx.
+// infinite activation, or a row scale that is not finite) takes a scalar loop over its columns instead, so no launch waits for the host to look at g_idx.
 // Q, K and V of 2048 x 2048 at 16 rows: 10.0 us, the finish 3.4 and the bitmaps 9.5, against 504 us of the exact VALU
 // kernel (two launches) and seven host round trips to read g_idx.
 struct LinProj {
@@ -1404,7 +1404,8 @@ struct LinArgs {
   int batch, slices, chunks;
 };
 
-// The exact weight of column k (of the whole matrix) for output n, from memory (chunks with split K tiles or infinities).
+// The exact weight of column k (of the whole matrix) for output n, from memory (chunks with split K tiles, infinities or scales that are not
+// finite).
 __device__ __forceinline__ float lin_weight(const LinProj& a, int k, int n) {
   const tris_compact3_payload& p = a.p;
   const int N = p.outfeatures;
@@ -1532,6 +1533,15 @@ __global__ __launch_bounds__(kMfThreads) __attribute__((amdgpu_waves_per_eu(3, 8
       }
     }
     const bool infinite = top[0] == 0xFFFF || top[1] == 0xFFFF;
+    // a row scale that is not finite: where no column picks it (R_d without a split column, R0 and R1 without a salient
+    // one) it must not count, but the GEMM multiplies it by the zero factors of salient columns and padding slots
+    u16x2 expo = {0, 0};
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      expo = __builtin_elementwise_max(expo, __builtin_bit_cast(u16x2, static_cast<uint32_t>(rp[h]) & 0x7C007C00u));
+      expo = __builtin_elementwise_max(expo, __builtin_bit_cast(u16x2, static_cast<uint32_t>(rp[h] >> 32) & 0x7C007C00u));
+    }
+    const bool unbounded = expo[0] == 0x7C00 || expo[1] == 0x7C00;
     const MfChunkMeta cm = mf_chunk_meta(cols, kMfChunk);
     {
       const int row = lane / 4;
@@ -1544,7 +1554,7 @@ __global__ __launch_bounds__(kMfThreads) __attribute__((amdgpu_waves_per_eu(3, 8
             make_uint2(static_cast<uint32_t>(rp[h]), static_cast<uint32_t>(rp[h] >> 32));
       }
     }
-    if (!__syncthreads_or(split || infinite ? 1 : 0)) {
+    if (!__syncthreads_or(split || infinite || unbounded ? 1 : 0)) {
       uint32_t q2w[1][2];
       mf_q2_issue(q2, p.qweight2_sparse_rows, N, n[0], cm, q2w[0]);
       mf_compute<1, kRt, false>(q2, p.qweight2_sparse_rows, N, rank, kMfMaxGroups, kc, n, xr, lane, ch, cm, wb, q2w, acc);

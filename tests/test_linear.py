@@ -266,3 +266,28 @@ def test_linear_without_split_columns(tris, oracle_mod, cuda):
         want = oracle_mod.compact3_linear(x, mods[i])
         assert_close(_linear(ext, xd, dm[i]).cpu().numpy(), want, f"empty stream {i}")
         assert_close(qkv[i].cpu().numpy(), want, f"empty stream qkv {i}")
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("batch", [1, 20])
+def test_linear_unused_scales_not_finite(tris, oracle_mod, cuda, batch):
+    """Row scales that no column picks may hold anything (a mean over no column): R_nd where every plain column is
+    split, R0 and R1 of a group without salient columns, the first among them.  The outputs stay the oracle's."""
+    from test_gpu_parity import assert_close, note
+
+    note(f"compact3 linear with unused scales not finite, batch={batch}")
+    ext = tris["ext"]
+    n, k, group = 72, 640, 128
+    rng = np.random.default_rng(33)
+    norm = np.where(np.arange(k) // group == 2, 9.0, 1.0)  # every salient column in group 2
+    proj = synthetic.make_projection(rng, 1, n, k, 1.0, norm, ext.gr_encode, salient_counts=[9])
+    m = {key: np.ascontiguousarray(proj[key][0]) for key in MODULE_KEYS}
+    rp = m["row_pack3"].view(np.uint16).reshape(n, k // group, 4)  # R0, R1, R_d, R_nd
+    rp[:, :, 3] = 0x7C00                     # inf
+    rp[:, [0, 1, 3, 4], 0] = 0x7E00          # NaN
+    rp[:, [0, 1, 3, 4], 1] = 0xFC00          # -inf
+    x = (rng.standard_normal((batch, k)) * 1.5).astype(np.float16)
+    want = oracle_mod.compact3_linear(x, m)
+    assert np.isfinite(want).all()
+    got = _linear(ext, torch.from_numpy(x).to(cuda), _dev(m, cuda)).cpu().numpy()
+    assert_close(got, want, f"unused scales, batch={batch}")
