@@ -689,7 +689,7 @@ int tris_compact3_dual_linear_forward(const uint16_t* input, int32_t batch, cons
  * One to TRIS_MAX_LINEARS non-expert compact3 linears of one input (no reference counterpart: batches
  * compact3_linear_forward calls, TriSMoE_cuda.cpp:497-700) on the matrix cores: tris_compact3_linear_forward's results
  * up to the order of the fp32 sums, for any g_idx (512-column chunks with K tiles of several groups, with an
- * infinite activation or with a row scale that is not finite take a scalar loop on the device).  Every
+ * infinite activation or with a row scale that is not finite build their weights column by column on the device).  Every
  * payload has num_experts == 1 and the same rank, a multiple of 64; input and workspace are 16-byte aligned; input_scale
  * applies to all, addend to the first; outputs[i] fp16 [batch, outfeatures of payload i].  The workspace (of
  * tris_compact3_linears_workspace_bytes bytes) holds the decoded split bitmaps and fp32 partial sums.  A matrix gives the

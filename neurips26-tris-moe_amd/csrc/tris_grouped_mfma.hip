@@ -1387,7 +1387,10 @@ void grouped_mfma_kernel(MfmaArgs a) {
 // [slice][batch][N]; linear_finish_kernel adds the slices in order, then the addend, scale and bias.  Slices are taken
 // until the launch fills the GPU.  The row scales are staged per K tile (the decode kernel's per group would not fit), and
 // whether every K tile of a chunk lies in one group is found on the way: a chunk where one does not (or with an
-// infinite activation, or a row scale that is not finite) takes a scalar loop over its columns instead, so no launch waits for the host to look at g_idx.
+// infinite activation, or a row scale that is not finite) builds its operands column by column from memory instead
+// (lin_exact_row), so no launch waits for the host to look at g_idx.  Bound by the loads of each column's scales: a
+// matrix of 4096 x 4096 with a shuffled g_idx takes 65 us at 16 rows and 406 at 256 (the exact kernel 697 and 873, one
+// output column's weights at a time in every wavefront 340 and 3003; with a uniform g_idx 45 and 87).
 // Q, K and V of 2048 x 2048 at 16 rows: 10.0 us, the finish 3.4 and the bitmaps 9.5, against 504 us of the exact VALU
 // kernel (two launches) and seven host round trips to read g_idx.
 struct LinProj {
@@ -1404,32 +1407,49 @@ struct LinArgs {
   int batch, slices, chunks;
 };
 
-// The exact weight of column k (of the whole matrix) for output n, from memory (chunks with split K tiles, infinities or scales that are not
-// finite).
-__device__ __forceinline__ float lin_weight(const LinProj& a, int k, int n) {
-  const tris_compact3_payload& p = a.p;
-  const int N = p.outfeatures;
-  const int pr = k >> 5, bit = k & 31;
-  const int g = p.g_idx[k];
-  const uint64_t rp = g >= 0 && g < p.num_groups
-                          ? static_cast<uint64_t>(p.row_pack3[static_cast<int64_t>(n) * p.num_groups + g]) : 0ull;
-  const uint64_t cp = static_cast<uint64_t>(p.col_pack3[k]);
-  const uint32_t q1 = static_cast<uint32_t>(p.qweight1[static_cast<int64_t>(pr) * N + n]);
+// B operand of packed row pr, column n, straight from memory: the lane's 8 weights in mf_row_b's order, each with its own
+// column's group and salient columns in place (chunks with split K tiles, infinities or scales that are not finite).
+// q1, gw: the column's qweight1 and split words of the row.
+__device__ __forceinline__ f16x8 lin_exact_row(const tris_compact3_payload& p, int pr, int n, int kg, uint32_t q1,
+                                               uint32_t gw) {
+  const int N = p.outfeatures, G = p.num_groups;
   const uint32_t cm = static_cast<uint32_t>(p.c_map[pr]);
-  const auto prod = [&](int h) { return hmul_bits(static_cast<uint16_t>(cp >> (16 * h)), static_cast<uint16_t>(rp >> (16 * h))); };
-  const uint16_t neg1 = (q1 >> bit) & 1u ? 0u : 0x8000u;
-  if ((cm >> bit) & 1u) {
-    const int idx = p.qweight2_sparse_prefix[pr] + __popc(cm & ((1u << bit) - 1u));
-    const int row = idx >> 5;
-    const uint32_t q2 = row >= 0 && row < p.qweight2_sparse_rows
-                            ? static_cast<uint32_t>(p.qweight2_sparse[static_cast<int64_t>(row) * N + n]) : 0u;
-    const uint16_t neg2 = (q2 >> (idx & 31)) & 1u ? 0u : 0x8000u;
-    return h2f(hadd_bits(prod(0) ^ neg1, prod(1) ^ neg2));
+  const int64_t* const row = p.row_pack3 + static_cast<int64_t>(n) * G;
+  int g[8];
+  uint64_t cp[8], rp[8];
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {  // element i: column kg + 4 (i / 2) + 16 (i % 2) of the packed row
+    const int k = 32 * pr + kg + 4 * (i >> 1) + 16 * (i & 1);
+    g[i] = p.g_idx[k];
+    cp[i] = static_cast<uint64_t>(p.col_pack3[k]);
   }
-  const uint32_t gw = static_cast<uint32_t>(
-      a.decoded[(static_cast<int64_t>(pr >> 1) * ceil_div(N, kTileOut) + n / kTileOut) * kGrWords + (pr & 1) * kTileOut +
-                n % kTileOut]);
-  return h2f(((gw >> bit) & 1u ? prod(2) : prod(3)) ^ neg1);
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    const bool gv = g[i] >= 0 && g[i] < G;
+    const uint64_t v = static_cast<uint64_t>(row[gv ? g[i] : 0]);
+    rp[i] = gv ? v : 0ull;
+  }
+  uint32_t w[8];
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    const int bit = kg + 4 * (i >> 1) + 16 * (i & 1);
+    const auto prod = [&](int h) {
+      return hmul_bits(static_cast<uint16_t>(cp[i] >> (16 * h)), static_cast<uint16_t>(rp[i] >> (16 * h)));
+    };
+    const uint16_t neg1 = (q1 >> bit) & 1u ? 0u : 0x8000u;
+    uint16_t v = ((gw >> bit) & 1u ? prod(2) : prod(3)) ^ neg1;
+    if ((cm >> bit) & 1u) {
+      const int idx = p.qweight2_sparse_prefix[pr] + __popc(cm & ((1u << bit) - 1u));
+      const int r2 = idx >> 5;
+      const uint32_t q2 = r2 >= 0 && r2 < p.qweight2_sparse_rows
+                              ? static_cast<uint32_t>(p.qweight2_sparse[static_cast<int64_t>(r2) * N + n]) : 0u;
+      const uint16_t neg2 = (q2 >> (idx & 31)) & 1u ? 0u : 0x8000u;
+      v = hadd_bits(prod(0) ^ neg1, prod(1) ^ neg2);
+    }
+    w[i] = v;
+  }
+  return __builtin_bit_cast(f16x8, make_uint4(w[0] | (w[1] << 16), w[2] | (w[3] << 16), w[4] | (w[5] << 16),
+                                              w[6] | (w[7] << 16)));
 }
 
 template <int kRows, bool kSingle>
@@ -1481,12 +1501,8 @@ __global__ __launch_bounds__(kMfThreads) __attribute__((amdgpu_waves_per_eu(3, 8
   for (int m = 0; m < kRt; ++m) xr[m] = xs + (16 * m + i16 < rc ? 16 * m + i16 : 0) * mf_xstride(false);
   const int n[1] = {n0w + i16};
   f32x4 acc[1][kRt];
-  float scalar[kRows / kMfWaves];  // the scalar loop's sums: rows wave + 4 i, column ob * 64 + lane
-  bool any_split = false;
 #pragma unroll
   for (int m = 0; m < kRt; ++m) acc[0][m] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-  for (int i = 0; i < kRows / kMfWaves; ++i) scalar[i] = 0.0f;
   for (int c = c_lo; c < c_hi; ++c) {
     const int kc = c * kMfChunk;
     if (c > c_lo) __syncthreads();  // the previous chunk's readers are done
@@ -1559,31 +1575,18 @@ __global__ __launch_bounds__(kMfThreads) __attribute__((amdgpu_waves_per_eu(3, 8
       mf_q2_issue(q2, p.qweight2_sparse_rows, N, n[0], cm, q2w[0]);
       mf_compute<1, kRt, false>(q2, p.qweight2_sparse_rows, N, rank, kMfMaxGroups, kc, n, xr, lane, ch, cm, wb, q2w, acc);
     } else {  // uniform over the workgroup
-      any_split = true;
-      const int ns = ob * kTileOut + lane;
-      const int kn = rank - kc < kMfChunk ? rank - kc : kMfChunk;
-      for (int k = 0; k < kn && ns < N; ++k) {
-        const float w = lin_weight(lp, kc + k, ns);
-        const int pos = (k & ~31) + mf_perm32(k & 31);
+      const int npr = (rank - kc < kMfChunk ? rank - kc : kMfChunk) / 32;
+      const int nc = n[0] < N ? n[0] : N - 1;  // (columns past N are not stored)
+#pragma unroll 1
+      for (int j = 0; j < npr; ++j) {
+        const uint2 w = *reinterpret_cast<const uint2*>(wb + kMfWw + ((j >> 1) * kMfWCols + i16) * 4 + 2 * (j & 1));
+        const f16x8 bv = lin_exact_row(p, kc / 32 + j, nc, kg, w.x, w.y);
 #pragma unroll
-        for (int i = 0; i < kRows / kMfWaves; ++i) {
-          const int r = wave + kMfWaves * i;
-          if (r < rc) scalar[i] = fmaf(h2f(xs[r * mf_xstride(false) + pos]), w, scalar[i]);
+        for (int m = 0; m < kRt; ++m) {
+          const f16x8 av = __builtin_bit_cast(f16x8, *reinterpret_cast<const uint4*>(xr[m] + 32 * j + 8 * kg));
+          acc[0][m] = __builtin_amdgcn_mfma_f32_16x16x32_f16(av, bv, acc[0][m], 0, 0, 0);
         }
       }
-    }
-  }
-  if (any_split) {  // uniform: the scalar sums join the accumulators through LDS (the staged rows are done with)
-    static_assert(kRows * kTileOut * 4 <= sizeof(xs), "the scalar sums fit the staged rows");
-    float* const ex = reinterpret_cast<float*>(xs);
-    __syncthreads();
-#pragma unroll
-    for (int i = 0; i < kRows / kMfWaves; ++i) ex[(wave + kMfWaves * i) * kTileOut + lane] = scalar[i];
-    __syncthreads();
-#pragma unroll
-    for (int m = 0; m < kRt; ++m) {
-#pragma unroll
-      for (int v = 0; v < 4; ++v) acc[0][m][v] += ex[(16 * m + 4 * kg + v) * kTileOut + kMfWCols * wave + i16];
     }
   }
   float* const part = lp.part + (static_cast<int64_t>(sl) * a.batch + row0) * N;
