@@ -1385,7 +1385,7 @@ void grouped_mfma_kernel(MfmaArgs a) {
 // batch, up to three of them on one input.  A workgroup takes one 64-output tile, kRows rows and a run of 512-column
 // chunks (blockIdx.y = row tile x slice), stages each chunk as the decode kernel does, and leaves fp32 partial sums
 // [slice][batch][N]; linear_finish_kernel adds the slices in order, then the addend, scale and bias.  Slices are taken
-// until the launch fills the GPU.  The row scales are staged per K tile (the decode kernel's per group would not fit), and
+// until the launch fills the GPU; where the tiles alone do, there is one, and the workgroup writes the outputs itself.  The row scales are staged per K tile (the decode kernel's per group would not fit), and
 // whether every K tile of a chunk lies in one group is found on the way: a chunk where one does not (or with an
 // infinite activation, or a row scale that is not finite) builds its operands column by column from memory instead
 // (lin_exact_row), so no launch waits for the host to look at g_idx.  Bound by the loads of each column's scales: a
@@ -1396,7 +1396,7 @@ void grouped_mfma_kernel(MfmaArgs a) {
 struct LinProj {
   tris_compact3_payload p;
   const int32_t* decoded;  // [packed rows / 2][tiles][128]
-  float* part;             // [slices][batch][N]
+  float* part;             // [slices][batch][N] (null with one slice)
   const float* addend;     // [batch][N] or null
   uint16_t* out;           // [batch][N]
 };
@@ -1406,6 +1406,14 @@ struct LinArgs {
   const uint16_t* in_scale;  // [rank] or null
   int batch, slices, chunks;
 };
+
+// A sum's output, as the exact kernel ends: fp16((v + addend) * scale + bias).
+__device__ __forceinline__ void lin_store(const LinProj& lp, int64_t at, float v, float scale, float bias) {
+  if (lp.addend != nullptr) v += lp.addend[at];
+  if (lp.p.has_output_scale) v = v * scale;
+  if (lp.p.has_bias) v = v + bias;
+  lp.out[at] = f2h_bits(v);
+}
 
 // B operand of packed row pr, column n, straight from memory: the lane's 8 weights in mf_row_b's order, each with its own
 // column's group and salient columns in place (chunks with split K tiles, infinities or scales that are not finite).
@@ -1589,18 +1597,26 @@ __global__ __launch_bounds__(kMfThreads) __attribute__((amdgpu_waves_per_eu(3, 8
       }
     }
   }
-  float* const part = lp.part + (static_cast<int64_t>(sl) * a.batch + row0) * N;
+  const bool whole = a.slices == 1;  // the workgroup has the whole sums: no partial sums, no finishing launch
+  float* const part = whole ? nullptr : lp.part + (static_cast<int64_t>(sl) * a.batch + row0) * N;
+  const float scale = whole && p.has_output_scale && n[0] < N ? h2f(p.output_scale[n[0]]) : 1.0f;
+  const float bias = whole && p.has_bias && n[0] < N ? h2f(p.bias[n[0]]) : 0.0f;
 #pragma unroll
   for (int m = 0; m < kRt; ++m) {
 #pragma unroll
     for (int v = 0; v < 4; ++v) {
       const int r = 16 * m + 4 * kg + v;
-      if (r < rc && n[0] < N) part[static_cast<int64_t>(r) * N + n[0]] = acc[0][m][v];
+      if (r >= rc || n[0] >= N) continue;
+      if (whole) {
+        lin_store(lp, static_cast<int64_t>(row0 + r) * N + n[0], acc[0][m][v], scale, bias);
+      } else {
+        part[static_cast<int64_t>(r) * N + n[0]] = acc[0][m][v];
+      }
     }
   }
 }
 
-// out[b][n] = fp16((sum of the slices, in order, + addend) * scale + bias), as the exact kernel ends.
+// The outputs from the slices' sums, added in order (more than one slice).
 __global__ __launch_bounds__(256) void linear_finish_kernel(LinArgs a) {
   const LinProj& lp = a.proj[blockIdx.z];
   const tris_compact3_payload& p = lp.p;
@@ -1615,10 +1631,7 @@ __global__ __launch_bounds__(256) void linear_finish_kernel(LinArgs a) {
     float v = 0.0f;
 #pragma unroll 4
     for (int s = 0; s < a.slices; ++s) v += lp.part[s * step + at];
-    if (lp.addend != nullptr) v += lp.addend[at];
-    if (p.has_output_scale) v = v * scale;
-    if (p.has_bias) v = v + bias;
-    lp.out[at] = f2h_bits(v);
+    lin_store(lp, at, v, scale, bias);
   }
 }
 
@@ -2287,7 +2300,9 @@ int launch_grouped_mfma(const uint16_t* hidden_a, const uint16_t* hidden_b, int 
 }
 
 // Slices of a linear's K: chunks are split until one matrix's launch has about three workgroups a CU (whatever the number
-// of matrices, so that each gives the same bits alone and beside others of its width).
+// of matrices, so that each gives the same bits alone and beside others of its width).  With more than one slice there
+// are fewer than 1536 (tile, slice) pairs of at most 32 x 64 sums, so the partial sums stay below 12 MiB a matrix however
+// long the batch.
 static int lin_slices(int batch, int rank, int max_n) {
   const int chunks = ceil_div(rank, kMfChunk);
   const int64_t tiles = static_cast<int64_t>(ceil_div(max_n, kTileOut)) * ceil_div(batch, batch <= kMfRows ? kMfRows : 32);
@@ -2307,7 +2322,8 @@ int64_t linear_mfma_workspace(int batch, int rank, const int32_t* outfeatures, i
     words += lin_decoded_words(rank, outfeatures[i]);
     sums += static_cast<int64_t>(batch) * outfeatures[i];
   }
-  return 4 * (words + sums * lin_slices(batch, rank, max_n));
+  const int slices = lin_slices(batch, rank, max_n);
+  return 4 * (words + (slices > 1 ? sums * slices : 0));
 }
 
 // The matrix sizes linear_mfma_kernel takes: whole 64-column K tiles, every 32-bit buffer offset below 2 GiB.
@@ -2371,7 +2387,7 @@ int launch_linear_mfma(const uint16_t* input, int batch, const tris_compact3_pay
     wide = wide && mf_wide(probe);
   }
   float* sums = reinterpret_cast<float*>(words);
-  for (int i = 0; i < count; ++i) {
+  for (int i = 0; i < count && args.slices > 1; ++i) {
     args.proj[i].part = sums;
     sums += static_cast<int64_t>(args.slices) * batch * widths[i];
   }
@@ -2388,7 +2404,7 @@ int launch_linear_mfma(const uint16_t* input, int batch, const tris_compact3_pay
     part.x = input + static_cast<int64_t>(b0) * rank;
     part.batch = batch - b0 < per ? batch - b0 : per;
     for (int i = 0; i < count; ++i) {
-      part.proj[i].part = args.proj[i].part + static_cast<int64_t>(args.slices) * b0 * widths[i];
+      if (args.slices > 1) part.proj[i].part = args.proj[i].part + static_cast<int64_t>(args.slices) * b0 * widths[i];
       part.proj[i].out = args.proj[i].out + static_cast<int64_t>(b0) * widths[i];
       if (args.proj[i].addend != nullptr) part.proj[i].addend = args.proj[i].addend + static_cast<int64_t>(b0) * widths[i];
     }
@@ -2400,6 +2416,7 @@ int launch_linear_mfma(const uint16_t* input, int batch, const tris_compact3_pay
       if (wide) hipLaunchKernelGGL((linear_mfma_kernel<32, false>), grid, dim3(kMfThreads), 0, s, part);
       else hipLaunchKernelGGL((linear_mfma_kernel<32, true>), grid, dim3(kMfThreads), 0, s, part);
     }
+    if (args.slices == 1) continue;
     const int ty = part.batch < 4096 ? part.batch : 4096;
     hipLaunchKernelGGL(linear_finish_kernel, dim3(ceil_div(max_n, 256), ty, count), dim3(256), 0, s, part);
   }

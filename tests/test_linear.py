@@ -291,3 +291,51 @@ def test_linear_unused_scales_not_finite(tris, oracle_mod, cuda, batch):
     assert np.isfinite(want).all()
     got = _linear(ext, torch.from_numpy(x).to(cuda), _dev(m, cuda)).cpu().numpy()
     assert_close(got, want, f"unused scales, batch={batch}")
+
+
+def test_linears_workspace_is_bounded(tris):
+    """The linears' workspace holds the bitmaps, and partial sums only while the K slices fill the GPU: at most 12 MiB a
+    matrix above the bitmaps, none once the tiles do."""
+    import ctypes
+
+    from tris_moe_amd import _lib
+
+    size = _lib.load().tris_compact3_linears_workspace_bytes
+    for rank, n in ((2048, 2048), (4096, 4096), (14336, 1024), (640, 200)):
+        bitmaps = rank // 64 * -(-n // 64) * 512
+        for count in (1, 3):
+            widths = (ctypes.c_int32 * count)(*[n] * count)
+            for batch in (1, 16, 17, 64, 300, 1024, 4096, 100000, 1 << 20):
+                sums = size(batch, rank, widths, count) - count * bitmaps
+                assert 0 <= sums <= count * (12 << 20)
+                assert batch < 32768 or sums == 0
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("groups", ["uniform", "split", "infinite"])
+def test_linear_prompt_sizes(tris, oracle_mod, cuda, groups):
+    """Enough rows and columns that a workgroup takes both chunks of a matrix itself (no slices): the staging between
+    chunks, one chunk of two with split K tiles or with an infinity, scales and bias; the last row tile is ragged."""
+    from test_gpu_parity import assert_close, note
+
+    n, k, batch = 1540, 1024, 1010
+    note(f"compact3 linear prompt sizes groups={groups}")
+    ext = tris["ext"]
+    rng = np.random.default_rng(63)
+    gidx = np.arange(k) // 128
+    if groups == "split":
+        gidx[700:710] = 0  # the second chunk
+    proj = synthetic.make_projection(rng, 1, n, k, 0.15, rng.random(k).astype(np.float32) + 0.5, ext.gr_encode,
+                                     g_idx=gidx.astype(np.int32))
+    m = {key: np.ascontiguousarray(proj[key][0]) for key in MODULE_KEYS}
+    x = rng.standard_normal((batch, k)).astype(np.float16)
+    if groups == "infinite":
+        x[5, 17] = np.inf  # the first chunk
+    s_out, bias = (rng.random(n) * 2 + 0.25).astype(np.float16), rng.standard_normal(n).astype(np.float16)
+    t = lambda a: torch.from_numpy(np.ascontiguousarray(a)).to(cuda)
+    got = _linear(ext, t(x), _dev(m, cuda), None, t(s_out), t(bias)).cpu().numpy()
+    want = oracle_mod.compact3_linear(x, m, None, s_out, bias)
+    if groups == "infinite":
+        np.testing.assert_array_equal(got[5], want[5])
+        got, want = np.delete(got, 5, 0), np.delete(want, 5, 0)
+    assert_close(got, want, f"prompt sizes {groups}")
