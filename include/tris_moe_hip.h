@@ -690,8 +690,8 @@ int tris_compact3_dual_linear_forward(const uint16_t* input, int32_t batch, cons
  * compact3_linear_forward calls, TriSMoE_cuda.cpp:497-700) on the matrix cores: tris_compact3_linear_forward's results
  * up to the order of the fp32 sums, for any g_idx (512-column chunks with K tiles of several groups, with an
  * infinite activation or with a row scale that is not finite build their weights column by column on the device).  Every
- * payload has num_experts == 1 and the same rank, a multiple of 64; input and workspace are 16-byte aligned; input_scale
- * applies to all, addend to the first; outputs[i] fp16 [batch, outfeatures of payload i].  The workspace (of
+ * payload has num_experts == 1 and the same rank, a multiple of 64; input, input_scale and workspace are 16-byte aligned;
+ * input_scale applies to all, addend to the first; outputs[i] fp16 [batch, outfeatures of payload i].  The workspace (of
  * tris_compact3_linears_workspace_bytes bytes) holds the decoded split bitmaps and, while K is split to fill the GPU, fp32
  * partial sums (at most 12 MiB a matrix).  A matrix gives the
  * same bits alone and beside others of its output width (the split of K follows the widest).

@@ -2360,8 +2360,9 @@ int launch_linear_mfma(const uint16_t* input, int batch, const tris_compact3_pay
   }
   if (batch == 0) return TRIS_OK;
   TRIS_REQUIRE(input && workspace, "%s: null pointer", who);
-  TRIS_REQUIRE(reinterpret_cast<uintptr_t>(input) % 16 == 0 && reinterpret_cast<uintptr_t>(workspace) % 16 == 0,
-               "%s: input and workspace must be 16-byte aligned", who);
+  TRIS_REQUIRE(reinterpret_cast<uintptr_t>(input) % 16 == 0 && reinterpret_cast<uintptr_t>(input_scale) % 16 == 0 &&
+                   reinterpret_cast<uintptr_t>(workspace) % 16 == 0,
+               "%s: input, input_scale and workspace must be 16-byte aligned", who);
   const int rank = payloads[0].rank;
   TRIS_REQUIRE(workspace_bytes >= linear_mfma_workspace(batch, rank, widths, count), "%s: workspace too small", who);
   void* ids = nullptr;

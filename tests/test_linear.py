@@ -339,3 +339,22 @@ def test_linear_prompt_sizes(tris, oracle_mod, cuda, groups):
         np.testing.assert_array_equal(got[5], want[5])
         got, want = np.delete(got, 5, 0), np.delete(want, 5, 0)
     assert_close(got, want, f"prompt sizes {groups}")
+
+
+def test_linears_refuse_a_misaligned_input_scale(tris):
+    """The linears' C entry reads input_scale 16 bytes at a time: it refuses one off a 16-byte boundary (before it
+    touches any tensor, so the addresses here need not be real)."""
+    import ctypes
+
+    from tris_moe_amd import _lib
+
+    lib = _lib.load()
+    at = 1 << 20
+    pay = _lib.TrisPayload(1, 64, 64, 1, 1, 4, *[at] * 10, None, None, 0, 0, 1)
+    outs = (ctypes.c_void_p * 1)(at)
+    call = lambda scale: (lib.tris_compact3_linears_forward(at, 4, (_lib.TrisPayload * 1)(pay), 1, scale, None, outs, at,
+                                                            0, None), lib.tris_last_error().decode())
+    rc, msg = call(at + 2)
+    assert rc < 0 and "aligned" in msg
+    rc, msg = call(at)  # (the workspace is too small)
+    assert rc < 0 and "workspace too small" in msg
