@@ -2396,16 +2396,14 @@ int launch_linear_mfma(const uint16_t* input, int batch, const tris_compact3_pay
   if (rc) return rc;
   hipStream_t s = static_cast<hipStream_t>(stream);
   const int rows = batch <= kMfRows ? kMfRows : 32;
-  const int64_t y = static_cast<int64_t>(ceil_div(batch, rows)) * args.slices;
-  TRIS_REQUIRE(y < (int64_t{1} << 31), "%s: too many row tiles", who);
-  // (grid.y is limited to 65535: longer batches go in several launches of whole row tiles)
-  const int per = 65535 / args.slices * rows;
+  // grid.y is limited to 65535: longer batches go in several launches of whole row tiles (with more than one slice there
+  // are fewer than 1536 (tile, slice) pairs, so one launch)
+  const int per = args.slices > 1 ? batch : 65535 * rows;
   for (int b0 = 0; b0 < batch; b0 += per) {
     LinArgs part = args;
     part.x = input + static_cast<int64_t>(b0) * rank;
     part.batch = batch - b0 < per ? batch - b0 : per;
     for (int i = 0; i < count; ++i) {
-      if (args.slices > 1) part.proj[i].part = args.proj[i].part + static_cast<int64_t>(args.slices) * b0 * widths[i];
       part.proj[i].out = args.proj[i].out + static_cast<int64_t>(b0) * widths[i];
       if (args.proj[i].addend != nullptr) part.proj[i].addend = args.proj[i].addend + static_cast<int64_t>(b0) * widths[i];
     }

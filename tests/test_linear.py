@@ -358,3 +358,55 @@ def test_linears_refuse_a_misaligned_input_scale(tris):
     assert rc < 0 and "aligned" in msg
     rc, msg = call(at)  # (the workspace is too small)
     assert rc < 0 and "workspace too small" in msg
+
+
+@pytest.mark.gpu
+def test_linear_longer_than_one_launch(tris, oracle_mod, cuda):
+    """A batch past the row tiles of one launch (65535 of 32 rows) goes in two: rows at the start, on both sides of the
+    seam and at the ragged end are the oracle's."""
+    from test_gpu_parity import assert_close, note
+
+    n, k, seam = 64, 64, 65535 * 32
+    batch = seam + 33
+    note("compact3 linear in two launches")
+    ext = tris["ext"]
+    m = _modules(ext, 1, n, k, 71)[0][0]
+    x = torch.randn((batch, k), generator=torch.Generator(device=cuda).manual_seed(5), device=cuda).to(torch.float16)
+    rows = [0, 1, 31, 32, seam - 33, seam - 1, seam, seam + 1, seam + 31, seam + 32]
+    got = _linear(ext, x, _dev(m, cuda))
+    assert got.shape == (batch, n)
+    assert_close(got[rows].cpu().numpy(), oracle_mod.compact3_linear(x[rows].cpu().numpy(), m), "two launches")
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("batch", [3, 70])
+def test_exact_kernel_entries(tris, oracle_mod, cuda, batch):
+    """A rank that is no multiple of 64 takes the exact kernel in every entry: the single linear with scales, bias and the
+    null-space term, the dual linear, and Q / K / V (a pair and a single launch), with an uneven g_idx on one of them."""
+    from test_gpu_parity import assert_close, note
+
+    n, k = 136, 160
+    note(f"exact linears batch={batch}")
+    ext = tris["ext"]
+    mods, rng = _modules(ext, 3, n, k, 55)
+    mods[1]["g_idx"] = (np.arange(k) % 2).astype(np.int32)
+    dm = [_dev(m, cuda) for m in mods]
+    x = (rng.standard_normal((batch, k)) * 1.5).astype(np.float16)
+    t = lambda a: torch.from_numpy(np.ascontiguousarray(a)).to(cuda)
+    assert not ext._linears_ok(t(x), ())
+    args = lambda m: [m[key] for key in MODULE_KEYS]
+    dual = ext.compact3_dual_linear_forward(t(x), *args(dm[0]), *args(dm[1]))
+    biases = [rng.standard_normal(n).astype(np.float16) for _ in range(3)]
+    qkv = ext.compact3_qkv_linear_forward(t(x), *(a for m, b in zip(dm, biases) for a in [*args(m), t(b)]))
+    for i in range(3):
+        if i < 2:
+            assert_close(dual[i].cpu().numpy(), oracle_mod.compact3_linear(x, mods[i]), f"exact dual[{i}]")
+        assert_close(qkv[i].cpu().numpy(), oracle_mod.compact3_linear(x, mods[i], bias=biases[i]), f"exact qkv[{i}]")
+    s_in, s_out = (rng.random(k) + 0.5).astype(np.float16), (rng.random(n) * 2 + 0.25).astype(np.float16)
+    c2p, c1p = _ns(rng, n, k, 24, 32)
+    c2 = oracle_mod.packed4_dequant(c2p["qweight"], c2p["qzeros"], c2p["scales"], c2p["g_idx"], 24, k)
+    c1 = oracle_mod.packed4_dequant(c1p["qweight"], c1p["qzeros"], c1p["scales"], c1p["g_idx"], n, 24)
+    got = _linear(ext, t(x), dm[0], t(s_in), t(s_out), t(biases[0]),
+                  ns=({kk: t(v) for kk, v in c2p.items()}, {kk: t(v) for kk, v in c1p.items()}))
+    want = oracle_mod.compact3_linear(x, mods[0], s_in, s_out, biases[0], c2, c1)
+    assert_close(got.cpu().numpy(), want, "exact single with every extra")
