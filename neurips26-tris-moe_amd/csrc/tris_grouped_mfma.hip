@@ -1308,8 +1308,13 @@ void grouped_mfma_kernel(MfmaArgs a) {
       __builtin_amdgcn_sched_barrier(0);  // the loads stay ahead of the pass they overlap
       mf_compute<kNs, kRt, kCompact>(q2, q2rows, N, rank, G, 0, n, xr, ln, ch, cm, wb, q2w, acc);
       __builtin_amdgcn_sched_barrier(0);
+      // the words pass between lanes: the last pass's reads come before these writes, and the next pass's after
+      __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+      __builtin_amdgcn_wave_barrier();
 #pragma unroll
       for (int b = 0; b < 2; ++b) mf_wave_tile_write<kCompact>(wr[b], ln, wb + b * WW::kAlloc);
+      __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+      __builtin_amdgcn_wave_barrier();
     } else {
       for (int kc = 0; kc < rank; kc += kMfChunk) {
         if (ob > ob_begin || kc > 0) {
