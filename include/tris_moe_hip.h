@@ -130,7 +130,9 @@ int tris_route_topk(const float* router_logits, int32_t num_tokens, int32_t num_
  * Router softmax + top-k fused with the grouped route for decode-sized batches
  * (no reference counterpart: fuses F.softmax(router_logits, dtype=float),
  * torch.topk, the optional renormalisation and the routing-weight cast of
- * modeling_mixtral.py:548-555 with tris_build_grouped_route).  One launch.
+ * modeling_mixtral.py:548-555 with tris_build_grouped_route).  One launch up to 64
+ * tokens (72 for two picks and 80 for one of at most 64 experts), two above when
+ * selected_experts is given.
  * router_logits fp32 [num_tokens, num_experts]; top-k by probability with ties
  * to the lower expert id; weights renormalised over the k picks when
  * renormalize != 0.  routing_weights_f16 fp16 [num_tokens, top_k] (required),

@@ -881,14 +881,17 @@ static void launch_route_tokens(const RouteArgs& ra, hipStream_t s) {
   }
 }
 
-// More than one 64-token chunk: the one-workgroup router routes 16 tokens at a time and scatters a chunk at a time on
-// one CU, so the token-parallel softmax / top-k and the per-expert scatter take over (8 experts, top 2: 64 tokens 7.7
-// against 8.5 us, 333 tokens 26.5 against 9.1, 1000 tokens 71 against 10.6; 128 experts, top 8: 32 tokens 8.7 against
-// 9.6, 250 tokens 44 against 11.4).  The same outputs: both give each expert its tokens in order.
-constexpr int kRouteSmallMaxTokens = 64;
+// Tokens up to which the one-workgroup router is the faster one.  It routes 16 tokens at a time and scatters 64 at a time
+// on one CU; past that the token-parallel softmax / top-k and the per-expert scatter take over, a launch more.  The same
+// outputs: both give each expert its tokens in order.  One workgroup against two launches, us: 8 experts, top 1: 72 tokens
+// 7.4 / 8.3, 80 tokens 8.0 / 8.3, 96 tokens 8.9 / 8.2; top 2: 72 tokens 8.2 / 8.4, 80 tokens 9.0 / 8.4, 333 tokens
+// 26.5 / 9.1; top 4: 65 tokens 9.4 / 8.7; 128 experts: top 1, 72 tokens 8.5 / 8.5, top 8, 65 tokens 14.1 / 9.5.
+static int route_small_max_tokens(int num_experts, int top_k) {
+  return num_experts <= kWave && top_k <= 2 ? 88 - 8 * top_k : 64;
+}
 
 static int launch_route(const RouteArgs& ra, hipStream_t s, const char* who) {
-  if (ra.tokens > kRouteSmallMaxTokens && ra.selected != nullptr) {
+  if (ra.tokens > route_small_max_tokens(ra.num_experts, ra.top_k) && ra.selected != nullptr) {
     launch_route_tokens(ra, s);
     const int rc = check_launch(who);
     if (rc) return rc;

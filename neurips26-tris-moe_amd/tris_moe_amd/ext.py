@@ -281,7 +281,8 @@ def route_topk(router_logits: torch.Tensor, top_k: int, renormalize: bool):
 
 def route_topk_grouped(router_logits: torch.Tensor, top_k: int, renormalize: bool, m_tile: int = 4) -> dict:
     """Router softmax / top-k / renormalisation (modeling_mixtral.py:548-555) and the padded grouped
-    route in one launch, for decode-sized batches (an extension; see build_grouped_route_device).
+    route in one call, for up to 2048 routed rows (an extension; see build_grouped_route_device): one launch up to
+    64 tokens (72 for two picks and 80 for one of at most 64 experts), two above.
     Returns the route dict plus routing_weights_f16 [T, k], routing_weights [T, k] fp32 and
     selected_experts [T, k] int64."""
     logits, out = _route_topk_outputs(router_logits, top_k, "route_topk_grouped")

@@ -398,11 +398,31 @@ def test_route_topk_fused_matches_oracle(tris, oracle_mod, cuda, t, k, e, renorm
     np.testing.assert_array_equal(r["perm"].cpu().numpy()[inv], np.arange(t * k))
 
 
-@pytest.mark.parametrize("t,k,e,renorm", [(64, 2, 8, True), (65, 2, 8, True), (65, 8, 128, False), (333, 2, 8, True)])
+@pytest.mark.parametrize("t,k,e,renorm", [(64, 2, 8, True), (65, 2, 8, True), (65, 8, 128, False), (333, 2, 8, True),
+                                          (64, 4, 8, True), (65, 4, 8, True), (72, 2, 8, True), (73, 2, 60, True),
+                                          (80, 1, 64, True), (81, 1, 8, False), (65, 1, 65, True)])
 def test_route_topk_one_chunk_edge(tris, oracle_mod, cuda, t, k, e, renorm):
-    """The one-workgroup router up to 64 tokens and the two launches of tris_route_topk_grouped above: the same
-    exact route and weights, within the same bounds."""
+    """The one-workgroup router up to 64 tokens (72 for two picks and 80 for one of at most 64 experts) and the two
+    launches of tris_route_topk_grouped above: the same exact route and weights, within the same bounds."""
     test_route_topk_fused_matches_oracle(tris, oracle_mod, cuda, t, k, e, renorm)
+
+
+@pytest.mark.parametrize("t,k,e", [(200, 2, 8), (130, 8, 128)])
+def test_route_topk_without_selected_experts(tris, cuda, t, k, e):
+    """tris_route_topk_grouped with selected_experts NULL stays on one workgroup at any size, several 64-token scatter
+    chunks here: the outputs are those of the call that writes them."""
+    note(f"route topk without selected experts t={t} k={k} e={e}")
+    ext = tris["ext"]
+    from tris_moe_amd import _lib
+
+    logits = torch.from_numpy(np.random.default_rng(t).standard_normal((t, e)).astype(np.float32)).to(cuda)
+    want = ext.route_topk_grouped(logits, k, True, 4)
+    got = {key: torch.full_like(v, -7) for key, v in want.items()}
+    args = list(ext._route_topk_args(logits, got, k, True, 4))
+    args[8] = None  # selected_experts
+    _lib.check(_lib.load().tris_route_topk_grouped(*args, ext._stream(logits)), "route")
+    for key, v in want.items():
+        assert torch.equal(got[key], v) or key == "selected_experts", key
 
 
 @pytest.mark.parametrize("t,k,e,renorm", [(2048, 2, 8, True), (1024, 8, 256, True), (3000, 1, 64, False),
