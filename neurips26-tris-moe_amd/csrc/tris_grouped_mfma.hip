@@ -205,8 +205,9 @@ constexpr int kMfTbWords = kMfTbRs + kTileOut * kMfMaxGroups * 2;
 static_assert(kMfTbGw % 4 == 0 && kMfTbRs % 4 == 0, "tile buffer pieces must be 16-byte aligned");
 constexpr int kMfCus = 256;  // MI355X compute units
 constexpr int kMfTallMinRows = 12;  // mean rows a segment from which the decode kernel takes 32- or 64-row tiles
+constexpr int kMfTallMinRowsSingle = 17;
 // Decode kernel: row-scale groups and salient slots per chunk its LDS holds; the compact variant (at most 4
-// groups and 64 salient columns per expert) fits four workgroups per CU.
+// groups and 64 salient columns per expert, a rank of at most 256) stages half the columns.
 constexpr int mf_groups_cap(bool compact) { return compact ? 4 : kMfMaxGroups; }
 constexpr int mf_sal_slots(bool compact) { return compact ? 64 : kMfChunk; }
 constexpr int mf_chunk(bool compact) { return compact ? kMfChunk / 2 : kMfChunk; }  // K columns staged
@@ -1038,18 +1039,19 @@ __device__ __forceinline__ void mf_compute(const uint32_t* q2, int q2rows, int N
 }
 
 // Workgroup = kUnits units of 4 wavefronts.  The grid is sized to what the GPU holds at once, and the
-// workgroups share the (row tile, output tile) pairs evenly: with R row tiles (tiles of <= 16 rows of one
-// segment) and W = gridDim.x workgroups, each row tile gets W / R (or one more) workgroups that split its
-// output tiles into runs; with R > W, workgroup w takes row tiles w, w + W, ... whole.
+// workgroups share the (row tile, output tile) pairs evenly, row-tile major (a row tile is up to kRows rows of one
+// segment): as long as there are enough workgroups, each row tile's output tiles are split into runs, else all pairs are,
+// and a run may go on in the next row tile.
 // kUnits == 1: one projection (blockIdx.z picks it when two are given, unfused).
 // kUnits == 2: unit 0 computes the gate and unit 1 the up projection of the same tiles, side by side;
 // the output is fp16(silu(g) * u).
 // Along a run the units compute two output tiles at a time (mf_compute) while the next two tiles' weight words are
-// in flight to registers.  With more than one 512-column chunk (rank > 512) the chunk data is restaged per tile and
-// nothing is prefetched.
-// Registers are capped at what the LDS lets reside anyway: one unit with 4 staged rows fits four workgroups per CU
-// (128 VGPRs), with 16 rows three.
-// Wavefronts a SIMD each instance is held to: what its LDS lets reside anyway.
+// in flight to registers.  kSingle: weight words loaded one at a time (column counts that are no multiple of 4, misaligned
+// tensors).  kChunks: more than one 512-column chunk (rank > 512), staged in turn for each two tiles, with nothing in
+// flight meanwhile.  Both ran one tile a pass, word by word and restaged for every tile: SwiGLU launch of 8 segments of 33
+// rows, N = 8194, rank 512: 85.8 -> 49.4 us; 4 segments of 33, N = 2048, rank 576: 22.6 -> 16.4.
+// Wavefronts a SIMD each instance is held to: what its LDS lets reside anyway (one unit: three workgroups a CU, with 32
+// staged rows of 512 columns two).
 constexpr int mf_waves(int units, int rows, bool compact) {
   return units == 2 ? 2 : (rows > kMfRows && !compact ? 2 : 3);
 }
@@ -1065,7 +1067,7 @@ __device__ __forceinline__ uint32_t mf_div(uint32_t a, uint32_t b) {
   return static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(q));
 }
 
-template <int kUnits, int kRows, bool kCompact, bool kGeneral>
+template <int kUnits, int kRows, bool kCompact, bool kSingle, bool kChunks>
 __global__ __launch_bounds__(kUnits * kMfThreads)
 __attribute__((amdgpu_waves_per_eu(mf_waves(kUnits, kRows, kCompact), 8)))
 void grouped_mfma_kernel(MfmaArgs a) {
@@ -1196,7 +1198,7 @@ void grouped_mfma_kernel(MfmaArgs a) {
   const int ds = a.decoded_by_expert ? e : s;  // the decoded bitmaps' slot
   // activations from partial sums: only the 4-row instances carry that staging (the host sends at most 4 rows),
   // so the others keep no register for it across their tile loop
-  const bool part = kRows == 4 && pa.partials != nullptr;
+  const bool part = kRows == 4 && !kChunks && pa.partials != nullptr;
   if (e < 0 || e >= num_experts) {  // rows routed to no expert: zero output
     if (unit == 0) {
       const int span = (ob_end - ob_begin) * kTileOut;
@@ -1234,14 +1236,15 @@ void grouped_mfma_kernel(MfmaArgs a) {
     MfRowRegs<kRows, kCompact> rows;
     mf_cols_issue<kCompact>(pa, e, 0, utid, cols);
     mf_rows_issue<kRows, kCompact>(r_hid, rank, 0, wave, ln, roff, tok0, rows);
-    mf_wave_tile_issue<kCompact, kGeneral>(src, G, ob_begin, ln, wr[0]);
-    mf_wave_tile_issue<kCompact, kGeneral>(src, G, ob_begin + 1, ln, wr[1], !kGeneral && ob_begin + 1 < ob_end);
+    mf_wave_tile_issue<kCompact, kSingle>(src, G, ob_begin, ln, wr[0]);
+    const bool two = !(kSingle || kChunks) || ob_begin + 1 < ob_end;  // uniform
+    if (two) mf_wave_tile_issue<kCompact, kSingle>(src, G, ob_begin + 1, ln, wr[1], ob_begin + 1 < ob_end);
     mf_cols_write<kCompact>(pa, rc, 0, utid, ch, cols, kSal);
     if (!part) mf_rows_write<kRows, kCompact>(rows, rc, wave, ln, ch.xs);
     if (part) mf_partials_stage<kCompact>(pa, row0, rc, utid, ch);  // one chunk (host-checked)
     cm = mf_chunk_meta(cols, kSal);
     mf_wave_tile_write<kCompact>(wr[0], ln, wb);
-    mf_wave_tile_write<kCompact>(wr[1], ln, wb + WW::kAlloc);
+    if (two) mf_wave_tile_write<kCompact>(wr[1], ln, wb + WW::kAlloc);
     __syncthreads();
   }
   // The outputs of rows 16 m .. of tile ob, from their accumulators.  Stores go through a buffer resource over the
@@ -1298,12 +1301,12 @@ void grouped_mfma_kernel(MfmaArgs a) {
       for (int m = 0; m < kRt; ++m) acc[b][m] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
       n[b] = (ob + b) * kTileOut + 16 * wave + i16;
     }
-    if constexpr (!kGeneral) {
+    if constexpr (!kChunks) {
 #pragma unroll
       for (int b = 0; b < kNs; ++b) mf_q2_issue(q2, q2rows, N, n[b], cm, q2w[b]);
 #pragma unroll
       for (int b = 0; b < 2; ++b) {
-        mf_wave_tile_issue<kCompact, kGeneral>(src, G, ob + kNs + b, ln, wr[b], ob + kNs + b < ob_end);
+        mf_wave_tile_issue<kCompact, kSingle>(src, G, ob + kNs + b, ln, wr[b], ob + kNs + b < ob_end);
       }
       __builtin_amdgcn_sched_barrier(0);  // the loads stay ahead of the pass they overlap
       mf_compute<kNs, kRt, kCompact>(q2, q2rows, N, rank, G, 0, n, xr, ln, ch, cm, wb, q2w, acc);
@@ -1316,21 +1319,27 @@ void grouped_mfma_kernel(MfmaArgs a) {
       __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
       __builtin_amdgcn_wave_barrier();
     } else {
+      // (the next chunk's loads in flight during this one's pass made every launch 2 to 10% longer: spilled registers and
+      // more instructions to fetch)
       for (int kc = 0; kc < rank; kc += kMfChunk) {
         if (ob > ob_begin || kc > 0) {
           __syncthreads();  // the previous chunk's readers are done
           MfColRegs cols;
           MfRowRegs<kRows, kCompact> rows;
-          mf_wave_tile_issue<kCompact, kGeneral>(mf_wave_src<kCompact>(pa, ds, e, kc, wave, ln), G, ob, ln, wr[0]);
           mf_cols_issue<kCompact>(pa, e, kc, utid, cols);
           mf_rows_issue<kRows, kCompact>(r_hid, rank, kc, wave, ln, roff, tok0, rows);
+          const MfWaveSrc at = mf_wave_src<kCompact>(pa, ds, e, kc, wave, ln);
+#pragma unroll
+          for (int b = 0; b < kNs; ++b) mf_wave_tile_issue<kCompact, kSingle>(at, G, ob + b, ln, wr[b]);
           mf_cols_write<kCompact>(pa, rc, kc, utid, ch, cols, kSal);
-          if (!part) mf_rows_write<kRows, kCompact>(rows, rc, wave, ln, ch.xs);  // (partial sums: one chunk, staged already)
+          mf_rows_write<kRows, kCompact>(rows, rc, wave, ln, ch.xs);
           cm = mf_chunk_meta(cols, kSal);
-          mf_wave_tile_write<kCompact>(wr[0], ln, wb);
+#pragma unroll
+          for (int b = 0; b < kNs; ++b) mf_wave_tile_write<kCompact>(wr[b], ln, wb + b * WW::kAlloc);
           __syncthreads();
         }
-        mf_q2_issue(q2, q2rows, N, n[0], cm, q2w[0]);
+#pragma unroll
+        for (int b = 0; b < kNs; ++b) mf_q2_issue(q2, q2rows, N, n[b], cm, q2w[b]);
         mf_compute<kNs, kRt, kCompact>(q2, q2rows, N, rank, G, kc, n, xr, ln, ch, cm, wb, q2w, acc);
       }
     }
@@ -1362,15 +1371,13 @@ void grouped_mfma_kernel(MfmaArgs a) {
   // the run's output tiles, two at a time, with as many row sub-tiles as the row tile's rows need
   auto run = [&](auto nrt) {
     for (int ob = ob_begin; ob < ob_end;) {
-      if constexpr (!kGeneral) {
-        if (ob + 1 < ob_end) {
-          tiles(std::integral_constant<int, 2>{}, nrt, ob);
-          ob += 2;
-          continue;
-        }
+      if (ob + 1 < ob_end) {
+        tiles(std::integral_constant<int, 2>{}, nrt, ob);
+        ob += 2;
+      } else {
+        tiles(std::integral_constant<int, 1>{}, nrt, ob);
+        ob += 1;
       }
-      tiles(std::integral_constant<int, 1>{}, nrt, ob);
-      ob += 1;
     }
   };
   if (kRows <= 16 || rc <= 16) {  // uniform
@@ -1657,7 +1664,7 @@ constexpr int kWsSalWindows = 2;  // salient columns per item <= 64
 // rows 240 / 243.  The general decode instance (16-row tiles) hands over earlier.
 constexpr int kWsMinRows = 120;
 constexpr int kWsMinRowsCompact = 500;
-constexpr int kWsMinRowsGeneral = 64;
+constexpr int kWsMinRowsSingle = 64;
 #ifndef TRIS_WS_SUB
 #define TRIS_WS_SUB 2
 #endif
@@ -2244,12 +2251,10 @@ int launch_grouped_mfma(const uint16_t* hidden_a, const uint16_t* hidden_b, int 
     return p->num_groups <= mf_groups_cap(true) && p->qweight2_sparse_rows * kMfSalWin <= mf_sal_slots(true) &&
            p->rank <= kMfChunk / 2;
   };
-  const bool compact = compact_ok(pa) && (!pb || compact_ok(pb));
-  // more than one chunk (rank > 512), or columns that 16-byte loads do not fit: the general instance, which computes
-  // a tile at a time and loads nothing ahead
-  const bool general = pa->rank > kMfChunk || !mf_wide(args.proj[0]) ||
-                       (pb && (pb->rank > kMfChunk || !mf_wide(args.proj[1])));
-  const int ws_min = general ? kWsMinRowsGeneral : (compact ? kWsMinRowsCompact : kWsMinRows);
+  const bool chunks = pa->rank > kMfChunk || (pb && pb->rank > kMfChunk);  // more than one 512-column chunk
+  const bool single = !mf_wide(args.proj[0]) || (pb && !mf_wide(args.proj[1]));  // weight words loaded one at a time
+  const bool compact = !single && compact_ok(pa) && (!pb || compact_ok(pb));
+  const int ws_min = single ? kWsMinRowsSingle : (compact ? kWsMinRowsCompact : kWsMinRows);
   // long segments: keep each output tile's weights in registers and stream the segment's rows through them
   // (its buffer resources address a segment's rows in 32-bit byte offsets: the whole batch must stay below 2 GiB)
   if (partials == nullptr && num_segments <= kWave &&
@@ -2261,10 +2266,10 @@ int launch_grouped_mfma(const uint16_t* hidden_a, const uint16_t* hidden_b, int 
   // Staged activation rows: a row tile has at most min(row tile, batch).  From kMfTallMinRows rows a segment on average,
   // row tiles of 32 rows (64 at rank <= 256, where they take half the LDS): a segment then rarely needs two, and its
   // weights are built once, not once every 16 rows.
-  const bool tall = !general && partials == nullptr &&
-                    static_cast<int64_t>(batch) >= static_cast<int64_t>(kMfTallMinRows) * num_segments;
-  const int rows = general ? (partials != nullptr ? 4 : kMfRows) : (batch <= 4 ? 4 : (!tall ? kMfRows : (compact ? 64 : 32)));
-  const int lds_total = mf_static_lds_bytes(units, rows, compact && !general);
+  const int64_t tall_min = single ? kMfTallMinRowsSingle : kMfTallMinRows;
+  const bool tall = !chunks && partials == nullptr && static_cast<int64_t>(batch) >= tall_min * num_segments;
+  const int rows = batch <= 4 ? 4 : (!tall ? kMfRows : (compact ? 64 : 32));
+  const int lds_total = mf_static_lds_bytes(units, rows, compact);
   TRIS_REQUIRE(lds_total <= 160 * 1024, "%s: LDS request %d exceeds a CU", who, lds_total);
   // Workgroups: as many as the GPU holds at once (LDS and the kernel's registers, mf_waves, bound them), shared by the
   // projections of an unfused pair.
@@ -2280,25 +2285,28 @@ int launch_grouped_mfma(const uint16_t* hidden_a, const uint16_t* hidden_b, int 
   if (comb_out != nullptr && ceil_div(max_n, kTileOut) < wgs) wgs = ceil_div(max_n, kTileOut);  // output tiles only
   const dim3 grid(wgs > 0 ? wgs : 1, 1, nproj);
   const dim3 block(units * kMfThreads);
-#define TRIS_MF_LAUNCH(U, ROWS, C, M) hipLaunchKernelGGL((grouped_mfma_kernel<U, ROWS, C, M>), grid, block, 0, s, args)
-  if (units == 2) {
-    if (general && rows == 4) TRIS_MF_LAUNCH(2, 4, false, true);
-    else if (general) TRIS_MF_LAUNCH(2, kMfRows, false, true);
-    else if (rows == 4 && compact) TRIS_MF_LAUNCH(2, 4, true, false);
-    else if (rows == 4) TRIS_MF_LAUNCH(2, 4, false, false);
-    else if (rows == 64) TRIS_MF_LAUNCH(2, 64, true, false);
-    else if (rows == 32) TRIS_MF_LAUNCH(2, 32, false, false);
-    else if (compact) TRIS_MF_LAUNCH(2, kMfRows, true, false);
-    else TRIS_MF_LAUNCH(2, kMfRows, false, false);
+#define TRIS_MF_LAUNCH(ROWS, C, S, M)                                                                        \
+  do {                                                                                                       \
+    if (units == 2) hipLaunchKernelGGL((grouped_mfma_kernel<2, ROWS, C, S, M>), grid, block, 0, s, args);    \
+    else hipLaunchKernelGGL((grouped_mfma_kernel<1, ROWS, C, S, M>), grid, block, 0, s, args);               \
+  } while (0)
+  if (chunks) {
+    if (rows == 4 && single) TRIS_MF_LAUNCH(4, false, true, true);
+    else if (rows == 4) TRIS_MF_LAUNCH(4, false, false, true);
+    else if (single) TRIS_MF_LAUNCH(kMfRows, false, true, true);
+    else TRIS_MF_LAUNCH(kMfRows, false, false, true);
+  } else if (single) {
+    if (rows == 4) TRIS_MF_LAUNCH(4, false, true, false);
+    else if (rows == 32) TRIS_MF_LAUNCH(32, false, true, false);
+    else TRIS_MF_LAUNCH(kMfRows, false, true, false);
+  } else if (compact) {
+    if (rows == 4) TRIS_MF_LAUNCH(4, true, false, false);
+    else if (rows == 64) TRIS_MF_LAUNCH(64, true, false, false);
+    else TRIS_MF_LAUNCH(kMfRows, true, false, false);
   } else {
-    if (general && rows == 4) TRIS_MF_LAUNCH(1, 4, false, true);
-    else if (general) TRIS_MF_LAUNCH(1, kMfRows, false, true);
-    else if (rows == 4 && compact) TRIS_MF_LAUNCH(1, 4, true, false);
-    else if (rows == 4) TRIS_MF_LAUNCH(1, 4, false, false);
-    else if (rows == 64) TRIS_MF_LAUNCH(1, 64, true, false);
-    else if (rows == 32) TRIS_MF_LAUNCH(1, 32, false, false);
-    else if (compact) TRIS_MF_LAUNCH(1, kMfRows, true, false);
-    else TRIS_MF_LAUNCH(1, kMfRows, false, false);
+    if (rows == 4) TRIS_MF_LAUNCH(4, false, false, false);
+    else if (rows == 32) TRIS_MF_LAUNCH(32, false, false, false);
+    else TRIS_MF_LAUNCH(kMfRows, false, false, false);
   }
 #undef TRIS_MF_LAUNCH
   return check_launch(who);

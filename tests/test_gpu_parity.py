@@ -764,6 +764,15 @@ def test_predecoded_long_segments(tris, oracle_mod, cuda, drop):
     (448, 68, [20, 40, 1, 33]),
     (512, 66, [20, 40, 1, 33]),                                    # columns no multiple of 4: the general instance
     (576, 128, [5, 33, 20]),                                       # more than one chunk
+    (512, 66, [5, 9]),                                             # columns no multiple of 4: 16-row tiles, 4-row tiles
+    (512, 130, [1, 2]),
+    (576, 130, [5, 33, 20]),                                       # the same with more than one chunk
+    (640, 128, [1, 2]),
+    (512, 6400, [20, 40, 33, 1]),                                  # runs of several tiles a workgroup, odd ones among them
+    (512, 6402, [20, 40, 33, 1]),
+    (256, 6400, [64, 100, 33, 1]),
+    (576, 6400, [20, 40, 33, 1]),
+    (576, 6402, [1, 2]),
 ], ids=lambda v: str(v) if isinstance(v, int) else f"{len(v)}seg")
 def test_predecoded_row_tiles(tris, oracle_mod, cuda, rank, n, segs):
     """Segments around the decode GEMM's row tiles (16, 32 and 64 rows, chosen by the mean rows a segment and the
