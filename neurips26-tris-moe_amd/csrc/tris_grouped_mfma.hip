@@ -1304,20 +1304,27 @@ void grouped_mfma_kernel(MfmaArgs a) {
     if constexpr (!kChunks) {
 #pragma unroll
       for (int b = 0; b < kNs; ++b) mf_q2_issue(q2, q2rows, N, n[b], cm, q2w[b]);
+      // the next tiles' words, if any (uniform; the one-unit 64-row instance always loads and writes two tiles, of zeros
+      // at the end: at its register limit the branch spills, and A3B's 64-row segments took 10 to 25% longer)
+      const bool more = (kUnits == 1 && kRows == 64) || ob + kNs < ob_end;
+      if (more) {
 #pragma unroll
-      for (int b = 0; b < 2; ++b) {
-        mf_wave_tile_issue<kCompact, kSingle>(src, G, ob + kNs + b, ln, wr[b], ob + kNs + b < ob_end);
+        for (int b = 0; b < 2; ++b) {
+          mf_wave_tile_issue<kCompact, kSingle>(src, G, ob + kNs + b, ln, wr[b], ob + kNs + b < ob_end);
+        }
       }
       __builtin_amdgcn_sched_barrier(0);  // the loads stay ahead of the pass they overlap
       mf_compute<kNs, kRt, kCompact>(q2, q2rows, N, rank, G, 0, n, xr, ln, ch, cm, wb, q2w, acc);
       __builtin_amdgcn_sched_barrier(0);
-      // the words pass between lanes: the last pass's reads come before these writes, and the next pass's after
-      __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-      __builtin_amdgcn_wave_barrier();
+      if (more) {
+        // the words pass between lanes: the last pass's reads come before these writes, and the next pass's after
+        __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+        __builtin_amdgcn_wave_barrier();
 #pragma unroll
-      for (int b = 0; b < 2; ++b) mf_wave_tile_write<kCompact>(wr[b], ln, wb + b * WW::kAlloc);
-      __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-      __builtin_amdgcn_wave_barrier();
+        for (int b = 0; b < 2; ++b) mf_wave_tile_write<kCompact>(wr[b], ln, wb + b * WW::kAlloc);
+        __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+      }
     } else {
       // (the next chunk's loads in flight during this one's pass made every launch 2 to 10% longer: spilled registers and
       // more instructions to fetch)
