@@ -356,6 +356,17 @@ int tris_grouped_dual_forward_block_gr_predecoded_rows(
     const int32_t* expert_ids, const int32_t* segment_offsets, int32_t num_segments, int64_t total_problem_tiles,
     const int32_t* decoded_a, const int32_t* decoded_b, const tris_compact3_payload* payload_a,
     const tris_compact3_payload* payload_b, uint16_t* output_a, uint16_t* output_b, void* stream);
+
+/*
+ * The kernel that the predecoded MFMA entries pick for a launch of these sizes: 1 the weight-stationary one, which keeps
+ * an output tile's weights in registers and streams a segment's rows through them (and would rather have them
+ * materialised than gathered through a row index), 0 the decode one.  Of two projections (swiglu: fused) each size is the
+ * larger one's; wide: outfeatures is a multiple of 4 and qweight1, row_pack3 and the decoded words are 16-byte aligned.
+ * A caller can ask before it decides whether to gather.
+ */
+int tris_grouped_predecoded_weight_stationary(int32_t rank, int32_t outfeatures, int32_t num_groups,
+                                              int32_t qweight2_sparse_rows, int32_t wide, int32_t projections,
+                                              int32_t swiglu, int32_t gathered, int64_t rows, int32_t segments);
 int tris_grouped_swiglu_forward_block_gr_predecoded_rows(
     const uint16_t* hidden_gate, const uint16_t* hidden_up, const int64_t* row_index, int32_t hidden_rows,
     int32_t batch, const int32_t* expert_ids, const int32_t* segment_offsets, int32_t num_segments,

@@ -1664,14 +1664,6 @@ __global__ __launch_bounds__(256) void linear_finish_kernel(LinArgs a) {
 // of LDS reads per clock on a CU (4 SIMDs), twice what the LDS delivers.  kUnits == 2 runs the gate and up
 // projections of the same item side by side and writes fp16(silu(g) * u).
 constexpr int kWsSalWindows = 2;  // salient columns per item <= 64
-// Mean rows per active segment from which the host picks this kernel: below, the decode kernel's row tiles of 32 rows
-// (64 at rank <= 256), which rebuild the operands for each row tile but start at once, are faster.  Gate/up + down
-// launches, decode against weight-stationary: rank 512 (Mixtral) at 83 rows 109 against 130 us, 112 rows 135 / 142, 130
-// rows 153 / 149, 150 rows 167 / 155; rank 256 (OLMoE) at 75 rows 63 / 109, 125 rows 83 / 129, 250 rows 132 / 171, 500
-// rows 240 / 243.  The general decode instance (16-row tiles) hands over earlier.
-constexpr int kWsMinRows = 120;
-constexpr int kWsMinRowsCompact = 500;
-constexpr int kWsMinRowsSingle = 64;
 #ifndef TRIS_WS_SUB
 #define TRIS_WS_SUB 2
 #endif
@@ -2172,15 +2164,112 @@ static int launch_grouped_mfma_ws(const MfmaArgs& args, int units, int nproj, in
   return check_launch(who);
 }
 
-static bool ws_fits(const tris_compact3_payload* p) {
-  return p->rank <= kMfChunk && p->qweight2_sparse_rows <= kWsSalWindows && !p->has_output_scale && !p->has_bias;
-}
-
 // The decode kernel may load a projection's weight words 16 bytes at a time: 16-byte aligned tensors and a column
 // count that is a multiple of 4, so that no load straddles a row's or the tensor's end.
 static bool mf_wide(const MfmaProj& p) {
   const auto al = [](const void* q) { return reinterpret_cast<uintptr_t>(q) % 16 == 0; };
   return p.p.outfeatures % 4 == 0 && al(p.p.qweight1) && al(p.p.row_pack3) && al(p.decoded);
+}
+
+// Workgroups of a decode launch: as many as the GPU holds at once (LDS and the kernel's registers, mf_waves, bound them),
+// shared by the projections of an unfused pair.
+static int mf_workgroups(int units, int rows, bool compact, int nproj) {
+  int per_cu = (160 * 1024) / mf_static_lds_bytes(units, rows, compact);
+  const int by_regs = units == 1 ? mf_waves(units, rows, compact) : 1;
+  per_cu = per_cu < by_regs ? per_cu : by_regs;
+  return kMfCus * (per_cu > 0 ? per_cu : 1) / nproj;
+}
+
+// The sizes of a predecoded launch that pick its kernel (of a pair: the larger of the two).
+struct MfShape {
+  int rank, n, groups, q2rows;
+  bool single;    // weight words one at a time (mf_wide does not hold)
+  bool swiglu;    // the pair side by side (two units)
+  bool gathered;  // rows read through row_index
+  int nproj;      // projections of one unit each
+};
+
+// The compact LDS layout: a chunk of 256 columns (rank <= 256), at most 4 row-scale groups and 64 salient columns per
+// expert.  The 64-row tiles fit in it three workgroups a CU.
+static bool mf_compact(const MfShape& h) {
+  return !h.single && h.groups <= mf_groups_cap(true) && h.q2rows * kMfSalWin <= mf_sal_slots(true) &&
+         h.rank <= kMfChunk / 2;
+}
+
+// Whether a launch goes weight-stationary.  Up to 64 rows a segment on average the decode kernel always is the faster one,
+// from 120 rows on (500 in the compact layout) the weight-stationary one.  Between them neither is, by up to 1.4 (64
+// segments of 65 rows, N = 512, rank 512, SwiGLU: 39 against 28 us) and 0.58 (8 of 65, N = 2048, single: 13 against 21):
+// the weight-stationary kernel pays for each item a workgroup touches (building its operands) and little for the rows,
+// the decode kernel for each pair of a 32- or 64-row tile and an output tile, and both wait for the workgroup with the
+// most of them.  So their times are estimated, us = constant + cost x that workgroup's count with the costs' parts
+// proportional to the rank apart, fitted over 769 launches of 1 to 64 segments, N 512 to 14336, ranks 64 to 512 (90 with
+// gathered rows): the one picked is at most 3% slower than weight-stationary ever was there, 20% faster in the mean (25%
+// in the compact layout), and 0.5% slower in the mean than always the better one.  Single-word launches, which no size
+// here covers, keep the weight-stationary kernel from 64 rows.
+constexpr int kWsMinRows = 64;
+constexpr int kWsAlwaysRows = 120;
+constexpr int kWsAlwaysRowsCompact = 500;
+struct MfCost {
+  float ws, build, build_k, row, row_k;  // weight-stationary: constant, an item, 16 rows of one (_k: times rank / 512)
+  float dec, tile, tile_k;               // decode: constant, a pair of a row tile and an output tile
+};
+constexpr MfCost kMfCost[3][2] = {
+    // one unit                                                    SwiGLU
+    {{10.4f, 2.1f, 4.5f, 1.65f, 0.45f, 6.0f, 0.8f, 2.6f}, {7.7f, 5.9f, 5.2f, 1.46f, 0.41f, 6.9f, 1.3f, 2.8f}},
+    {{7.6f, 6.0f, 5.7f, 0.73f, 0.82f, 7.2f, 2.0f, 4.0f}, {8.0f, 6.3f, 6.0f, 1.08f, 0.79f, 7.0f, 2.2f, 2.9f}},  // compact
+    {{7.7f, -0.4f, 12.9f, 2.67f, -0.72f, 6.0f, 0.8f, 2.6f}, {5.6f, -2.9f, 18.8f, 3.45f, -1.46f, 6.9f, 1.3f, 2.8f}},  // gathered
+};
+
+static bool mf_weight_stationary(const MfShape& h, int64_t batch, int segments) {
+  if (segments < 1 || segments > kWave || batch < int64_t{kWsMinRows} * segments) return false;
+  // one chunk, the salient windows it holds, and 32-bit byte offsets over the whole batch
+  if (h.rank > kMfChunk || h.q2rows > kWsSalWindows || batch * h.n * 2 >= (int64_t{1} << 31) ||
+      batch * kMfChunk * 2 >= (int64_t{1} << 31)) {
+    return false;
+  }
+  if (h.single) return true;
+  const bool compact = mf_compact(h);
+  if (batch >= int64_t{compact ? kWsAlwaysRowsCompact : kWsAlwaysRows} * segments) return true;
+  if (compact && h.gathered) return false;  // gathering costs the weight-stationary kernel more than its rows save
+  const MfCost& c = kMfCost[compact ? 1 : h.gathered ? 2 : 0][h.swiglu ? 1 : 0];
+  const float f = static_cast<float>(h.rank) / 512.0f;
+  const int nob = ceil_div(h.n, kTileOut);
+  const int64_t mean = (batch + segments - 1) / segments;
+  // weight-stationary: `items` shared by W workgroups in equal parts, p / q items each: the unluckiest starts (q - 1) / q
+  // into one
+  const int64_t items = static_cast<int64_t>(segments) * ceil_div(nob, kWsSub);
+  const int64_t row_tiles = (mean + kMfRows - 1) / kMfRows;
+  const int64_t cost = items * (row_tiles + kWsBuildCost);
+  int64_t w = h.swiglu ? kMfCus : 2 * kMfCus / h.nproj;
+  w = cost < w ? cost : w;
+  int64_t p = items, q = w;
+  for (int64_t x = p, y = q;;) {  // by their greatest common divisor
+    const int64_t m = x % y;
+    if (m == 0) {
+      p /= y;
+      q /= y;
+      break;
+    }
+    x = y;
+    y = m;
+  }
+  const float visits = static_cast<float>((p + 2 * q - 2) / q);
+  const float rows = static_cast<float>(row_tiles) * static_cast<float>(items) / static_cast<float>(w);
+  const float ws = c.ws + visits * (c.build + c.build_k * f) + rows * (c.row + c.row_k * f);
+  // decode: the longest run, as the kernel splits them
+  const int tile = compact ? 64 : 32;
+  const int64_t rt = segments * ((mean + tile - 1) / tile);
+  const int64_t pairs = rt * nob;
+  const int64_t wd = mf_workgroups(h.swiglu ? 2 : 1, tile, compact, h.nproj);
+  int64_t run;
+  if (rt * 3 <= wd || (rt <= wd && pairs < 8 * wd)) {
+    const int64_t per = wd / rt < nob ? wd / rt : nob;
+    run = (nob + per - 1) / per;
+  } else {
+    run = (pairs + wd - 1) / wd;
+  }
+  const float dec = c.dec + static_cast<float>(run) * (c.tile + c.tile_k * f);
+  return dec * 1.08f >= ws;  // (the estimates' own error)
 }
 
 int launch_grouped_mfma(const uint16_t* hidden_a, const uint16_t* hidden_b, int batch, const int32_t* expert_ids,
@@ -2252,22 +2341,19 @@ int launch_grouped_mfma(const uint16_t* hidden_a, const uint16_t* hidden_b, int 
   const int units = (swiglu || comb_out != nullptr) ? 2 : 1;
   const int nproj = (pb && !swiglu) ? 2 : 1;
   hipStream_t s = static_cast<hipStream_t>(stream);
-  // the compact LDS layout: a chunk of 256 columns (rank <= 256), at most 4 row-scale groups and 64 salient columns per
-  // expert.  The 64-row tiles fit in it three workgroups a CU
-  const auto compact_ok = [](const tris_compact3_payload* p) {
-    return p->num_groups <= mf_groups_cap(true) && p->qweight2_sparse_rows * kMfSalWin <= mf_sal_slots(true) &&
-           p->rank <= kMfChunk / 2;
-  };
-  const bool chunks = pa->rank > kMfChunk || (pb && pb->rank > kMfChunk);  // more than one 512-column chunk
-  const bool single = !mf_wide(args.proj[0]) || (pb && !mf_wide(args.proj[1]));  // weight words loaded one at a time
-  const bool compact = !single && compact_ok(pa) && (!pb || compact_ok(pb));
-  const int ws_min = single ? kWsMinRowsSingle : (compact ? kWsMinRowsCompact : kWsMinRows);
+  MfShape shape{pa->rank, max_n, pa->num_groups, pa->qweight2_sparse_rows, !mf_wide(args.proj[0]), swiglu,
+                row_index != nullptr, nproj};
+  if (pb) {
+    shape.rank = pb->rank > shape.rank ? pb->rank : shape.rank;
+    shape.groups = pb->num_groups > shape.groups ? pb->num_groups : shape.groups;
+    shape.q2rows = pb->qweight2_sparse_rows > shape.q2rows ? pb->qweight2_sparse_rows : shape.q2rows;
+    shape.single = shape.single || !mf_wide(args.proj[1]);
+  }
+  const bool chunks = shape.rank > kMfChunk;  // more than one 512-column chunk
+  const bool single = shape.single;
+  const bool compact = mf_compact(shape);
   // long segments: keep each output tile's weights in registers and stream the segment's rows through them
-  // (its buffer resources address a segment's rows in 32-bit byte offsets: the whole batch must stay below 2 GiB)
-  if (partials == nullptr && num_segments <= kWave &&
-      static_cast<int64_t>(batch) >= static_cast<int64_t>(ws_min) * num_segments &&
-      ws_fits(pa) && (!pb || ws_fits(pb)) && static_cast<int64_t>(batch) * max_n * 2 < (int64_t{1} << 31) &&
-      static_cast<int64_t>(batch) * kMfChunk * 2 < (int64_t{1} << 31)) {
+  if (partials == nullptr && comb_out == nullptr && mf_weight_stationary(shape, batch, num_segments)) {
     return launch_grouped_mfma_ws(args, units, nproj, max_n, batch, s, who);
   }
   // Staged activation rows: a row tile has at most min(row tile, batch).  From kMfTallMinRows rows a segment on average,
@@ -2278,13 +2364,7 @@ int launch_grouped_mfma(const uint16_t* hidden_a, const uint16_t* hidden_b, int 
   const int rows = batch <= 4 ? 4 : (!tall ? kMfRows : (compact ? 64 : 32));
   const int lds_total = mf_static_lds_bytes(units, rows, compact);
   TRIS_REQUIRE(lds_total <= 160 * 1024, "%s: LDS request %d exceeds a CU", who, lds_total);
-  // Workgroups: as many as the GPU holds at once (LDS and the kernel's registers, mf_waves, bound them), shared by the
-  // projections of an unfused pair.
-  int wgs_per_cu = (160 * 1024) / lds_total;
-  const int by_regs = units == 1 ? mf_waves(units, rows, compact) : 1;
-  wgs_per_cu = wgs_per_cu < by_regs ? wgs_per_cu : by_regs;
-  wgs_per_cu = wgs_per_cu > 0 ? wgs_per_cu : 1;
-  int wgs = (kMfCus * wgs_per_cu) / nproj;
+  int wgs = mf_workgroups(units, rows, compact, nproj);
   // no more than the (row tile, output tile) pairs there can be: row tiles <= batch / row tile + min(segments, batch)
   const int64_t pairs = (static_cast<int64_t>(batch) / (rows > kMfRows ? rows : kMfRows) +
                          (num_segments < batch ? num_segments : batch)) * ceil_div(max_n, kTileOut);
@@ -2460,6 +2540,16 @@ bool grouped_mfma_supported(const tris_compact3_payload* p, const uint16_t* hidd
 }
 
 }  // namespace tris
+
+extern "C" int tris_grouped_predecoded_weight_stationary(int32_t rank, int32_t outfeatures, int32_t num_groups,
+                                                         int32_t qweight2_sparse_rows, int32_t wide,
+                                                         int32_t projections, int32_t swiglu, int32_t gathered,
+                                                         int64_t rows, int32_t segments) {
+  if (rank < 1 || outfeatures < 1 || rows < 0 || projections < 1 || projections > 2 || (swiglu && projections != 2)) return 0;
+  const tris::MfShape h{rank, outfeatures, num_groups, qweight2_sparse_rows, wide == 0, swiglu != 0, gathered != 0,
+                        swiglu ? 1 : projections};
+  return tris::mf_weight_stationary(h, rows, segments) ? 1 : 0;
+}
 
 extern "C" int64_t tris_compact3_linears_workspace_bytes(int32_t batch, int32_t rank, const int32_t* outfeatures,
                                                          int32_t count) {

@@ -773,6 +773,22 @@ def _segments_total(segment_offsets) -> int:
     return int(segment_offsets.numel()) - 1
 
 
+def predecoded_weight_stationary(payloads, rows: int, segments: int, swiglu: bool = False,
+                                 gathered: bool = False) -> bool:
+    """Whether the predecoded MFMA GEMM of one or two projections over ``rows`` rows in ``segments`` segments runs on the
+    weight-stationary kernel (tris_grouped_predecoded_weight_stationary)."""
+    rank = n = groups = q2 = 0
+    wide = True
+    for p in payloads:
+        qw, rp = p["qweight1"], p["row_pack3"]
+        cols = qw.shape[2]
+        rank, n = max(rank, p["g_idx"].shape[1]), max(n, cols)
+        groups, q2 = max(groups, rp.shape[2]), max(q2, p["qweight2_sparse"].shape[1])
+        wide = wide and not (cols % 4 or qw.data_ptr() % 16 or rp.data_ptr() % 16)
+    return bool(_lib.load().tris_grouped_predecoded_weight_stationary(rank, n, groups, q2, wide, len(payloads), swiglu,
+                                                                      gathered, rows, segments))
+
+
 def compact3_tris_precomputed_grouped_forward_block_gr_predecoded_hybrid(
         hidden, expert_ids, segment_offsets, full_problem_offsets, full_problem_tiles, tail_problem_offsets,
         tail_problem_tiles, decoded_q_gmap_words, qweight1, qweight2_sparse, qweight2_sparse_prefix, c_map, g_idx,

@@ -573,3 +573,34 @@ def test_shared_expert_stack_conditions_and_layout():
     assert not moe.SharedExpertStack.ok({**backbones, "gate_in_scale": mk(H)}, shared)
     assert not moe.SharedExpertStack.ok(backbones, (shared[0].float(), shared[1], shared[2]))
     assert not moe.SharedExpertStack.ok(backbones, None)
+
+
+def test_weight_stationary_rule(tris):
+    """Which kernel a predecoded launch takes: the decode one up to 64 rows a segment, the weight-stationary one from 120
+    (500 in the compact layout: rank <= 256, 4 groups, 64 salient columns), by estimated times between, and only where it
+    fits at all."""
+    from tris_moe_amd import _lib
+
+    rule = _lib.load().tris_grouped_predecoded_weight_stationary
+
+    def ws(rank=512, n=2048, groups=4, q2=1, wide=1, nproj=2, swiglu=0, gathered=0, rows=1000, segments=8):
+        return rule(rank, n, groups, q2, wide, nproj, swiglu, gathered, rows, segments)
+
+    for rank in (64, 256, 320, 512):
+        for n in (64, 2050, 14336):
+            for segments in (1, 8, 64):
+                for kw in ({}, {"swiglu": 1}, {"gathered": 1}, {"nproj": 1}):
+                    line = 500 if rank <= 256 else 120
+                    assert not ws(rank, n, rows=64 * segments - 1, segments=segments, **kw)
+                    assert ws(rank, n, rows=line * segments, segments=segments, **kw)
+                    assert ws(rank, n, wide=0, rows=64 * segments, segments=segments, **kw)
+                    assert not ws(rank, n, rows=65 * line, segments=65, **kw)
+    assert not ws(576) and not ws(q2=3)
+    assert ws(256, groups=5, rows=960) and ws(256, q2=2, rows=4000) and not ws(256, rows=960)
+    # between: few and long runs of output tiles decode, many segments and one item a workgroup stay put
+    assert not ws(n=2048, rows=8 * 83) and not ws(n=14336, nproj=1, rows=8 * 83)
+    assert ws(n=512, rows=64 * 65, segments=64) and ws(n=4096, rows=8 * 97, swiglu=1)
+    # a Mixtral prompt of 333 tokens gathers its rows, one of 512 does not
+    assert not ws(n=14336, gathered=1, rows=666) and ws(n=14336, gathered=1, rows=1024)
+    # shapes past the 32-bit offsets stay on the decode kernel, senseless ones are no launch at all
+    assert not ws(n=1 << 20, rows=2000) and not ws(rows=0) and not ws(segments=0) and not ws(nproj=1, swiglu=1)
