@@ -151,20 +151,24 @@ def gathered_inputs(rng, tokens, rows, k, dev):
     return to(ha), to(hb), to(ridx), to(ga), to(gb), ga, gb
 
 
-@pytest.mark.parametrize("lengths", [[2, 37, 0, 5], [300, 0, 200, 90]], ids=["decode", "prefill-ws"])
-def test_gathered_predecoded_gemms_match_materialised_rows(tris, oracle_mod, cuda, lengths):
+@pytest.mark.parametrize("lengths,k", [([2, 37, 0, 5], 256), ([300, 0, 200, 90], 256), ([300, 0, 200, 90], 512)],
+                         ids=["decode", "prefill", "prefill-ws"])
+def test_gathered_predecoded_gemms_match_materialised_rows(tris, oracle_mod, cuda, lengths, k):
     """Grouped row r reads hidden[row_index[r]]: the dual and SwiGLU outputs equal the calls on the
     materialised rows bit for bit (on the decode kernel, and on the weight-stationary kernel for long
-    segments), and the oracle's within tolerance."""
-    note(f"gathered dual/swiglu segments={lengths}")
+    segments at a rank above 256), and the oracle's within tolerance."""
+    note(f"gathered dual/swiglu segments={lengths} k={k}")
     ext = tris["ext"]
-    E, n, k = 4, 320, 256
+    E, n = 4, 320
     pa, pb = make_projection(tris, 81, E, n, k), make_projection(tris, 82, E, n, k)
     da, db = (tris["qlinear"].payload_to_device(p, cuda) for p in (pa, pb))
     ids = np.asarray([e for e in range(E) if lengths[e] > 0], dtype=np.int32)
     offs = np.concatenate([[0], np.cumsum([lengths[e] for e in ids])]).astype(np.int32)
     prob = np.concatenate([[0], np.cumsum((np.diff(offs) + 3) // 4)]).astype(np.int32)
     rows = int(offs[-1])
+    for gathered in (False, True):
+        for fused in (False, True):
+            assert ext.predecoded_weight_stationary([da, db], rows, ids.size, fused, gathered) == (k > 256)
     rng = np.random.default_rng(rows)
     ha, hb, ridx, ga, gb, ga_np, gb_np = gathered_inputs(rng, max(8, rows // 3), rows, k, cuda)
     args = (t_i32(ids, cuda), t_i32(offs, cuda), t_i32(prob, cuda), torch.tensor([int(prob[-1])]))

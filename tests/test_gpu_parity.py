@@ -696,22 +696,22 @@ def test_predecoded_mfma_one_hot_is_bit_exact(tris, oracle_mod, cuda, rank, n, s
     """With one-hot activation rows the MFMA grouped GEMM returns single dequantised weights, which
     must equal the reference's fp16 weights bit for bit: every lane group, packed row, split bit,
     sign and salient column of the operand construction is checked.  Each expert gets `rank` rows (row r
-    is e_r), as one segment (long segments: the weight-stationary kernel) or as segments of `split` rows
-    of the same expert (the row-tile kernel)."""
+    is e_r), as one segment (512 rows, the rows again below that rank: the weight-stationary kernel) or as segments
+    of `split` rows of the same expert (the row-tile kernel)."""
     note(f"mfma one-hot rank={rank} n={n} split={split}")
     ext = tris["ext"]
     E = 2
     pay = make_projection(tris, 70 + rank, E, n, rank, salient_counts=salient)
     d = tris["qlinear"].payload_to_device(pay, cuda)
-    step = rank if split is None else split
-    ids = np.repeat(np.arange(E, dtype=np.int32), ceil_div(rank, step))
-    offs = np.concatenate([[0], np.cumsum([min(step, rank - c) for _ in range(E) for c in range(0, rank, step)])])
+    per = rank if split is not None else 512
+    step = per if split is None else split
+    ids = np.repeat(np.arange(E, dtype=np.int32), ceil_div(per, step))
+    offs = np.concatenate([[0], np.cumsum([min(step, per - c) for _ in range(E) for c in range(0, per, step)])])
     offs = offs.astype(np.int32)
-    rows = E * rank
+    rows = E * per
+    assert ext.predecoded_weight_stationary([d], rows, ids.size) == (split is None)
     h = np.zeros((rows, rank), dtype=np.float16)
-    for e in range(E):
-        for r in range(rank):
-            h[e * rank + r, r] = 1.0
+    h[np.arange(rows), np.arange(rows) % rank] = 1.0
     hd = torch.from_numpy(h).to(cuda)
     prob = np.concatenate([[0], np.cumsum((np.diff(offs) + 3) // 4)]).astype(np.int32)
     nblk = tris["synthetic"].packing.num_gr_blocks(rank, n)
@@ -724,13 +724,13 @@ def test_predecoded_mfma_one_hot_is_bit_exact(tris, oracle_mod, cuda, rank, n, s
         True).cpu().numpy()
     for e in range(E):
         w = oracle_mod.dequant_grouped_expert(pay, e, True)   # [n, rank] fp16
-        np.testing.assert_array_equal(got[e * rank:(e + 1) * rank].view(np.uint16),
-                                      w.T.astype(np.float16).view(np.uint16))
+        np.testing.assert_array_equal(got[e * per:(e + 1) * per].view(np.uint16),
+                                      np.tile(w.T.astype(np.float16), (per // rank, 1)).view(np.uint16))
 
 
 @pytest.mark.parametrize("drop", [None, 0])
 def test_predecoded_long_segments(tris, oracle_mod, cuda, drop):
-    """Segments of 64 rows and more (the weight-stationary MFMA kernel): ragged N (a partial output tile),
+    """Segments of 120 rows and more on average (the weight-stationary MFMA kernel): ragged N (a partial output tile),
     rows not a multiple of 16, a full second salient window (64 salient columns) and, with drop=0, a
     segment routed to no expert (zero rows)."""
     note(f"predecoded long segments drop={drop}")
@@ -738,8 +738,9 @@ def test_predecoded_long_segments(tris, oracle_mod, cuda, drop):
     E, n, k = 3, 200, 512
     pay = make_projection(tris, 81, E, n, k, salient_counts=[64, 0, 33])
     d = tris["qlinear"].payload_to_device(pay, cuda)
-    ids, offs = _segments([130, 0, 75], E, drop)
+    ids, offs = _segments([200, 0, 75], E, drop)
     prob = np.concatenate([[0], np.cumsum((np.diff(offs) + 3) // 4)]).astype(np.int32)
+    assert ext.predecoded_weight_stationary([d], int(offs[-1]), ids.size)
     rng = np.random.default_rng(12)
     rows = int(offs[-1])
     h = (rng.standard_normal((rows, k)) * 1.5).astype(np.float16)
@@ -810,23 +811,27 @@ def test_predecoded_row_tiles(tris, oracle_mod, cuda, rank, n, segs):
         assert torch.equal(one, y)
 
 
-@pytest.mark.parametrize("seg", [[3, 21, 0, 9], [90, 150, 0, 70]], ids=["short", "long"])
-def test_swiglu_fused_matches_dual_then_silu(tris, oracle_mod, cuda, seg):
+@pytest.mark.parametrize("seg,k,drop", [([3, 21, 0, 9], 256, None), ([90, 150, 0, 70], 256, None),
+                                        ([190, 150, 0, 71], 512, None), ([190, 150, 0, 71], 448, 1)],
+                         ids=["short", "long", "ws", "ws-no-expert"])
+def test_swiglu_fused_matches_dual_then_silu(tris, oracle_mod, cuda, seg, k, drop):
     """The fused gate/up GEMM + SwiGLU equals silu(g) * u computed from the dual kernel's own fp16
     outputs with the oracle's fp16 roundings; exp may differ in its last fp32 bit from numpy's,
-    so a rare one-ulp difference is allowed.  Long segments run the weight-stationary kernel, whose
-    dual outputs are also checked against the oracle."""
-    note(f"swiglu fused seg={seg}")
+    so a rare one-ulp difference is allowed.  Long segments at a rank above 256 run the weight-stationary kernel
+    (one of them routed to no expert), whose dual outputs are also checked against the oracle."""
+    note(f"swiglu fused seg={seg} k={k} drop={drop}")
     ext = tris["ext"]
-    E, k, n = 4, 256, 320
+    E, n = 4, 320
     pa = make_projection(tris, 61, E, n, k)
     pb = make_projection(tris, 62, E, n, k)
     da = tris["qlinear"].payload_to_device(pa, cuda)
     db = tris["qlinear"].payload_to_device(pb, cuda)
-    ids, offs = _segments(seg, E)
+    ids, offs = _segments(seg, E, drop)
     prob = np.concatenate([[0], np.cumsum((np.diff(offs) + 3) // 4)]).astype(np.int32)
     rng = np.random.default_rng(9)
     rows = int(offs[-1])
+    for fused in (False, True):
+        assert ext.predecoded_weight_stationary([da, db], rows, ids.size, swiglu=fused) == (k > 256)
     ha = torch.from_numpy((rng.standard_normal((rows, k)) * 3).astype(np.float16)).to(cuda)
     hb = torch.from_numpy((rng.standard_normal((rows, k)) * 3).astype(np.float16)).to(cuda)
     args = (t_i32(ids, cuda), t_i32(offs, cuda), t_i32(prob, cuda), int(prob[-1]))
