@@ -1269,16 +1269,20 @@ void grouped_mfma_kernel(MfmaArgs a) {
     }
     f32x4 up = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
     if (kUnits == 2) up = *reinterpret_cast<const f32x4*>(&ex[utid * 4]);
-    const __amdgpu_buffer_rsrc_t r_out = make_rsrc(out0 + ob * kTileOut, static_cast<uint32_t>(rc * N - ob * kTileOut) * 2u);
+    const uint32_t bytes = (static_cast<uint32_t>(rc) * N - ob * kTileOut) * 2u;
+    const __amdgpu_buffer_rsrc_t r_out = make_rsrc(out0 + ob * kTileOut, bytes);
     const int r0 = 16 * m + 4 * kg;  // the lane's rows r0 .. r0 + 3
-    const uint32_t vo = n < N ? static_cast<uint32_t>(r0 * N + 16 * wave + i16) * 2u : kMfOob;
+    // Where a lane without an output stores: past the buffer.  The launcher keeps the 32- and 64-row tiles' outputs below
+    // 2 GiB; a 16-row tile's can be larger, and kMfOob inside them.  (The size in a register made the 64-row instance spill.)
+    const uint32_t drop = kRows > kMfRows ? kMfOob : bytes;
+    const uint32_t vo = n < N ? static_cast<uint32_t>(r0 * N + 16 * wave + i16) * 2u : drop;
 #pragma unroll
     for (int v = 0; v < 4; ++v) {
       // two units: g and u rounded to fp16 as the two outputs would be.  One unit: no output scale or bias here, the
       // host sends none (launch_grouped_mfma rejects payloads with them)
       const uint16_t y = kUnits == 2 ? swiglu_bits(f2h_bits(acc[v]), f2h_bits(up[v])) : f2h_bits(acc[v]);
-      __builtin_amdgcn_raw_buffer_store_b16(y, r_out, r0 + v < rc ? vo + static_cast<uint32_t>(v * N) * 2u : kMfOob, 0u,
-                                            0);
+      __builtin_amdgcn_raw_buffer_store_b16(y, r_out, r0 + v < rc && (kRows > kMfRows || n < N) ? vo + static_cast<uint32_t>(v * N) * 2u : drop,
+                                            0u, 0);
     }
   };
   // kNs output tiles from `ob`, whose words are in wb, kRt 16-row sub-tiles; with one chunk the next tiles' words are
@@ -2360,7 +2364,8 @@ int launch_grouped_mfma(const uint16_t* hidden_a, const uint16_t* hidden_b, int 
   // row tiles of 32 rows (64 at rank <= 256, where they take half the LDS): a segment then rarely needs two, and its
   // weights are built once, not once every 16 rows.
   const int64_t tall_min = single ? kMfTallMinRowsSingle : kMfTallMinRows;
-  const bool tall = !chunks && partials == nullptr && static_cast<int64_t>(batch) >= tall_min * num_segments;
+  const bool tall = !chunks && partials == nullptr && static_cast<int64_t>(batch) >= tall_min * num_segments &&
+                    static_cast<int64_t>(max_n) * (compact ? 64 : 32) * 2 < (int64_t{1} << 31);
   const int rows = batch <= 4 ? 4 : (!tall ? kMfRows : (compact ? 64 : 32));
   const int lds_total = mf_static_lds_bytes(units, rows, compact);
   TRIS_REQUIRE(lds_total <= 160 * 1024, "%s: LDS request %d exceeds a CU", who, lds_total);

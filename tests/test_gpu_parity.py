@@ -811,6 +811,40 @@ def test_predecoded_row_tiles(tris, oracle_mod, cuda, rank, n, segs):
         assert torch.equal(one, y)
 
 
+@pytest.mark.parametrize("n,rows,step", [(18_000_000, 63, 16), (72_000_000, 15, 4)])
+def test_predecoded_outputs_past_2_gib(tris, cuda, n, rows, step):
+    """Rows whose outputs span more than 2 GiB (of a 64- and of a 16-row tile): the rows computed together are those
+    computed in parts, and the lanes without a row write nothing."""
+    rank = 64
+    note(f"predecoded row tile past 2 GiB n={n} rows={rows}")
+    ext = tris["ext"]
+    gen = torch.Generator(device=cuda).manual_seed(3)
+
+    def words(*shape):
+        return torch.randint(-(1 << 31), (1 << 31) - 1, shape, generator=gen, device=cuda, dtype=torch.int32)
+
+    def halves(lo, hi, *shape):
+        parts = [(torch.rand(shape, generator=gen, device=cuda) * (hi - lo) + lo).to(torch.float16) for _ in range(4)]
+        return sum((p.view(torch.int16).to(torch.int64) & 0xFFFF) << (16 * i) for i, p in enumerate(parts))
+
+    c_map = t_i32(np.asarray([[1 << 5, 1 << 9]]), cuda)
+    pay = (words(1, 2, n), words(1, 1, n), t_i32(np.asarray([[0, 1, 2]]), cuda), c_map,
+           torch.zeros((1, rank), dtype=torch.int32, device=cuda), halves(0.75, 1.25, 1, rank),
+           halves(0.01, 0.02, 1, n, 1))
+    dec = words(1, ceil_div(n, 64), 128)
+    h = torch.randn((rows, rank), generator=gen, device=cuda).to(torch.float16)
+
+    def run(x):
+        r = x.shape[0]
+        return ext.compact3_tris_precomputed_grouped_forward_block_gr_predecoded(
+            x, t_i32(np.asarray([0]), cuda), t_i32(np.asarray([0, r]), cuda),
+            t_i32(np.asarray([0, ceil_div(r, 4)]), cuda), ceil_div(r, 4), dec, *pay, True)
+
+    got = run(h)
+    for r0 in range(0, rows, step):
+        assert torch.equal(got[r0:r0 + step], run(h[r0:r0 + step].contiguous())), r0
+
+
 @pytest.mark.parametrize("seg,k,drop", [([3, 21, 0, 9], 256, None), ([90, 150, 0, 70], 256, None),
                                         ([190, 150, 0, 71], 512, None), ([190, 150, 0, 71], 448, 1)],
                          ids=["short", "long", "ws", "ws-no-expert"])
