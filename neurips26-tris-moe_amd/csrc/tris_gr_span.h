@@ -22,12 +22,13 @@
 //                       mid-remainder whose last bits are zero ends at bit 0)
 //                       and the F advance in bits 26..31.
 // The table reads and the emission's ORs hit random LDS banks: at the Mixtral
-// shape (8 experts, 32768 blocks) LDS was busy 61% of the kernel, two thirds
-// of it conflicts, when the walk read 64-bit entries twice.  The advances ride
+// shape (8 experts, 32768 blocks) two thirds of the LDS's active cycles were
+// conflicts when the walk read 64-bit entries twice.  The advances ride
 // in the words that A reads, an entry is 32 bits and read once, an OR whose
 // word is empty is skipped and the ones are counted in the finished bitmap:
-// LDS busy 44%, 22.3 -> 20.4 us (Mixtral, 16 tokens), 15.9 -> 14.0 us (one
-// token), 24.9 -> 23.2 us (A3B, 32 tokens).  What is left is the latency of
+// 164 -> 133 LDS instructions a wavefront, conflicts 67 -> 57% of its active
+// cycles (a third of the launch), 22.3 -> 20.4 us (Mixtral, 16 tokens), 15.9
+// -> 14.0 us (one token), 24.9 -> 23.2 us (A3B, 32 tokens).  What is left is the latency of
 // the header, words and table chain: fewer VALU (17 instead of 23 a byte) or
 // an even number of items a wavefront changed nothing.
 // Each lane of the block's group of S lanes:

@@ -13,14 +13,14 @@
 // kernel (TriSMoE_cuda_kernel.cu:4889-5093).
 //
 // Operand layout of the decode kernel (v_mfma_f32_16x16x32_f16): A rows are up to 16 rows
-// of one segment; lane group kg (lanes 16kg..16kg+15) supplies the 8 columns kg + 4i and
+// of one segment (a sub-tile of its row tile); lane group kg (lanes 16kg..16kg+15) supplies the 8 columns kg + 4i and
 // kg + 4i + 16 (i < 4) of each 32-column packed row.  Activations and the column factors are
 // staged in LDS in the same permuted column order, so each lane reads its 8
 // values with one 16-byte LDS load.
 //
 // Work decomposition of the decode kernel: workgroup = 4 wavefronts = a run of 64-output
-// tiles x one tile of <= 16 rows of one segment x one projection (blockIdx.z).  The
-// workgroup stages the rows' activations and the column factors of a 512-column
+// tiles x one row tile (up to 4, 16, 32 or 64 rows of one segment) x one projection (blockIdx.z;
+// two units of 4 wavefronts take two projections side by side).  The workgroup stages the rows' activations and the column factors of a 512-column
 // chunk in LDS once; wavefront w then owns outputs [16w, 16w+16) of each tile over the whole
 // chunk, two tiles at a time, while its weight words of the next two are in flight, so no
 // partial sums cross wavefronts.  Salient columns are zero in that pass; afterwards each lane
@@ -36,8 +36,8 @@
 // the kernel asks for its scalars and row indices at once, keeps the K loop rolled, and hides
 // the sizes and the lane index from the compiler per row tile, which otherwise computes
 // every address of the rare paths ahead of the loop.  T = 16 gate/up launch at the Mixtral shape
-// 31.5 -> 27.7 us, T = 64 42.3 -> 36.3 us; OLMoE T = 16 gate/up 17.6 -> 12.7, down 16.3 -> 11.9 us;
-// A3B T = 1024 gate/up 67 -> 49, down 113 -> 79 us.
+// 31.5 -> 27.7 us, T = 64 42.3 -> 36.3 us (32-row tiles: 32.3); OLMoE T = 16 gate/up 17.6 -> 12.7, down
+// 16.3 -> 11.9 us; A3B T = 1024 gate/up 67 -> 49, down 113 -> 79 us (64-row tiles and even runs: 39 and 58).
 #include <type_traits>
 
 #include "tris_common.h"
@@ -204,7 +204,13 @@ constexpr int kMfTbRs = kMfTbGw + kMfPR * kTileOut;
 constexpr int kMfTbWords = kMfTbRs + kTileOut * kMfMaxGroups * 2;
 static_assert(kMfTbGw % 4 == 0 && kMfTbRs % 4 == 0, "tile buffer pieces must be 16-byte aligned");
 constexpr int kMfCus = 256;  // MI355X compute units
-constexpr int kMfTallMinRows = 12;  // mean rows a segment from which the decode kernel takes 32- or 64-row tiles
+// Mean rows a segment from which the decode kernel takes 32-row tiles (64 in the compact layout): a segment's weights are
+// then built once where two 16-row tiles would build them twice, but the taller instances hold more LDS and registers.
+// Tall against 16-row tiles, segments of random length, us: 8 of N = 14336, rank 512, pair: mean 11 28.3 / 27.6, 13 30.5 /
+// 31.3, 16 30.4 / 36.2, 24 31.7 / 44.8; 128 of N = 2048, rank 256, pair: 11 37.9 / 37.8, 13 38.1 / 42.4, 16 39.0 / 46.6.
+// (One or two tiles a workgroup gain later: 64 of N = 1024, rank 256, one projection 11.3 / 9.5 at 12 and 12.9 / 11.9 at
+// 24.)  With single-word loads: 8 of N = 8194, rank 512, pair: 12 22.7 / 20.9, 14 24.8 / 25.5, 17 24.5 / 27.4.
+constexpr int kMfTallMinRows = 12;
 constexpr int kMfTallMinRowsSingle = 17;
 // Decode kernel: row-scale groups and salient slots per chunk its LDS holds; the compact variant (at most 4
 // groups and 64 salient columns per expert, a rank of at most 256) stages half the columns.
@@ -885,9 +891,6 @@ __device__ __forceinline__ void mf_salient_operands(const MfChunk& ch, const uin
   }
 }
 
-// The lane's qweight2_sparse words of the chunk's first salient window (a window of kMfSalWin salient
-// columns spans at most two qweight2_sparse rows), for output column n.  Issued before the next tile's
-// LDS copies so that waiting for them does not wait for the copies.
 // A staged chunk's first salient index and its salient count, in scalar registers, the count held to the slots staged.
 struct MfChunkMeta {
   int sbase0, num_sal;
@@ -900,7 +903,9 @@ __device__ __forceinline__ MfChunkMeta mf_chunk_meta(const MfColRegs& R, int sal
   return r;
 }
 
-// q2: the expert's qweight2_sparse [q2rows][N].
+// The lane's qweight2_sparse words of the chunk's first salient window (a window of kMfSalWin salient columns spans at
+// most two qweight2_sparse rows), for output column n.  Issued before the next tiles' loads, so that waiting for them does
+// not wait for those.  q2: the expert's qweight2_sparse [q2rows][N].
 __device__ __forceinline__ void mf_q2_issue(const uint32_t* q2, int q2rows, int N, int n, const MfChunkMeta& cm,
                                             uint32_t (&q2w)[2]) {
   const uint32_t v_q2 = n < N ? static_cast<uint32_t>(n) * 4u : kMfOob;
@@ -2200,16 +2205,17 @@ static bool mf_compact(const MfShape& h) {
          h.rank <= kMfChunk / 2;
 }
 
-// Whether a launch goes weight-stationary.  Up to 64 rows a segment on average the decode kernel always is the faster one,
-// from 120 rows on (500 in the compact layout) the weight-stationary one.  Between them neither is, by up to 1.4 (64
-// segments of 65 rows, N = 512, rank 512, SwiGLU: 39 against 28 us) and 0.58 (8 of 65, N = 2048, single: 13 against 21):
-// the weight-stationary kernel pays for each item a workgroup touches (building its operands) and little for the rows,
-// the decode kernel for each pair of a 32- or 64-row tile and an output tile, and both wait for the workgroup with the
-// most of them.  So their times are estimated, us = constant + cost x that workgroup's count with the costs' parts
-// proportional to the rank apart, fitted over 769 launches of 1 to 64 segments, N 512 to 14336, ranks 64 to 512 (90 with
-// gathered rows): the one picked is at most 3% slower than weight-stationary ever was there, 20% faster in the mean (25%
-// in the compact layout), and 0.5% slower in the mean than always the better one.  Single-word launches, which no size
-// here covers, keep the weight-stationary kernel from 64 rows.
+// Whether a launch goes weight-stationary.  Below 64 rows a segment on average none does; from 120 rows on (500 in the
+// compact layout) every one does (Mixtral's gate/up + down, decode against weight-stationary: 130 rows 153 / 149 us, 150
+// rows 167 / 155; OLMoE's 500 rows 240 / 243).  Between them neither kernel is always the faster one: weight-stationary
+// takes from 0.70 (64 segments of 65 rows, N = 512, rank 512, SwiGLU: 28 against 39 us) to 1.6 times the decode kernel's
+// time (8 of 65, N = 2048, one projection: 21 against 13).  It pays for each item a workgroup touches (building its
+// operands) and little for the rows, the decode kernel for each pair of a 32- or 64-row tile and an output tile, and both
+// wait for the workgroup with the most of them.  So their times are estimated, us = constant + cost x that workgroup's
+// count, the part of a cost proportional to the rank apart, fitted over 769 launches of 1 to 64 segments, N 512 to 14336,
+// ranks 64 to 512 (90 with gathered rows).  The kernel picked there is at most 3% slower than the weight-stationary one,
+// 20 to 25% faster in the mean, and 0.3 to 0.7% slower in the mean than always the better one.  Single-word launches,
+// which the fit does not cover, go weight-stationary from 64 rows.
 constexpr int kWsMinRows = 64;
 constexpr int kWsAlwaysRows = 120;
 constexpr int kWsAlwaysRowsCompact = 500;

@@ -401,8 +401,9 @@ def _side_stream(device: torch.device, which: int = 0) -> torch.cuda.Stream:
 
 
 # Up to this many routed rows the gate/up GEMM applies act_fn(g) * u in its epilogue; above it the
-# separate gate and up workgroups plus tris_swiglu_mul are faster (measured on MI355X at the Mixtral
-# decode shape: 17.6 vs 18.9 us at 2 rows, 49.7 vs 42.3 us at 32 rows).
+# separate gate and up workgroups, with act_fn(g) * u formed inside the down backbone, are faster (layer step at the
+# Mixtral decode shape on MI355X, in the epilogue against apart: 2 rows 48.7 / 52.1 us, 4 rows 59.3 / 58.3, 6 rows
+# 69.0 / 64.7, 32 rows 89.6 / 79.6).
 FUSED_SWIGLU_MAX_ROWS = 4
 
 # The down projection's null-space compensation runs on the side stream beside the down backbone and GEMM
@@ -410,13 +411,13 @@ FUSED_SWIGLU_MAX_ROWS = 4
 NS_DOWN_BESIDE_GEMM = True
 
 # The gate/up null-space compensation runs on a side stream beside the decodes and backbones (True) or on the
-# caller's stream before them (False; measured on MI355X at the Mixtral decode shape, T = 16: 133.2 us beside,
-# 136.7 us before).
+# caller's stream before them (False; measured on MI355X at the Mixtral decode shape: T = 16 123 us beside, 128 us
+# before, T = 1 83 and 87).
 NS_GATE_UP_BESIDE = True
 
 # The block runs its shared expert as extra columns of the routed launches when the batch fits them
-# (SharedExpertStack, _SharedFold; measured on MI355X at the A3B shape: T = 1 60.6 -> 48.9 us, T = 32 140.2 ->
-# 133.4 us); False keeps its four launches of its own.
+# (SharedExpertStack, _SharedFold; measured on MI355X at the A3B shape: T = 1 56.4 -> 44.6 us, T = 32 118.0 ->
+# 110.1 us); False keeps its four launches of its own.
 FOLD_SHARED_EXPERT = True
 
 # After the fused gate/up GEMM the down backbone's split-K partial sums go straight to the down GEMM, whose
@@ -426,8 +427,9 @@ DOWN_PARTIALS_IN_GEMM = True
 # Stacked rows (routed + shared) up to which the folded shared expert's down projection runs as extra columns of the
 # routed down backbone's launch (tris_backbone_swiglu_linear_split); above, in launches of its own.  The decode
 # kernel's row groups would take up to 512, but the stacked product's unused quadrants (routed rows x the shared
-# columns) cost more than the two launches: measured on MI355X at the A3B shape, T = 32 134.5 against 133.8 us,
-# T = 48 156.1 against 152.5 us.
+# columns) cost more than the two launches: measured on MI355X at the A3B shape, as extra columns against in launches of
+# its own: T = 8 (72 rows) 63.8 / 68.6 us, T = 14 (126 rows) 77.9 / 81.0, T = 32 (288 rows) 111.1 / 110.2, T = 48 128.2 /
+# 123.7.
 FOLD_SPLIT_DOWN_MAX_ROWS = 128
 
 # One token on two experts (Mixtral at T = 1): the routed combine in the down GEMM's launch
@@ -435,16 +437,16 @@ FOLD_SPLIT_DOWN_MAX_ROWS = 128
 COMBINE_IN_DOWN_GEMM = True
 
 # The decode step decodes every expert's split bitmaps (slot e for expert e) when the batch routes at least this
-# many rows per expert, so the predecode does not wait for the router's selection (measured on MI355X at the
-# Mixtral shape: T = 8, 16 rows over 8 experts, 92.4 -> 89.0 us; T = 4, 8 rows over ~5 experts, 78.8 against
-# 78.4 us, where decoding every expert is 1.6 times the blocks; T = 16 routes 32 rows and leaves an expert idle
-# about once in 12 steps).
+# many rows per expert, so the predecode does not wait for the router's selection (layer step at the Mixtral shape on
+# MI355X, every expert against the picked ones: T = 16 78.5 / 83.5 us, T = 8, 16 rows over 8 experts, 75.0 / 78.8; T = 4,
+# 8 rows over ~5 experts, 68.3 / 70.1, though that decodes 1.6 times the blocks, and more with fewer rows).
 DECODE_ALL_MIN_ROWS_PER_EXPERT = 2
 
 # From this many tokens the shared expert, when it runs in launches of its own, runs on a side stream beside the
 # routed experts; below it on the
 # caller's stream, since a graph's cross-queue join costs more than the overlap saves there (measured on MI355X at
-# the A3B shape: T = 1 64.3 -> 59.0 us inline; T = 32 138 vs 139 us; T = 1024 339 vs 356 us).
+# the A3B shape, on the side stream against inline: T = 1 65.7 / 56.8 us, T = 32 120.8 / 115.9, T = 256 197 / 203,
+# T = 1024 243 / 257; up to 64 tokens the block folds the shared expert where it fits).
 SHARED_EXPERT_SIDE_STREAM_MIN_TOKENS = 32
 
 
