@@ -2556,7 +2556,7 @@ extern "C" int tris_grouped_predecoded_weight_stationary(int32_t rank, int32_t o
                                                          int32_t qweight2_sparse_rows, int32_t wide,
                                                          int32_t projections, int32_t swiglu, int32_t gathered,
                                                          int64_t rows, int32_t segments) {
-  if (rank < 1 || outfeatures < 1 || rows < 0 || projections < 1 || projections > 2 || (swiglu && projections != 2)) return 0;
+  if (rank < 1 || outfeatures < 1 || rows < 0 || rows > INT32_MAX || projections < 1 || projections > 2 || (swiglu && projections != 2)) return 0;
   const tris::MfShape h{rank, outfeatures, num_groups, qweight2_sparse_rows, wide == 0, swiglu != 0, gathered != 0,
                         swiglu ? 1 : projections};
   return tris::mf_weight_stationary(h, rows, segments) ? 1 : 0;

@@ -779,13 +779,14 @@ def predecoded_weight_stationary(payloads, rows: int, segments: int, swiglu: boo
     weight-stationary kernel (tris_grouped_predecoded_weight_stationary)."""
     rank = n = groups = q2 = 0
     wide = True
-    for p in payloads:
+    for p in payloads:  # (each attribute read once: a prompt's host path runs this)
         qw, rp = p["qweight1"], p["row_pack3"]
-        cols = qw.shape[2]
-        rank, n = max(rank, p["g_idx"].shape[1]), max(n, cols)
-        groups, q2 = max(groups, rp.shape[2]), max(q2, p["qweight2_sparse"].shape[1])
+        _, packed_rows, cols = qw.shape
+        g, q = rp.shape[2], p["qweight2_sparse"].shape[1]
+        rank, n = packed_rows if packed_rows > rank else rank, cols if cols > n else n
+        groups, q2 = g if g > groups else groups, q if q > q2 else q2
         wide = wide and not (cols % 4 or qw.data_ptr() % 16 or rp.data_ptr() % 16)
-    return bool(_lib.load().tris_grouped_predecoded_weight_stationary(rank, n, groups, q2, wide, len(payloads), swiglu,
+    return bool(_lib.load().tris_grouped_predecoded_weight_stationary(32 * rank, n, groups, q2, wide, len(payloads), swiglu,
                                                                       gathered, rows, segments))
 
 
@@ -834,14 +835,14 @@ def mfma_payload_ok(p: dict) -> bool:
     """The payload suits the predecoded MFMA kernel (the one that can gather its rows through a row index):
     uniform 64-column groups, rank a multiple of 64, at most MFMA_MAX_GROUPS groups and 32-bit buffer offsets
     per expert."""
-    rank = int(p["g_idx"].size(1))
-    n = int(p["qweight1"].size(2))
-    groups = int(p["row_pack3"].size(2))
+    rank = p["g_idx"].shape[1]
+    n = p["qweight1"].shape[2]
+    groups = p["row_pack3"].shape[2]
     packed_rows = (rank + 31) // 32
     limit = 1 << 31
     return (bool(p.get("_compact3_k64_groups_uniform", False)) and rank > 0 and rank % 64 == 0
             and 1 <= groups <= MFMA_MAX_GROUPS and packed_rows * n * 4 < limit
-            and int(p["qweight2_sparse"].size(1)) * n * 4 < limit and n * groups * 8 < limit
+            and p["qweight2_sparse"].shape[1] * n * 4 < limit and n * groups * 8 < limit
             and ((packed_rows + 1) // 2) * ((n + 63) // 64) * 128 * 4 < limit)
 
 

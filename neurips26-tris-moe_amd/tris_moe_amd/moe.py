@@ -383,7 +383,7 @@ def _combine(x16, d_out, route, w16, output_dtype, shared, d_comp=None):
 
 
 def _predecode_buffer(p, slots, device):
-    packed_rows, n = int(p["qweight1"].size(1)), int(p["qweight1"].size(2))
+    _, packed_rows, n = p["qweight1"].shape
     nblk = ((packed_rows + 1) // 2) * ((n + 63) // 64)
     return torch.empty((slots, nblk, 128), dtype=torch.int32, device=device)
 
@@ -516,7 +516,7 @@ def _predecoded_moe_forward(x16, w16, route, payloads, backbones, num_experts, R
     # Mixtral decode shape)
     order = (("gate", pg), ("up", pu), ("down", pd))
     pre_jobs = [(bufs[name], p["q_gmap_gr_words"], p["q_gmap_gr_offsets"], p["q_gmap_gr_meta"],
-                 int(p["qweight1"].size(1)), int(p["qweight1"].size(2))) for name, p in order]
+                 *p["qweight1"].shape[1:]) for name, p in order]
     decoded = bufs
     sc = _in_scales(backbones)
     if predecoded is not None:

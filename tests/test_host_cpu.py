@@ -604,3 +604,4 @@ def test_weight_stationary_rule(tris):
     assert not ws(n=14336, gathered=1, rows=666) and ws(n=14336, gathered=1, rows=1024)
     # shapes past the 32-bit offsets stay on the decode kernel, senseless ones are no launch at all
     assert not ws(n=1 << 20, rows=2000) and not ws(rows=0) and not ws(segments=0) and not ws(nproj=1, swiglu=1)
+    assert not ws(rows=1 << 62)
